@@ -159,6 +159,9 @@ struct ClusterArgs {
     int32_t* nleaders;  // [n_lig]
 };
 
+// 32-bit words of the clustering kernel's first LDS array (one per pose, an even number of them).
+__host__ __device__ constexpr size_t cluster_near_words(int nchain) { return size_t(nchain + 1) & ~size_t(1); }
+
 struct ScoreArgs {
     LigSetDev L;
     SceneDev S;

@@ -217,71 +217,165 @@ __global__ __launch_bounds__(256) void grid_kernel(GridArgs A) {
         if (k < A.nslot) A.maps[(size_t)k * npt + id] = acc[k];
 }
 
-// Heavy-atom RMSD of two poses, cal_rmsd_pair_warp (cluster.cu:16-37), in float
-// with rounded operations in atom order, so that it is bit-identical to a
-// scalar float loop on the host.
-__device__ __forceinline__ float rmsd_exact(const float* a, const float* b, const float4* x0, int natom) {
-    float s = 0.0f;
-    int n = 0;
-    for (int i = 0; i < natom; i++) {
-        if (__float_as_int(x0[i].w) == kTypeH) continue;
-        float d0 = __fsub_rn(a[3 * i], b[3 * i]);
-        s = __fadd_rn(s, __fmul_rn(d0, d0));
-        float d1 = __fsub_rn(a[3 * i + 1], b[3 * i + 1]);
-        s = __fadd_rn(s, __fmul_rn(d1, d1));
-        float d2 = __fsub_rn(a[3 * i + 2], b[3 * i + 2]);
-        s = __fadd_rn(s, __fmul_rn(d2, d2));
-        n++;
+// Candidates of one round whose RMSDs a thread forms together.
+constexpr int kClusterCand = 4;
+
+// RMSDs of pose xo (this thread's; `live` threads only) with kClusterCand poses xc, the same for the
+// whole wave: bit k set where the RMSD to xc[k] is below limit. cal_rmsd_pair_warp (cluster.cu:16-37)
+// over the heavy atoms in float with rounded operations in atom order, so that each is bit-identical to a
+// scalar float loop on the host. The partial sums only grow, so a wave stops at the first four atoms after
+// which every sum has passed `cut`, a value of the sum from which the rounded RMSD is not below limit.
+__device__ __forceinline__ uint32_t rmsd_below(const float* xo, const float* const xc[kClusterCand], bool live,
+                                               const unsigned long long heavy[kMaxApl], int natom, int n, float cut,
+                                               float limit) {
+    float s[kClusterCand];
+#pragma unroll
+    for (int k = 0; k < kClusterCand; k++) s[k] = live ? 0.0f : INFINITY;
+    for (int a0 = 0; a0 < natom; a0 += 4) {
+        const uint32_t hv = uint32_t(heavy[a0 / kWave] >> (a0 % kWave)) & 15u;  // no bits past natom
+        if (hv == 0) continue;
+        float o[12];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if ((hv >> i) & 1u) {
+                const float* p = xo + 3 * (a0 + i);
+                o[3 * i] = p[0]; o[3 * i + 1] = p[1]; o[3 * i + 2] = p[2];
+            }
+#pragma unroll
+        for (int k = 0; k < kClusterCand; k++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if ((hv >> i) & 1u) {
+                    const float* p = xc[k] + 3 * (a0 + i);
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        const float d = __fsub_rn(o[3 * i + c], uload(p + c));
+                        s[k] = __fadd_rn(s[k], __fmul_rn(d, d));
+                    }
+                }
+        }
+        bool open = false;
+#pragma unroll
+        for (int k = 0; k < kClusterCand; k++) open |= s[k] < cut;
+        if (__ballot(open) == 0ull) return 0u;
     }
-    return __fsqrt_rn(__fdiv_rn(s, float(n)));
+    uint32_t below = 0u;
+#pragma unroll
+    for (int k = 0; k < kClusterCand; k++)
+        if (live && __fsqrt_rn(__fdiv_rn(s[k], float(n))) < limit) below |= 1u << k;
+    return below;
 }
 
 // Greedy leader clustering of one ligand per block (cluster_cu, cluster.cu:93-129):
 // poses ranked by ascending energy (ties by index), a pose becomes a leader when
 // its RMSD to every current leader is >= limit.
-__global__ __launch_bounds__(256) void cluster_kernel(ClusterArgs A) {
-    int* sh = reinterpret_cast<int*>(s_lds);
+// The remaining poses are kept compacted in rank order, and a round takes the first of them as
+// candidates, 4 per group of threads: every remaining pose is measured against every candidate (a
+// thread holds one pose and reads its group's candidates by scalar loads), the candidates are resolved
+// among themselves in rank order, and the poses near a new leader drop out. As the poses get fewer, the
+// block splits into more groups (up to 8, 32 candidates a round). The RMSDs are a serial sum per pair,
+// so what bounds the kernel is the latency of those sums and how many run at once. One pose at a time
+// against the leaders so far (a thread per leader, three barriers a pose) took 4,410 us for 64 ligands
+// of 512 poses; this takes 290 us. Blocks of 512 threads took 315 us.
+constexpr int kClusterThreads = 1024;
+__global__ __launch_bounds__(kClusterThreads) void cluster_kernel(ClusterArgs A) {
     const int lig = blockIdx.x;
     if (lig >= A.n_lig) return;
-    const int E = A.nchain;
-    int* order = sh;           // [E]
-    int* lead = sh + E;        // [E]
-    __shared__ int nlead;
-    __shared__ int flag;
+    const int E = A.nchain, tid = threadIdx.x, ln = lane();
+    const int n_words = (E + kWave - 1) / kWave;
+    float* es = s_lds;                                          // [E], until the poses are ranked
+    uint32_t* near = reinterpret_cast<uint32_t*>(s_lds);        // [E] then: candidates near each remaining pose
+    unsigned long long* left = reinterpret_cast<unsigned long long*>(s_lds + cluster_near_words(E));  // ranks remaining
+    uint16_t* order = reinterpret_cast<uint16_t*>(left + n_words);  // [E] pose of each rank
+    uint16_t* list = order + E;                                     // [E] remaining ranks, compacted
     const DevLig d = A.L.ligs[lig];
     const float* e = A.e + (size_t)lig * E;
-    for (int i = threadIdx.x; i < E; i += blockDim.x) {
-        float ei = e[i];
-        ei = ei != ei ? INFINITY : ei;
+    for (int i = tid; i < E; i += kClusterThreads) {
+        const float ei = e[i];
+        es[i] = ei != ei ? INFINITY : ei;
+    }
+    for (int w = tid; w < n_words; w += kClusterThreads) {
+        const int m = E - w * kWave;
+        left[w] = m >= kWave ? ~0ull : (1ull << m) - 1ull;
+    }
+    unsigned long long heavy[kMaxApl];
+    int n = 0;
+#pragma unroll
+    for (int k = 0; k < kMaxApl; k++) {
+        const int a = ln + kWave * k;
+        heavy[k] = __ballot(a < d.natom && __float_as_int(A.L.atom_x0[d.atom_off + (a < d.natom ? a : 0)].w) != kTypeH);
+        n += __popcll(heavy[k]);
+    }
+    __syncthreads();
+    for (int i = tid; i < E; i += kClusterThreads) {
+        const float ei = es[i];
         int rank = 0;
         for (int j = 0; j < E; j++) {
-            float ej = e[j];
-            ej = ej != ej ? INFINITY : ej;
+            const float ej = es[j];
             rank += (ej < ei) || (ej == ei && j < i);
         }
-        order[rank] = i;
+        order[rank] = uint16_t(i);
     }
-    if (threadIdx.x == 0) nlead = 0;
-    __syncthreads();
+    // sums from which sqrt(sum / n) is not below limit whatever the roundings (a few 1e-7); no cut for
+    // limits whose square loses precision
+    float cut = A.limit * A.limit * float(n) * 1.00001f;
+    if (!(cut > 1e-30f)) cut = A.limit > 0.0f && n > 0 ? INFINITY : 0.0f;
     const float* xb = A.x + (size_t)d.atom_off * E * 3;
-    const float4* x0 = A.L.atom_x0 + d.atom_off;
-    const int stride = d.natom * 3;
-    for (int r = 0; r < E; r++) {
-        const int idx = order[r];
-        if (threadIdx.x == 0) flag = 0;
-        __syncthreads();
-        const int nl = nlead;
-        for (int k = threadIdx.x; k < nl; k += blockDim.x) {
-            const int l = lead[k];
-            const int a = idx < l ? idx : l, b = idx < l ? l : idx;
-            if (rmsd_exact(xb + (size_t)a * stride, xb + (size_t)b * stride, x0, d.natom) < A.limit) flag = 1;
+    const size_t stride = (size_t)d.natom * 3;
+    int n_lead = 0;
+    __syncthreads();
+    for (;;) {
+        // compact the remaining ranks
+        int total = 0;
+        for (int w = 0; w < n_words; w++) total += __popcll(left[w]);
+        if (total == 0) break;
+        for (int r = tid; r < E; r += kClusterThreads) {
+            const unsigned long long m = left[r / kWave];
+            if ((m >> (r % kWave)) & 1ull) {
+                int at = __popcll(m & ((1ull << (r % kWave)) - 1ull));
+                for (int w = 0; w < r / kWave; w++) at += __popcll(left[w]);
+                list[at] = uint16_t(r);
+                near[at] = 0u;
+            }
         }
         __syncthreads();
-        if (threadIdx.x == 0 && flag == 0) lead[nlead++] = idx;
+        int groups = 1;
+        while (groups < 8 && (2 * groups) * ((total + kWave - 1) / kWave) * kWave <= kClusterThreads) groups *= 2;
+        const int per = kClusterThreads / groups, g = __builtin_amdgcn_readfirstlane(tid / per);
+        const int n_cand = min(kClusterCand * groups, total);
+        if (kClusterCand * g < n_cand) {
+            const float* xc[kClusterCand];
+#pragma unroll
+            for (int k = 0; k < kClusterCand; k++) {
+                const int i = min(kClusterCand * g + k, n_cand - 1);
+                xc[k] = xb + stride * (size_t)__builtin_amdgcn_readfirstlane(int(order[list[i]]));
+            }
+            const uint32_t real = (1u << min(kClusterCand, n_cand - kClusterCand * g)) - 1u;
+            for (int q0 = (tid % per) & ~(kWave - 1); q0 < total; q0 += per) {
+                const int q = q0 + ln;
+                const bool live = q < total;
+                const float* xo = xb + stride * (size_t)order[list[live ? q : 0]];
+                const uint32_t b = rmsd_below(xo, xc, live, heavy, d.natom, n, cut, A.limit) & real;
+                if (b) atomicOr(&near[q], b << (kClusterCand * g));
+            }
+        }
+        __syncthreads();
+        // the candidates in rank order: one becomes a leader unless a leader before it is near
+        const uint32_t mine = ln < n_cand ? near[ln] : 0u;
+        uint32_t lead = 0u;
+        for (int i = 0; i < n_cand; i++)
+            if ((uint32_t(rdl_i(int(mine), i)) & lead) == 0u) lead |= 1u << i;
+        if (tid < n_cand && ((lead >> tid) & 1u))
+            A.leaders[(size_t)lig * E + n_lead + __popc(lead & ((1u << tid) - 1u))] = order[list[tid]];
+        n_lead += __popc(lead);
+        for (int q = tid; q < total; q += kClusterThreads)
+            if (q < n_cand || (near[q] & lead)) {
+                const int r = list[q];
+                atomicAnd(&left[r / kWave], ~(1ull << (r % kWave)));
+            }
         __syncthreads();
     }
-    for (int k = threadIdx.x; k < nlead; k += blockDim.x) A.leaders[(size_t)lig * E + k] = lead[k];
-    if (threadIdx.x == 0) A.nleaders[lig] = nlead;
+    if (tid == 0) A.nleaders[lig] = n_lead;
 }
 
 // Weighted Vina terms of one heavy pair at surface distance d (Vina::eval_decomp,
@@ -556,8 +650,9 @@ hipError_t launch_posevec(PoseVecArgs a, int apl, int n_blocks, hipStream_t s) {
 
 hipError_t launch_cluster(const ClusterArgs& a, hipStream_t s) {
     if (a.n_lig <= 0) return hipSuccess;
-    size_t lds = (size_t)2 * a.nchain * sizeof(int);
-    hipLaunchKernelGGL(cluster_kernel, dim3(a.n_lig), dim3(256), lds, s, a);
+    const size_t lds = cluster_near_words(a.nchain) * sizeof(float) + (a.nchain + kWave - 1) / kWave * sizeof(uint64_t) +
+                       2 * a.nchain * sizeof(uint16_t);
+    hipLaunchKernelGGL(cluster_kernel, dim3(a.n_lig), dim3(kClusterThreads), lds, s, a);
     return hipGetLastError();
 }
 
