@@ -49,6 +49,17 @@ int pair_flags_host(int ti, int tj) {
     return hyd | (hb << 1);
 }
 
+// pair_lut of an atom type: its pair flags with a partner of flags b at bits 2 b.
+uint32_t pair_lut_host(int type) {
+    const int a = kFlagsHost[type];
+    uint32_t t = 0;
+    for (int b = 0; b < 8; b++) {
+        const int hb = (((a >> 1) & (b >> 2)) | ((a >> 2) & (b >> 1))) & 1;
+        t |= uint32_t((a & b & 1) | (hb << 1)) << (2 * b);
+    }
+    return t;
+}
+
 // Packed pair steps of a ligand of 33-64 atoms (LigSetDev::pack). Each step holds at most 63 pairs,
 // one per lane, with every atom i (gradient +p) of at most two of them and j (-p) of at most two, so
 // an atom collects its shares with four lane reads. Greedy first fit, the pairs of the busiest atoms
@@ -196,7 +207,6 @@ struct ud2_scene {
     float gspacing = 0;
     std::vector<int32_t> probe_types;
     int32_t slot_of_type[kNumTypes];
-    int32_t* d_probe = nullptr;
     int32_t* d_slot = nullptr;
 
     SceneDev view() const {
@@ -664,12 +674,8 @@ static int set_probe_types(ud2_scene* sc, const int32_t* probe_types_h, int32_t 
         if (sc->slot_of_type[t] >= 0) return fail(UD2_ERR_ARG, "duplicate probe type");
         sc->slot_of_type[t] = k;
     }
-    if (sc->d_probe) (void)hipFree(sc->d_probe);
     if (sc->d_slot) (void)hipFree(sc->d_slot);
-    sc->d_probe = nullptr;
     sc->d_slot = nullptr;
-    int rc = upload(&sc->d_probe, sc->probe_types);
-    if (rc) return rc;
     return upload(&sc->d_slot, std::vector<int32_t>(sc->slot_of_type, sc->slot_of_type + kNumTypes));
 }
 
@@ -709,9 +715,18 @@ int ud2_scene_build_grids(ud2_scene* sc, float spacing, const int32_t* probe_typ
     if (sc->d_maps) UD2_HIP(hipFree(sc->d_maps));
     sc->d_maps = nullptr;
     UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_maps), size_t(npt) * n_types * sizeof(float)));
-    GridArgs A;
+    GridArgs A{};
     A.S = sc->view();
-    A.probe_types = sc->d_probe;
+    std::vector<int32_t> by_radius(n_types);
+    std::iota(by_radius.begin(), by_radius.end(), 0);
+    std::stable_sort(by_radius.begin(), by_radius.end(),
+                     [&](int a, int b) { return kVdwHost[probe_types_h[a]] < kVdwHost[probe_types_h[b]]; });
+    for (int k = 0; k < n_types; k++) {
+        const int t = probe_types_h[by_radius[k]];
+        A.radius[k] = kVdwHost[t];
+        A.lut[k] = pair_lut_host(t);
+        A.slot[k] = by_radius[k];
+    }
     A.nslot = n_types;
     A.maps = sc->d_maps;
     UD2_HIP(launch_grid_build(A, nullptr));
@@ -790,7 +805,6 @@ int ud2_scene_destroy(ud2_scene* sc) {
     if (sc->d_rec) hipFree(sc->d_rec);
     if (sc->d_maps) hipFree(sc->d_maps);
     if (sc->d_cells) (void)hipFree(sc->d_cells);
-    if (sc->d_probe) (void)hipFree(sc->d_probe);
     if (sc->d_slot) (void)hipFree(sc->d_slot);
     delete sc;
     return UD2_OK;

@@ -41,6 +41,7 @@ static __constant__ int c_tflags[kNumTypes] = {0, 0, 1, 0, 0, 4, 2, 6, 0, 4, 2, 
 constexpr float kPi = 3.1415927f;               // E/src/myutils/common.h:45
 constexpr float kEps = 1.1920928955078125e-7f;  // FLT_EPSILON (common.h:13)
 constexpr float kR2Cut = 64.0f;                 // E/src/score/vina.h:130
+constexpr float kR2Reach = 64.01f;              // squared reach of a cull: the cutoff and its roundings
 constexpr float kVCap = 10.0f, kVCapAuth = 1000.0f, kSlope = 1e6f;  // constants.h:16-19
 constexpr int kTypeH = 0;
 
@@ -241,6 +242,30 @@ __device__ __forceinline__ uint32_t pair_lut(int a) {
     }
     return t;
 }
+
+// The energy of eval_ef in two parts with the same roundings: what depends on the surface distance d alone
+// (the return value, and the unweighted hydrophobic and hydrogen-bond terms h and b), and the flag terms.
+__device__ __forceinline__ float eval_radial(float d, float& h, float& b) {
+    const float e1 = __builtin_amdgcn_exp2f(-5.7707801635558535f * (d * d));
+    const float u = d - 3.0f;
+    const float e2 = __builtin_amdgcn_exp2f(-0.36067376022224085f * (u * u));
+    const float dn = fminf(d, 0.0f);
+    h = fminf(fmaxf(1.5f - d, 0.0f), 1.0f);
+    b = fminf(fmaxf(-d * (1.0f / 0.7f), 0.0f), 1.0f);
+    return fmaf_(0.840245f * dn, dn, msub2(-0.035579f, e1, 0.005156f, e2));
+}
+__device__ __forceinline__ float add_flag_terms(float e0, float h, float b, int flags) {
+    const float e = fmaf_((flags & 1) ? -0.035069f : 0.0f, h, e0);
+    return fmaf_((flags & 2) ? -0.587439f : 0.0f, b, e);
+}
+
+// A receptor atom's vdW radius and type flags in one word: the radius is in [1, 4), so its bits less
+// those of 1.0 take 24 bits; the doubled flags (as pair_lut takes them) take the bits above.
+__device__ __forceinline__ uint32_t atom_word(int type) {
+    return (__float_as_uint(c_vdw[type]) - 0x3F800000u) | (uint32_t(2 * c_tflags[type]) << 24);
+}
+__device__ __forceinline__ float word_radius(uint32_t w) { return __uint_as_float((w & 0xFFFFFFu) + 0x3F800000u); }
+__device__ __forceinline__ uint32_t word_flags2(uint32_t w) { return w >> 24; }
 
 // normalize_angle (E/src/myutils/mymath.h:38-47).
 __device__ __forceinline__ float normalize_angle(float x) {

@@ -176,7 +176,10 @@ struct ScoreArgs {
 
 struct GridArgs {
     SceneDev S;
-    const int32_t* probe_types;  // [nslot]
+    // the maps in order of their probe radius
+    float radius[kNumTypes];
+    uint32_t lut[kNumTypes];     // pair flags with a partner of doubled type flags f: (lut >> f) & 3
+    int32_t slot[kNumTypes];     // place in maps
     int32_t nslot;
     float* maps;
 };

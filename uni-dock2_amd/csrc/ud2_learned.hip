@@ -105,7 +105,7 @@ __device__ __forceinline__ void pose_features(const Ctx<APL>& C, const WPose<APL
 // the register allocation to the 80 VGPRs that six waves allow, which measured
 // 6 % faster than four waves at 128 VGPRs despite the spills (the search is
 // latency bound), and four waves faster than three. POL >= 0 compiles one
-// policy only (the learned search); POL = -1 takes the policy from the arguments. Wider ligands run at
+// policy only, on grid maps (the learned search); POL = -1 takes policy and inter term from the arguments. Wider ligands run at
 // three waves per SIMD (two slots) or two (three and four), as the MC kernel does.
 template <int APL, int POL>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) __attribute__((amdgpu_waves_per_eu(APL == 1 ? 6 : APL == 2 ? 3 : 2)))
@@ -128,7 +128,7 @@ void lmc_kernel(LmcArgs A) {
         const int chain = item % nchain;
         const size_t pid = (size_t)lig * nchain + chain;
         Ctx<APL> C;
-        load_ctx(C, A.L, A.S, lig, A.mode, base, A.hdim_ld);
+        load_ctx(C, A.L, A.S, lig, POL >= 0 ? int(kGrid) : A.mode, base, A.hdim_ld);
         Rng rng{A.seed, uint32_t(lig + A.lig_index_base), uint32_t(chain), 0u};
         C.evals = 0;
         int n_feat = 0;
@@ -352,10 +352,13 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void features_kernel(FeatArg
         default: return hipErrorInvalidValue; \
     }
 
+// Whether the build of lmc_kernel for the learned policy runs a search: it holds the grid inter term only.
+static bool lmc_learned_build(int policy, int mode) { return policy == kPolicyLearned && mode == kGrid; }
+
 template <int APL>
 static hipError_t launch_lmc_t(const LmcArgs& a, int n_blocks, hipStream_t s) {
     const size_t lds = (size_t)a.lds_floats_per_wave * kWavesPerBlock * sizeof(float);
-    if (a.policy == kPolicyLearned)
+    if (lmc_learned_build(a.policy, a.mode))
         hipLaunchKernelGGL((lmc_kernel<APL, kPolicyLearned>), dim3(n_blocks), dim3(kWave * kWavesPerBlock), lds, s, a);
     else
         hipLaunchKernelGGL((lmc_kernel<APL, -1>), dim3(n_blocks), dim3(kWave * kWavesPerBlock), lds, s, a);
@@ -384,9 +387,9 @@ hipError_t launch_features(FeatArgs a, int apl, hipStream_t s) {
 }
 
 template <int APL>
-static int lmc_occ_t(int policy, int lds_bytes) {
+static int lmc_occ_t(int policy, int mode, int lds_bytes) {
     int nb = 0;
-    const hipError_t e = policy == kPolicyLearned
+    const hipError_t e = lmc_learned_build(policy, mode)
                              ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, lmc_kernel<APL, kPolicyLearned>,
                                                                             kWave * kWavesPerBlock, lds_bytes)
                              : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, lmc_kernel<APL, -1>,
@@ -395,12 +398,12 @@ static int lmc_occ_t(int policy, int lds_bytes) {
     return nb > 0 ? nb : 1;
 }
 
-int lmc_blocks_per_cu(int apl, int policy, int lds_bytes) {
+int lmc_blocks_per_cu(int apl, int policy, int mode, int lds_bytes) {
     switch (apl) {
-        case 1: return lmc_occ_t<1>(policy, lds_bytes);
-        case 2: return lmc_occ_t<2>(policy, lds_bytes);
-        case 3: return lmc_occ_t<3>(policy, lds_bytes);
-        default: return lmc_occ_t<4>(policy, lds_bytes);
+        case 1: return lmc_occ_t<1>(policy, mode, lds_bytes);
+        case 2: return lmc_occ_t<2>(policy, mode, lds_bytes);
+        case 3: return lmc_occ_t<3>(policy, mode, lds_bytes);
+        default: return lmc_occ_t<4>(policy, mode, lds_bytes);
     }
 }
 
