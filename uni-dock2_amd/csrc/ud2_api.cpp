@@ -208,6 +208,12 @@ struct ud2_scene {
     std::vector<int32_t> probe_types;
     int32_t slot_of_type[kNumTypes];
     int32_t* d_slot = nullptr;
+    // reach lists of the direct sum (SceneDev::reach)
+    float4* d_reach = nullptr;
+    int32_t* d_reach_off = nullptr;
+    int32_t rn[3] = {0, 0, 0};
+    float rorigin[3] = {0, 0, 0}, redge = 1.0f;
+    float rec_lo[3], rec_hi[3];
 
     SceneDev view() const {
         SceneDev s;
@@ -218,7 +224,14 @@ struct ud2_scene {
             s.box_hi[d] = box_hi[d];
             s.gn[d] = gn[d];
             s.gorigin[d] = gorigin[d];
+            s.rn[d] = rn[d];
+            s.rorigin[d] = rorigin[d];
+            s.rec_lo[d] = rec_lo[d];
+            s.rec_hi[d] = rec_hi[d];
         }
+        s.reach = d_reach;
+        s.reach_off = d_reach_off;
+        s.rinv = 1.0f / redge;
         s.cells = d_cells;
         s.gspacing = gspacing;
         s.ginv = gspacing > 0 ? 1.0f / gspacing : 0.0f;
@@ -464,6 +477,8 @@ McArgs mc_args(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P, co
 int launch_mc_part(McArgs A, int apl, int variant, const int32_t* order, int n, int32_t* counter, int dmax,
                    int nchain, hipStream_t st, bool shared = false) {
     if (n <= 0) return UD2_OK;
+    // in direct mode the sum over the receptor outweighs what two chains per wave share: whole waves only
+    if (A.mode == kDirect) variant = kMcWhole;
     const int tw = mc_variant_tw(variant);
     const int cpw = kWave / tw;  // chains per wave
     A.order = order;
@@ -475,7 +490,7 @@ int launch_mc_part(McArgs A, int apl, int variant, const int32_t* order, int n, 
     if (lds_bytes > 160 * 1024) return fail(UD2_ERR_LIMIT, "per-block LDS exceeds 160 KB");
     const int64_t items = int64_t(n) * ((nchain + cpw - 1) / cpw);
     const int64_t need = (items + kWavesPerBlock - 1) / kWavesPerBlock;
-    int bpc = mc_blocks_per_cu(apl, variant, lds_bytes);
+    int bpc = mc_blocks_per_cu(apl, variant, A.mode, lds_bytes);
     if (shared && apl > 1) bpc = std::max(1, bpc - 1);
     const int64_t cap = int64_t(n_cus()) * bpc;
     const int nb = int(std::max<int64_t>(1, std::min(need, cap)));
@@ -626,6 +641,89 @@ int ud2_device_memory(int64_t* free_h, int64_t* total_h) {
 }
 
 // ------------------------------------------------------------------- scene
+namespace {
+
+// The scene's reach lists: cells of kReachEdge A over the box and kReachMargin A around it, where a receptor atom is
+// within 8 A at all; coarser where that makes more than kReachCells cells or kReachEntries entries. A
+// finer cell lists fewer atoms out of the cutoff (2 A: 1.65 listed per atom in reach, 3 A: 2.06) and
+// the lists then take more memory (a 30 A box: 15,625 cells, 15 MB). The margin holds the atoms of most poses
+// that the penalty is about to push back into the box.
+constexpr double kReachEdge = 2.0, kReachMargin = 10.0, kReachDist = 8.02;
+constexpr int64_t kReachCells = 1 << 14, kReachEntries = 1 << 23;
+
+int build_reach(ud2_scene* sc, const std::vector<float4>& rec) {
+    double lo[3], hi[3];
+    for (int d = 0; d < 3; d++) {
+        lo[d] = INFINITY;
+        hi[d] = -INFINITY;
+    }
+    for (const float4& r : rec) {
+        const float x[3] = {r.x, r.y, r.z};
+        if (!std::isfinite(r.x) || !std::isfinite(r.y) || !std::isfinite(r.z)) continue;  // never in reach
+        for (int d = 0; d < 3; d++) {
+            lo[d] = std::min(lo[d], double(x[d]) - kReachDist);
+            hi[d] = std::max(hi[d], double(x[d]) + kReachDist);
+        }
+    }
+    bool any = true;
+    for (int d = 0; d < 3; d++) {
+        sc->rec_lo[d] = float(lo[d]);
+        sc->rec_hi[d] = float(hi[d]);
+        lo[d] = std::max(lo[d], double(sc->box_lo[d]) - kReachMargin);
+        hi[d] = std::min(hi[d], double(sc->box_hi[d]) + kReachMargin);
+        any = any && hi[d] > lo[d];
+    }
+    if (!any) return UD2_OK;
+    double edge = kReachEdge;
+    for (;; edge *= 1.25) {
+        int64_t cells = 1;
+        for (int d = 0; d < 3; d++) {
+            const double n = std::ceil((hi[d] - lo[d]) / edge);
+            if (!(n <= double(kReachCells))) cells = kReachCells + 1;
+            else {
+                sc->rn[d] = std::max(1, int32_t(n));
+                cells = std::min(cells * sc->rn[d], kReachCells + 1);
+            }
+        }
+        if (cells > kReachCells) continue;
+        sc->redge = float(edge);
+        ReachArgs A{};
+        A.rec = sc->d_rec;
+        A.nrec = sc->nrec;
+        for (int d = 0; d < 3; d++) {
+            A.rn[d] = sc->rn[d];
+            A.rorigin[d] = sc->rorigin[d] = float(lo[d]);
+        }
+        A.edge = sc->redge;
+        std::vector<int32_t> off(cells + 1, 0);
+        if (sc->d_reach_off) UD2_HIP(hipFree(sc->d_reach_off));
+        sc->d_reach_off = nullptr;
+        UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_reach_off), off.size() * sizeof(int32_t)));
+        A.count = sc->d_reach_off;
+        A.off = sc->d_reach_off;
+        UD2_HIP(launch_reach(A, false, nullptr));
+        UD2_HIP(hipMemcpy(off.data() + 1, sc->d_reach_off, cells * sizeof(int32_t), hipMemcpyDeviceToHost));
+        int64_t total = 0;
+        for (int64_t c = 1; c <= cells; c++) {
+            total += (off[c] + kReachPad - 1) / kReachPad * kReachPad;
+            off[c] = int32_t(std::min(total, kReachEntries + kReachPad));
+        }
+        if (total > kReachEntries && cells > 1) continue;
+        if (total > kReachEntries) {  // one cell and still too many: the whole receptor, by scalar loads
+            for (int d = 0; d < 3; d++) sc->rn[d] = 0;
+            return UD2_OK;
+        }
+        UD2_HIP(hipMemcpy(sc->d_reach_off, off.data(), off.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+        UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_reach), std::max<size_t>(total, 1) * sizeof(float4)));
+        A.reach = sc->d_reach;
+        UD2_HIP(launch_reach(A, true, nullptr));
+        UD2_HIP(hipStreamSynchronize(nullptr));
+        return UD2_OK;
+    }
+}
+
+}  // namespace
+
 int ud2_scene_create(const float* rec_xyz_h, const int32_t* rec_types_h, int32_t n_rec, const float box_lo_h[3],
                      const float box_hi_h[3], ud2_scene** out) {
     if (!out) return fail(UD2_ERR_ARG, "null output");
@@ -656,8 +754,9 @@ int ud2_scene_create(const float* rec_xyz_h, const int32_t* rec_types_h, int32_t
     for (int t = 0; t < kNumTypes; t++) sc->slot_of_type[t] = -1;
     sc->nrec = int32_t(rec.size());
     int rc = upload(&sc->d_rec, rec);
+    if (!rc) rc = build_reach(sc, rec);
     if (rc) {
-        delete sc;
+        ud2_scene_destroy(sc);
         return rc;
     }
     *out = sc;
@@ -806,6 +905,8 @@ int ud2_scene_destroy(ud2_scene* sc) {
     if (sc->d_maps) hipFree(sc->d_maps);
     if (sc->d_cells) (void)hipFree(sc->d_cells);
     if (sc->d_slot) (void)hipFree(sc->d_slot);
+    if (sc->d_reach) (void)hipFree(sc->d_reach);
+    if (sc->d_reach_off) (void)hipFree(sc->d_reach_off);
     delete sc;
     return UD2_OK;
 }
@@ -1158,7 +1259,7 @@ int ud2_score_posevecs(const ud2_scene* sc, const ud2_ligset* ls, int32_t lig, i
     A.lds_floats_per_wave = lds_round4(lds_head_floats(d.apl, A.hdim_ld));
     const int lds_bytes = A.lds_floats_per_wave * kWavesPerBlock * int(sizeof(float));
     const int64_t need = (n + kWavesPerBlock - 1) / kWavesPerBlock;
-    const int64_t cap = int64_t(n_cus()) * posevec_blocks_per_cu(d.apl, lds_bytes);
+    const int64_t cap = int64_t(n_cus()) * posevec_blocks_per_cu(d.apl, mode, lds_bytes);
     const int nb = int(std::max<int64_t>(1, std::min(need, cap)));
     UD2_HIP(launch_posevec(A, d.apl, nb, static_cast<hipStream_t>(stream)));
     return UD2_OK;
@@ -1296,7 +1397,7 @@ int ud2_autotune(const ud2_scene* sc, const ud2_ligset* ls, const ud2_mc_params*
         hipEvent_t ev0 = nullptr, ev1 = nullptr;
         const int lds1 = kWavesPerBlock * int(sizeof(float)) *
                          lds_round4(lds_head_floats(1, odd_ld(kTileNarrow), kWave) + kTileNarrow * odd_ld(kTileNarrow));
-        const int64_t slots = int64_t(n_cus()) * mc_blocks_per_cu(1, kMcWhole, lds1) * kWavesPerBlock;
+        const int64_t slots = int64_t(n_cus()) * mc_blocks_per_cu(1, kMcWhole, prm->mode, lds1) * kWavesPerBlock;
         const int reps = int(std::max<int64_t>(1, (2 * slots + nchain - 1) / nchain));
         auto run = [&]() -> int {
             UD2_HIP(hipMalloc(&x, size_t(n_atoms) * nchain * 3 * sizeof(float)));
@@ -1782,7 +1883,7 @@ int ud2_lmc(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P, const
         if (lds_bytes > 160 * 1024) return fail(UD2_ERR_LIMIT, "per-block LDS exceeds 160 KB");
         const int64_t items = int64_t(cnt) * P->nchain;
         const int64_t need = (items + kWavesPerBlock - 1) / kWavesPerBlock;
-        const int64_t cap = int64_t(cus) * lmc_blocks_per_cu(apl, A.policy, lds_bytes);
+        const int64_t cap = int64_t(cus) * lmc_blocks_per_cu(apl, A.policy, A.mode, lds_bytes);
         const int nb = int(std::max<int64_t>(1, std::min(need, cap)));
         UD2_HIP(launch_lmc(A, apl, nb, st));
     }

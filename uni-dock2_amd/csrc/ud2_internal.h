@@ -82,6 +82,15 @@ struct SceneDev {
     float gorigin[3];
     float gspacing, ginv;
     const int32_t* slot_tab;  // [kNumTypes] map of each XS type (-1 = none), device memory
+    // Reach lists of the direct sum: the space around the box in cells of edge 1 / rinv from rorigin, and per
+    // cell the receptor atoms that a point in it can have within the cutoff, in receptor order: entries
+    // reach_off[cell] .. reach_off[cell + 1] of reach (x, y, z, atom_word), their number padded to a
+    // multiple of 4 with atoms out of any reach. Beyond rec_lo .. rec_hi no receptor atom is in reach.
+    const float4* reach;
+    const int32_t* reach_off;
+    int32_t rn[3];
+    float rorigin[3], rinv;
+    float rec_lo[3], rec_hi[3];
 };
 
 // Pose buffers of a ligand set with nchain poses per ligand, laid out by
@@ -173,6 +182,18 @@ struct ScoreArgs {
     float* decomp;        // [n_sel][decomp_stride][5] per-atom inter terms (decomposition launch)
     int32_t decomp_stride;
 };
+
+// Reach lists (SceneDev::reach): counts of every cell's list (fill false), or the lists.
+struct ReachArgs {
+    const float4* rec;
+    int32_t nrec;
+    int32_t rn[3];
+    float rorigin[3], edge;
+    int32_t* count;      // [cells]
+    const int32_t* off;  // [cells + 1]
+    float4* reach;
+};
+constexpr int kReachPad = 4;  // a list's length is a multiple of this
 
 struct GridArgs {
     SceneDev S;
@@ -278,6 +299,7 @@ struct FeatArgs {
 // Launchers (ud2_kernels.hip); each returns a hipError_t.
 hipError_t launch_grid_build(const GridArgs& a, hipStream_t s);
 hipError_t launch_brick(const BrickArgs& a, hipStream_t s);
+hipError_t launch_reach(const ReachArgs& a, bool fill, hipStream_t s);
 constexpr int kProbePerThread = 16;  // gathers per thread of the gather probe
 hipError_t launch_gather_probe(const float4* cells, uint32_t span, uint32_t seed, float* out, int64_t n_threads,
                                hipStream_t s);
@@ -288,7 +310,7 @@ hipError_t launch_posevec(PoseVecArgs a, int apl, int n_blocks, hipStream_t s);
 hipError_t launch_cluster(const ClusterArgs& a, hipStream_t s);
 hipError_t launch_final_score(const ScoreArgs& a, int apl, bool decomp, hipStream_t s);
 hipError_t launch_fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s);
-int mc_blocks_per_cu(int apl, int variant, int lds_bytes_per_block);
+int mc_blocks_per_cu(int apl, int variant, int mode, int lds_bytes_per_block);
 // LDS floats of a wave slice before its torsion table: coordinates + pair forces (7 * 64 * apl) and two
 // parked poses (64 * (3 * apl + 1) + 8 each), lds_flags_offset; a multiple of 4, so the table after it
 // stays 16-byte aligned. A tile of tw < 64 lanes (one chain of a wave that runs 64 / tw chains) has the
@@ -307,14 +329,14 @@ __host__ __device__ constexpr int lds_head_floats(int apl, int ld, int tw = kWav
 }
 // Per-wave slices are rounded to 4 floats so every slice starts 16-byte aligned.
 __host__ __device__ constexpr int lds_round4(int n) { return (n + 3) & ~3; }
-int posevec_blocks_per_cu(int apl, int lds_bytes_per_block);
+int posevec_blocks_per_cu(int apl, int mode, int lds_bytes_per_block);
 // LDS floats per wave of the features kernel: the head and 8 floats per atom of feature scratch.
 __host__ __device__ constexpr int lds_prop_floats(int apl, int ld) { return lds_head_floats(apl, ld) + 8 * kWave * apl; }
 
 // Learned proposal (ud2_learned.hip) and network (ud2_mlp.hip) launchers.
 hipError_t launch_lmc(LmcArgs a, int apl, int n_blocks, hipStream_t s);
 hipError_t launch_features(FeatArgs a, int apl, hipStream_t s);
-int lmc_blocks_per_cu(int apl, int policy, int lds_bytes_per_block);
+int lmc_blocks_per_cu(int apl, int policy, int mode, int lds_bytes_per_block);
 hipError_t launch_mlp_forward(const MlpDev& W, const uint16_t* x, const int32_t* groups, int64_t n_groups, float* y,
                               hipStream_t s);
 hipError_t launch_mlp_backward(const MlpDev& W, const MlpTrain& T, hipStream_t s);

@@ -23,7 +23,8 @@ namespace ud2 {
 // its LDS allows three blocks per CU), the three- and four-slot kernels at two: on ligands of 65-80
 // atoms three waves measured 25 % faster than the two that an unconstrained allocation (239 VGPRs)
 // allowed.
-template <int APL, int TW, int OCC>
+// MODE is the inter term: the grid builds hold nothing of the direct sum and the other way round.
+template <int APL, int TW, int OCC, int MODE>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) __attribute__((amdgpu_waves_per_eu(OCC)))
 void mc_kernel(McArgs A) {
     constexpr int CPW = kWave / TW;  // chains per wave
@@ -43,7 +44,7 @@ void mc_kernel(McArgs A) {
         const bool real = CPW == 1 || c < nchain;
         const int chain = real ? c : nchain - 1;
         Ctx<APL, TW> C;
-        load_ctx(C, A.L, A.S, lig, A.mode, base, A.hdim_ld);
+        load_ctx(C, A.L, A.S, lig, MODE, base, A.hdim_ld);
         Rng rng{A.seed, uint32_t(lig + A.lig_index_base), uint32_t(chain), 0u};
         WPose<APL> acc;
         initial_pose(C, A.L, lig, acc);
@@ -96,7 +97,7 @@ void mc_kernel(McArgs A) {
 // energy + gradient, one pose update, one line search from H = I
 // (line_search_one_gpu, E/src/cuda/bfgs_wrapper.cu:12-48), or a reset to the
 // input conformation.
-template <int APL>
+template <int APL, int MODE>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) void opt_kernel(OptArgs A) {
     const int w = threadIdx.x / kWave;
     const int s = blockIdx.x * kWavesPerBlock + w;
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void opt_kernel(OptArgs A) {
     const int lig = pid / A.P.nchain, chain = pid % A.P.nchain;
     const int o = A.pos ? A.pos[s] : s;
     Ctx<APL> C;
-    load_ctx(C, A.L, A.S, lig, A.mode, w * A.lds_floats_per_wave, A.hdim_ld);
+    load_ctx(C, A.L, A.S, lig, MODE, w * A.lds_floats_per_wave, A.hdim_ld);
     WPose<APL> P;
     const int ln = lane();
     if (A.op == 4) {
@@ -145,11 +146,11 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void opt_kernel(OptArgs A) {
 // of one ligand: torsions set on its input conformation in index order, then
 // the conformer rotated by q about its centroid and moved to the centre;
 // rot_vec = rotvec(q).
-template <int APL>
+template <int APL, int MODE>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) void posevec_kernel(PoseVecArgs A) {
     const int w = threadIdx.x / kWave;
     Ctx<APL> C;
-    load_ctx(C, A.L, A.S, A.lig, A.mode, w * A.lds_floats_per_wave, A.hdim_ld);
+    load_ctx(C, A.L, A.S, A.lig, MODE, w * A.lds_floats_per_wave, A.hdim_ld);
     WPose<APL> P0;
     initial_pose(C, A.L, A.lig, P0);
     const int ln = lane();
@@ -470,23 +471,24 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void final_score_kernel(Scor
         float t5[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
         if (ti != kTypeH) {
             const float ri = c_vdw[ti];
-            for (int j = 0; j < S.nrec; j++) {
-                const float4 r = S.rec[j];
-                float rx = r.x - px, ry = r.y - py, rz = r.z - pz;
-                float rr = rx * rx + ry * ry + rz * rz;
+            const uint32_t lut = pair_lut(c_tflags[ti]);
+            for_reach(S, reach_of(S, px, py, pz), [&](float qx, float qy, float qz, uint32_t word) {
+                const float rx = qx - px, ry = qy - py, rz = qz - pz;
+                const float rr = rx * rx + ry * ry + rz * rz;
                 if (rr < kR2Cut) {
-                    const int tj = __float_as_int(r.w);
+                    const float dist = sqrtf(rr) - (ri + word_radius(word));
+                    const int fl = int(lut >> word_flags2(word)) & 3;
                     if (DECOMP) {
                         float t[5];
-                        eval_terms(sqrtf(rr) - (ri + c_vdw[tj]), pair_flags(ti, tj), t);
+                        eval_terms(dist, fl, t);
 #pragma unroll
                         for (int q = 0; q < 5; q++) t5[q] += t[q];
                     } else {
                         float dd;
-                        e_inter += eval_ef(sqrtf(rr) - (ri + c_vdw[tj]), pair_flags(ti, tj), &dd);
+                        e_inter += eval_ef(dist, fl, &dd);
                     }
                 }
-            }
+            });
             if (px < S.box_lo[0]) e_pen += S.box_lo[0] - px;
             if (px > S.box_hi[0]) e_pen += px - S.box_hi[0];
             if (py < S.box_lo[1]) e_pen += S.box_lo[1] - py;
@@ -533,6 +535,50 @@ __global__ void fill_i32_kernel(int32_t* p, int32_t v, int64_t n) {
 hipError_t launch_fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(fill_i32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, v, n);
+    return hipGetLastError();
+}
+
+// Reach lists: one wave per cell takes the receptor in chunks of 64 atoms and keeps, in receptor order, those
+// within reach of the cell's cube (widened a little for points that round into it).
+template <bool FILL>
+__global__ __launch_bounds__(kWave* kWavesPerBlock) void reach_kernel(ReachArgs A) {
+    const int cell = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave, ln = lane();
+    if (cell >= A.rn[0] * A.rn[1] * A.rn[2]) return;
+    const int c[3] = {cell % A.rn[0], (cell / A.rn[0]) % A.rn[1], cell / (A.rn[0] * A.rn[1])};
+    float lo[3], hi[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        lo[d] = A.rorigin[d] + A.edge * float(c[d]) - 1e-3f;
+        hi[d] = A.rorigin[d] + A.edge * float(c[d] + 1) + 1e-3f;
+    }
+    int n = 0;
+    float4* out = FILL ? A.reach + A.off[cell] : nullptr;
+    for (int j0 = 0; j0 < A.nrec; j0 += kWave) {
+        const int j = j0 + ln;
+        const float4 r = A.rec[j < A.nrec ? j : A.nrec - 1];
+        const float ex = fmaxf(fmaxf(lo[0] - r.x, r.x - hi[0]), 0.0f);
+        const float ey = fmaxf(fmaxf(lo[1] - r.y, r.y - hi[1]), 0.0f);
+        const float ez = fmaxf(fmaxf(lo[2] - r.z, r.z - hi[2]), 0.0f);
+        const unsigned long long m = __ballot(j < A.nrec && sq_dist(ex, ey, ez) < kR2Reach);
+        if (FILL && ((m >> ln) & 1ull))
+            out[n + __popcll(m & ((1ull << ln) - 1ull))] =
+                make_float4(r.x, r.y, r.z, __uint_as_float(atom_word(__float_as_int(r.w))));
+        n += __popcll(m);
+    }
+    if (!FILL) {
+        if (ln == 0) A.count[cell] = n;
+        return;
+    }
+    const int pad = (kReachPad - n % kReachPad) % kReachPad;
+    if (ln < pad) out[n + ln] = make_float4(1e18f, 1e18f, 1e18f, 0.0f);
+}
+
+hipError_t launch_reach(const ReachArgs& a, bool fill, hipStream_t s) {
+    const int64_t n = (int64_t)a.rn[0] * a.rn[1] * a.rn[2];
+    if (n <= 0) return hipSuccess;
+    const dim3 grid((unsigned)((n + kWavesPerBlock - 1) / kWavesPerBlock)), block(kWave * kWavesPerBlock);
+    if (fill) hipLaunchKernelGGL(reach_kernel<true>, grid, block, 0, s, a);
+    else hipLaunchKernelGGL(reach_kernel<false>, grid, block, 0, s, a);
     return hipGetLastError();
 }
 
@@ -623,10 +669,10 @@ hipError_t launch_grid_build(const GridArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int APL, int TW, int OCC>
+template <int APL, int TW, int OCC, int MODE = kGrid>
 static hipError_t launch_mc_t(const McArgs& a, int n_blocks, hipStream_t s) {
     size_t lds = (size_t)a.lds_floats_per_wave * kWavesPerBlock * sizeof(float);
-    hipLaunchKernelGGL((mc_kernel<APL, TW, OCC>), dim3(n_blocks), dim3(kWave * kWavesPerBlock), lds, s, a);
+    hipLaunchKernelGGL((mc_kernel<APL, TW, OCC, MODE>), dim3(n_blocks), dim3(kWave * kWavesPerBlock), lds, s, a);
     return hipGetLastError();
 }
 
@@ -636,6 +682,18 @@ static hipError_t launch_mc_t(const McArgs& a, int n_blocks, hipStream_t s) {
 // six-wave build, 33.9 on the four-wave one, 34.9 on the two-wave one, which spills nothing).
 hipError_t launch_mc(McArgs a, int apl, int variant, int n_blocks, int waves, hipStream_t s) {
     if (variant != kMcWhole && apl != 1) return hipErrorInvalidValue;
+    if (a.mode == kDirect) {  // whole waves at two or four waves per SIMD (one slot), as below otherwise
+        if (variant != kMcWhole) return hipErrorInvalidValue;
+        switch (apl) {
+            case 1:
+                return waves <= 2 ? launch_mc_t<1, kWave, 2, kDirect>(a, n_blocks, s)
+                                  : launch_mc_t<1, kWave, 4, kDirect>(a, n_blocks, s);
+            case 2: return launch_mc_t<2, kWave, 3, kDirect>(a, n_blocks, s);
+            case 3: return launch_mc_t<3, kWave, 2, kDirect>(a, n_blocks, s);
+            case 4: return launch_mc_t<4, kWave, 2, kDirect>(a, n_blocks, s);
+            default: return hipErrorInvalidValue;
+        }
+    }
     switch (variant) {
         case kMcHalf4: return launch_mc_t<1, kTileNarrow, 4>(a, n_blocks, s);
         case kMcHalf3: return launch_mc_t<1, kTileNarrow, 3>(a, n_blocks, s);
@@ -659,7 +717,10 @@ template <int APL>
 static hipError_t launch_opt_t(const OptArgs& a, hipStream_t s) {
     size_t lds = (size_t)a.lds_floats_per_wave * kWavesPerBlock * sizeof(float);
     int nb = (a.n_sel + kWavesPerBlock - 1) / kWavesPerBlock;
-    hipLaunchKernelGGL(opt_kernel<APL>, dim3(nb), dim3(kWave * kWavesPerBlock), lds, s, a);
+    if (a.mode == kDirect)
+        hipLaunchKernelGGL((opt_kernel<APL, kDirect>), dim3(nb), dim3(kWave * kWavesPerBlock), lds, s, a);
+    else
+        hipLaunchKernelGGL((opt_kernel<APL, kGrid>), dim3(nb), dim3(kWave * kWavesPerBlock), lds, s, a);
     return hipGetLastError();
 }
 
@@ -677,7 +738,10 @@ hipError_t launch_opt(OptArgs a, int apl, hipStream_t s) {
 template <int APL>
 static hipError_t launch_posevec_t(const PoseVecArgs& a, int n_blocks, hipStream_t s) {
     size_t lds = (size_t)a.lds_floats_per_wave * kWavesPerBlock * sizeof(float);
-    hipLaunchKernelGGL(posevec_kernel<APL>, dim3(n_blocks), dim3(kWave * kWavesPerBlock), lds, s, a);
+    if (a.mode == kDirect)
+        hipLaunchKernelGGL((posevec_kernel<APL, kDirect>), dim3(n_blocks), dim3(kWave * kWavesPerBlock), lds, s, a);
+    else
+        hipLaunchKernelGGL((posevec_kernel<APL, kGrid>), dim3(n_blocks), dim3(kWave * kWavesPerBlock), lds, s, a);
     return hipGetLastError();
 }
 
@@ -719,16 +783,22 @@ hipError_t launch_final_score(const ScoreArgs& a, int apl, bool decomp, hipStrea
     }
 }
 
-template <int APL, int TW, int OCC>
+template <int APL, int TW, int OCC, int MODE = kGrid>
 static int mc_occ(int lds_bytes) {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, mc_kernel<APL, TW, OCC>, kWave * kWavesPerBlock, lds_bytes) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, mc_kernel<APL, TW, OCC, MODE>, kWave * kWavesPerBlock, lds_bytes) !=
         hipSuccess)
         return 1;
     return nb > 0 ? nb : 1;
 }
 
-int mc_blocks_per_cu(int apl, int variant, int lds_bytes) {
+int mc_blocks_per_cu(int apl, int variant, int mode, int lds_bytes) {
+    if (mode == kDirect) switch (apl) {
+            case 1: return mc_occ<1, kWave, 4, kDirect>(lds_bytes);
+            case 2: return mc_occ<2, kWave, 3, kDirect>(lds_bytes);
+            case 3: return mc_occ<3, kWave, 2, kDirect>(lds_bytes);
+            default: return mc_occ<4, kWave, 2, kDirect>(lds_bytes);
+        }
     switch (variant) {
         case kMcHalf4: return mc_occ<1, kTileNarrow, 4>(lds_bytes);
         case kMcHalf3: return mc_occ<1, kTileNarrow, 3>(lds_bytes);
@@ -744,20 +814,22 @@ int mc_blocks_per_cu(int apl, int variant, int lds_bytes) {
 }
 
 template <int APL>
-static int pv_occ(int lds_bytes) {
+static int pv_occ(int mode, int lds_bytes) {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, posevec_kernel<APL>, kWave * kWavesPerBlock, lds_bytes) !=
-        hipSuccess)
-        return 1;
-    return nb > 0 ? nb : 1;
+    const hipError_t e =
+        mode == kDirect ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, posevec_kernel<APL, kDirect>,
+                                                                       kWave * kWavesPerBlock, lds_bytes)
+                        : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, posevec_kernel<APL, kGrid>,
+                                                                       kWave * kWavesPerBlock, lds_bytes);
+    return e == hipSuccess && nb > 0 ? nb : 1;
 }
 
-int posevec_blocks_per_cu(int apl, int lds_bytes) {
+int posevec_blocks_per_cu(int apl, int mode, int lds_bytes) {
     switch (apl) {
-        case 1: return pv_occ<1>(lds_bytes);
-        case 2: return pv_occ<2>(lds_bytes);
-        case 3: return pv_occ<3>(lds_bytes);
-        default: return pv_occ<4>(lds_bytes);
+        case 1: return pv_occ<1>(mode, lds_bytes);
+        case 2: return pv_occ<2>(mode, lds_bytes);
+        case 3: return pv_occ<3>(mode, lds_bytes);
+        default: return pv_occ<4>(mode, lds_bytes);
     }
 }
 
