@@ -60,12 +60,46 @@ uint32_t pair_lut_host(int type) {
     return t;
 }
 
+uint32_t float_bits(float v) {
+    uint32_t u;
+    std::memcpy(&u, &v, sizeof(u));
+    return u;
+}
+
+// Entry of a lane without a pair, and a pair's part of an entry (LigSetDev::pack).
+const uint4 kNoPair = make_uint4(0u, 0u, float_bits(kRampNoPair), 0u);
+void set_pair(uint4& t, int i, int j, const int32_t* types) {
+    const int fl = pair_flags_host(types[i], types[j]);
+    t.x = uint32_t(16 * i) | (uint32_t(16 * j) << 16);
+    t.z = float_bits(ramp_hyd(fl));
+    t.w = float_bits(ramp_hb(fl));
+}
+
+// Pair steps of a ligand of at most 32 atoms (LigSetDev::pack), from its folded diagonals (mask bit l of diagonal
+// d: the pair {l, (l + d) mod na} is scored). Appends the steps' entries and returns their number.
+int pack_diagonals(int na, const unsigned long long* fold, int nfold, const int32_t* types, std::vector<uint4>& pack) {
+    for (int d = 1; d <= nfold; d += 2) {
+        const size_t base = pack.size();
+        pack.resize(base + kWave, kNoPair);
+        for (int l = 0; l < kWave; l++) {
+            const int a = l & 31, dl = d + (l >> 5);
+            uint4& t = pack[base + l];
+            if (a >= na) continue;
+            const int j = (a + dl) % na;
+            if (dl <= nfold && ((fold[dl - 1] >> a) & 1ull)) set_pair(t, a, j, types);
+            t.x = uint32_t(16 * j);
+            t.y = uint32_t(4 * ((a + na - d % na) % na)) | (uint32_t(4 * (32 + (a + na - (d + 1) % na) % na)) << 8);
+        }
+    }
+    return (nfold + 1) / 2;
+}
+
 // Packed pair steps of a ligand of 33-64 atoms (LigSetDev::pack). Each step holds at most 63 pairs,
 // one per lane, with every atom i (gradient +p) of at most two of them and j (-p) of at most two, so
 // an atom collects its shares with four lane reads. Greedy first fit, the pairs of the busiest atoms
 // first, each pair in the first step where either orientation fits. Appends the steps' entries and
 // returns their number, or -1 if the steps do not cover the pairs.
-int pack_pairs(int na, const std::vector<std::pair<int, int>>& pl, const int32_t* types, std::vector<uint2>& pack) {
+int pack_pairs(int na, const std::vector<std::pair<int, int>>& pl, const int32_t* types, std::vector<uint4>& pack) {
     constexpr int kSlots = 2, kLanes = kWave - 1, kNone = kLanes * 4;
     std::vector<int> deg(na, 0);
     for (auto& ij : pl) {
@@ -113,11 +147,10 @@ int pack_pairs(int na, const std::vector<std::pair<int, int>>& pl, const int32_t
         uint32_t src_i[kWave] = {}, src_j[kWave] = {};
         int ni[kWave] = {}, nj[kWave] = {};
         const size_t base = pack.size();
-        pack.resize(base + kWave, make_uint2(0u, 0u));
+        pack.resize(base + kWave, kNoPair);
         for (int l = 0; l < int(st.lanes.size()); l++) {
             const int i = st.lanes[l].first, j = st.lanes[l].second;
-            pack[base + l].x = uint32_t(i) | (uint32_t(j) << 8) |
-                               (uint32_t(pair_flags_host(types[i], types[j])) << 16) | (1u << 31);
+            set_pair(pack[base + l], i, j, types);
             src_i[i] |= uint32_t(4 * l) << (8 * ni[i]++);
             src_j[j] |= uint32_t(4 * l) << (8 * nj[j]++);
             covered++;
@@ -254,7 +287,7 @@ struct ud2_ligset {
     unsigned long long* d_mask = nullptr;
     uint2* d_pairs = nullptr;
     unsigned long long* d_fold = nullptr;
-    uint2* d_pack = nullptr;
+    uint4* d_pack = nullptr;
     int32_t* d_counter = nullptr;
     // Work order of the persistent search launches, fixed at creation: ligands by atoms-per-lane
     // class (widest first), within a class most expensive first, so each launch's tail holds the
@@ -934,7 +967,7 @@ int ud2_ligset_create(const ud2_ligand_batch* b, ud2_ligset** out) {
     std::vector<unsigned long long> mask(size_t(nt_all) * kMaxApl, 0ull);
     std::vector<uint2> pairs;
     std::vector<unsigned long long> fold;
-    std::vector<uint2> pack;
+    std::vector<uint4> pack;
     std::vector<uint8_t> has_type(kNumTypes, 0);
     for (int l = 0; l < n; l++) {
         const int a0 = b->atom_off_h[l], na = b->atom_off_h[l + 1] - a0;
@@ -1075,7 +1108,10 @@ int ud2_ligset_create(const ud2_ligand_batch* b, ud2_ligset** out) {
             if (n_steps < 0) return fail(UD2_ERR_STATE, tag + "packed pair steps do not cover the pairs");
             d.npack = n_steps;
         }
+        if (na <= kWave / 2 && !pl.empty())
+            d.npack = pack_diagonals(na, fold.data() + d.fold_off, d.nfold, b->types_h + a0, pack);
     }
+    pack.resize(pack.size() + kWave, kNoPair);  // the kernels load one step ahead
     ud2_ligset* ls = new ud2_ligset();
     hipGetDevice(&ls->device);
     ls->n_lig = n;
@@ -1092,7 +1128,7 @@ int ud2_ligset_create(const ud2_ligand_batch* b, ud2_ligset** out) {
         auto cost = [&](int l) {
             const DevLig& d = ligs[l];
             const double pairs = d.natom <= kWave / 2 ? 23.5 * d.natom
-                                 : d.npack > 0        ? 95.0 * d.npack
+                                 : d.apl == 1         ? 95.0 * d.npack
                                                       : 41.5 * double(d.apl) * d.natom;
             return (2800.0 + 36.0 * d.natom) * (1500.0 + pairs + 64.0 * d.ntors);
         };
@@ -1116,7 +1152,7 @@ int ud2_ligset_create(const ud2_ligand_batch* b, ud2_ligset** out) {
     if (!rc) rc = upload(&ls->d_mask, mask);
     if (!rc) rc = upload(&ls->d_pairs, pairs);
     if (!rc) rc = upload(&ls->d_fold, fold);
-    if (!rc) rc = upload(&ls->d_pack, pack.empty() ? std::vector<uint2>(kWave, make_uint2(0u, 0u)) : pack);
+    if (!rc) rc = upload(&ls->d_pack, pack);
     if (!rc) rc = upload(&ls->d_counter, std::vector<int32_t>(std::max(kMcHeads, kMaxApl + 1), 0));
     if (!rc) rc = upload(&ls->d_order, ls->h_order);
     if (!rc) rc = upload(&ls->d_split, std::vector<int32_t>(std::max(ls->cls_cnt[1], 1), 0));

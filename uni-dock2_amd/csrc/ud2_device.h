@@ -7,14 +7,12 @@
 // the dihedral vector and every BFGS vector (gradient, direction, y, -Hy) are
 // one VGPR each with component k on lane k; the inverse Hessian is a per-wave
 // LDS tile whose row i only lane i reads and writes. Energies, torques and
-// dot products are wave reductions. Intra-molecular pairs are scored along
-// folded diagonals (atom a with atom (a + d) mod natom), each atom keeping its
-// own pair forces in registers and passing the partner's share on by a lane
-// rotation (or, past 64 atoms, through a per-wave LDS tile); ligands of 33-64
-// atoms score them in packed steps of up to 63 pairs whose shares the atoms
-// gather by lane reads. No atomics anywhere. MFMA is not used: the physics is
-// gather and VALU work on chains of dependent operations, bound by latency at
-// the occupancy the registers and LDS allow.
+// dot products are wave reductions. Intra-molecular pairs of ligands of up to 64 atoms are scored in
+// packed steps, a pair per lane, whose shares the atoms collect through a per-wave LDS tile; past 64
+// atoms along folded diagonals (atom a with atom (a + d) mod natom), each atom keeping its own pair
+// forces in registers and passing the partner's share on through the tile. No atomics anywhere. MFMA is
+// not used: the physics is gather and VALU work on chains of dependent operations, bound by VALU issue,
+// the LDS pipe and latency together.
 //
 // The algorithm follows the reference's device code (E/ =
 // unidock/unidock_engine/): cal_e_f_tile / cal_grad_tile (E/src/cuda/bfgs.cuh:
@@ -121,6 +119,12 @@ __device__ __forceinline__ int tlane() { return TW == kWave ? __lane_id() : (__l
 template <int TW>
 __device__ __forceinline__ int tbase() { return TW == kWave ? 0 : (__lane_id() & ~(TW - 1)); }
 
+// A value that the compiler knows nothing of: it is rounded here and nothing is fused across.
+__device__ __forceinline__ float opaque(float v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
 // A value every lane of the tile agrees on: moved to a scalar register for a whole-wave tile, kept in
 // its vector register (one value per tile) otherwise. Either way the value is rounded and opaque at
 // this point: the compiler cannot fuse the operation that produced it into the ones that use it (a
@@ -130,8 +134,7 @@ __device__ __forceinline__ float tuni(float v) {
     if constexpr (TW == kWave) {
         return uni(v);
     } else {
-        asm("" : "+v"(v));
-        return v;
+        return opaque(v);
     }
 }
 
@@ -195,9 +198,13 @@ __device__ __forceinline__ void wave_lds_fence() {
 }
 
 // --------------------------------------------------------------- scoring
-// Vina::eval_ef (E/src/score/vina.h:216-245) for a heavy-atom pair with the
-// pair flags precomputed: bit0 both hydrophobic, bit1 hydrogen-bond capable.
-__device__ __forceinline__ float eval_ef(float d, int flags, float* dedd) {
+// Vina::eval_ef (E/src/score/vina.h:216-245) for a heavy-atom pair at surface distance d.
+// Written for CDNA4's issue rates: an FP32 add, multiply or FMA (its clamp to [0, 1] free) takes 2 cycles of a
+// SIMD, any compare, select, minimum or integer operation 4, a transcendental 8. So the ramps take their flags
+// from kh and kb instead of selects, the repulsion's min(d, 0) is -8 clamp(-d / 8) (d > -8; exact, as the
+// scaling by a power of two is), and a ramp r in (0, 1), where its derivative is not zero, is told by
+// r - r r > 0, which holds for exactly the d of the two compares with its ends.
+__device__ __forceinline__ float eval_ramps(float d, float kh, float kb, float* dedd) {
     // gauss1 (offset 0, width 0.5): exp(-4 d^2) = 2^(-4 log2(e) d^2), derivative -8 d exp(-4 d^2);
     // gauss2 (offset 3, width 2): exp(-(u / 2)^2) = 2^(-log2(e) / 4 u^2), u = d - 3, derivative -(u / 2) exp(..)
     const float e1 = __builtin_amdgcn_exp2f(-5.7707801635558535f * (d * d));
@@ -206,21 +213,24 @@ __device__ __forceinline__ float eval_ef(float d, int flags, float* dedd) {
     float e = msub2(-0.035579f, e1, 0.005156f, e2);
     float f = madd2((0.035579f * 8.0f) * d, e1, (0.005156f * 0.5f) * u, e2);
     // repulsion, d < 0
-    const float dn = fminf(d, 0.0f);
-    e = fmaf_(0.840245f * dn, dn, e);
-    f = fmaf_(0.840245f * 2.0f, dn, f);
+    const float m = fminf(fmaxf(d * -0.125f, 0.0f), 1.0f);
+    e = fmaf_((0.840245f * 64.0f) * m, m, e);
+    f = fmaf_(0.840245f * -16.0f, m, f);
     // hydrophobic, slope_interp(0.5, 1.5)
-    const float h = fminf(fmaxf(1.5f - d, 0.0f), 1.0f);
-    const bool hin = (flags & 1) && d > 0.5f && d < 1.5f;
-    e = fmaf_((flags & 1) ? -0.035069f : 0.0f, h, e);
-    f += hin ? 0.035069f : 0.0f;
+    const float h = fminf(fmaxf(kh - d, 0.0f), 1.0f);
+    e = fmaf_(-0.035069f, h, e);
+    f += fmaf_(-h, h, h) > 0.0f ? 0.035069f : 0.0f;
     // hydrogen bond, slope_interp(-0.7, 0)
-    const float b = fminf(fmaxf(-d * (1.0f / 0.7f), 0.0f), 1.0f);
-    const bool bin = (flags & 2) && d > -0.7f && d < 0.0f;
-    e = fmaf_((flags & 2) ? -0.587439f : 0.0f, b, e);
-    f += bin ? 0.587439f * (1.0f / 0.7f) : 0.0f;
+    const float b = fminf(fmaxf(d * kb, 0.0f), 1.0f);
+    e = fmaf_(-0.587439f, b, e);
+    f += fmaf_(-b, b, b) > 0.0f ? 0.587439f * (1.0f / 0.7f) : 0.0f;
     *dedd = f;
     return e;
+}
+
+// The same with the pair flags: bit0 both hydrophobic, bit1 hydrogen-bond capable.
+__device__ __forceinline__ float eval_ef(float d, int flags, float* dedd) {
+    return eval_ramps(d, ramp_hyd(flags), ramp_hb(flags), dedd);
 }
 
 __device__ __forceinline__ int pair_flags(int ti, int tj) {
@@ -942,32 +952,45 @@ __device__ __forceinline__ float bperm(int addr, float v) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(v)));
 }
 
-// One intra pair (bfgs.cuh:305-353): the energy gradient on atom i at (xi, yi, zi) (radius ri, pair-flag
-// table lut) from its partner, the LDS slot (x, y, z, radius) xj with doubled type flags fj2, under the
-// per-pair curl with cap v_cap; returns the curled pair energy, zero beyond the 8 A cutoff. The
-// partner's gradient is the negative.
-// The pair's separation (rx, ry, rz) = x_i - x_j, radius sum rs and pair flags fl (bit 0 both
-// hydrophobic, bit 1 a hydrogen-bond pair).
-__device__ __forceinline__ float pair_core(float rx, float ry, float rz, float rs, int fl, float v_cap, float& px,
-                                           float& py, float& pz) {
-    const float rr = sq_dist(rx, ry, rz);
+// Exchange of a vector per lane through the wave's pair-force tile (x, y and z, 64 floats each at f): every lane
+// puts its own, then reads those of any lanes by their byte offsets 4 * lane.
+__device__ __forceinline__ void share_put(int f, int ln, float x, float y, float z) {
+    wave_lds_fence();
+    s_lds[f + ln] = x;
+    s_lds[f + kWave + ln] = y;
+    s_lds[f + 2 * kWave + ln] = z;
+    wave_lds_fence();
+}
+__device__ __forceinline__ float3 share_get(int f, uint32_t off) {
+    const float* p = reinterpret_cast<const float*>(reinterpret_cast<const char*>(s_lds + f) + off);
+    return make_float3(p[0], p[kWave], p[2 * kWave]);
+}
+
+// One intra pair (bfgs.cuh:305-353) within the cutoff, at separation (rx, ry, rz) = x_i - x_j, its square rr,
+// radius sum rs and flag constants kh, kb: the curled pair energy and the energy gradient on i; the
+// partner's is the negative. The per-pair curl has cap v_cap.
+__device__ __forceinline__ float pair_core(float rx, float ry, float rz, float rr, float rs, float kh, float kb,
+                                           float v_cap, float& px, float& py, float& pz) {
     // r and 1 / r from one reciprocal square root; eps^2 keeps coincident atoms finite (it is below
     // half an ulp of any squared distance that is not tiny)
     const float inv = frsq(rr + kEps * kEps);
     float dd;
-    float ep = eval_ef(rr * inv - rs, fl, &dd);
-    // per-pair curl and the 8 A cutoff, branch-free
-    float cs = ep > 0.0f ? v_cap * frcp(v_cap + ep) : 1.0f;
-    const bool in = rr < kR2Cut;
-    ep = in ? ep * cs : 0.0f;
-    const float sc = in ? dd * inv * (cs * cs) : 0.0f;
+    const float ep = eval_ramps(fmaf_(rr, inv, -rs), kh, kb, &dd);
+    const float cs = ep > 0.0f ? v_cap * frcp(v_cap + ep) : 1.0f;
+    const float sc = dd * inv * (cs * cs);
     px = sc * rx; py = sc * ry; pz = sc * rz;
-    return ep;
+    return opaque(ep * cs);  // a rounded product, not fused into the sum it is added to
 }
 
+// The pair of an atom at (xi, yi, zi) (radius ri, pair-flag table lut) with the LDS slot (x, y, z, radius) xj of
+// doubled type flags fj2; zero beyond the 8 A cutoff.
 __device__ __forceinline__ float pair_grad(float xi, float yi, float zi, float ri, uint32_t lut, float4 xj, int fj2,
                                            float v_cap, float& px, float& py, float& pz) {
-    return pair_core(xi - xj.x, yi - xj.y, zi - xj.z, ri + xj.w, int(lut >> fj2) & 3, v_cap, px, py, pz);
+    const float rx = xi - xj.x, ry = yi - xj.y, rz = zi - xj.z;
+    const float rr = sq_dist(rx, ry, rz);
+    if (!(rr < kR2Cut)) return 0.0f;
+    const int fl = int(lut >> fj2) & 3;
+    return pair_core(rx, ry, rz, rr, ri + xj.w, ramp_hyd(fl), ramp_hb(fl), v_cap, px, py, pz);
 }
 
 // cal_e_f_tile (bfgs.cuh:221-394): energy under the curl cap v_cap and the
@@ -1079,95 +1102,68 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
         const float hi = ((rdl(r0, 32) + rdl(r0, 48)) + rdl(r1, 32)) + rdl(r1, 48);
         return (__lane_id() & 32) ? hi : lo;
     } else if constexpr (APL == 1) {
-        // intra-molecular pairs with the per-pair curl, each pair once, as folded diagonals: on
-        // diagonal d lane l scores the pair {l, (l + d) mod natom}; lane l keeps the pair gradient on
-        // its own atom in registers and hands the partner's share on by one lane rotation (the
-        // lane whose partner is l is (l - d) mod natom), so no LDS atomics are needed. Lanes past
-        // natom score nothing and their sums are never read.
+        // intra-molecular pairs with the per-pair curl, each pair once, in the packed steps of
+        // LigSetDev::pack: a lane scores at most one pair per step, and the atoms collect their shares from
+        // the wave's pair-force tile, so no LDS atomics are needed. Lanes past natom collect what is never
+        // read. The next step's entry is loaded while this one is scored (a step past the last is there).
+        // A step is bound by VALU issue (about 210 cycles of a SIMD) next to the LDS pipe (about 90
+        // cycles of a CU with the two 16-byte coordinate reads): the entries hold LDS offsets and flag
+        // constants, so that nothing is decoded or selected per pair, and twelve (nine) ds_bpermute per
+        // step, at 6 cycles of the LDS pipe each, are three writes and paired reads.
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
+        const char* tile = reinterpret_cast<const char*>(s_lds + C.lx);
+        const char* pk = reinterpret_cast<const char*>(C.L->pack + (size_t)C.pack_off * kWave);
+        uint32_t at = uint32_t(sizeof(uint4)) * uint32_t(ln);
+        uint4 t = *reinterpret_cast<const uint4*>(pk + at);
         if (n <= kWave / 2) {
-            // up to 32 atoms: two diagonals per step, lanes 0-31 on diagonal dg and lanes 32-63 on
-            // dg + 1, both for atom l % 32; lane a collects its atom's own share from lane a + 32
-            // and the partner shares of both diagonals. Partner and source indices advance by two
-            // per step (mod natom).
-            const int h = ln >> 5, a = ln & 31;
-            // atom a's coordinates and radius from the tile, its pair-flag table from lane a (the upper
-            // half's own atoms are past natom)
-            const float4 xa = lx4[a];
-            const uint32_t lut = uint32_t(__builtin_amdgcn_ds_bpermute(lane_addr(a), int(C.lut[0])));
-            int q = a + 1 + h;            // partner of atom a on diagonal 1 + h (mod natom)
-            q = q >= n ? q - n : q;
-            q = q >= n ? q - n : q;
-            int s0 = a - 1 < 0 ? a - 1 + n : a - 1;          // the lane whose partner on diagonal dg is a
-            int s1 = a - 2 < 0 ? a - 2 + n : a - 2;          // ... on diagonal dg + 1 (lanes 32-63)
-            s0 = s0 < 0 ? s0 + n : s0;
-            s1 = s1 < 0 ? s1 + n : s1;
-            const int own = lane_addr(a + 32);
-#pragma unroll 1
-            for (int dg = 1; dg <= C.nfold; dg += 2) {
-                const unsigned long long m0 = uload(fm + dg - 1);
-                const unsigned long long m1 = dg < C.nfold ? uload(fm + dg) : 0ull;
-                float px = 0.0f, py = 0.0f, pz = 0.0f;
-                if (__builtin_amdgcn_inverse_ballot_w64(m0 | (m1 << 32)))
-                    e += pair_grad(xa.x, xa.y, xa.z, xa.w, lut, lx4[q], lfl[q], v_cap, px, py, pz);
-                const float ox = bperm(own, px), oy = bperm(own, py), oz = bperm(own, pz);
-                const int b0 = lane_addr(s0), b1 = lane_addr(32 + s1);
-                const float b0x = bperm(b0, px), b0y = bperm(b0, py), b0z = bperm(b0, pz);
-                const float b1x = bperm(b1, px), b1y = bperm(b1, py), b1z = bperm(b1, pz);
-                ax += (px + ox) - (b0x + b1x);
-                ay += (py + oy) - (b0y + b1y);
-                az += (pz + oz) - (b0z + b1z);
-                q = q + 2 >= n ? q + 2 - n : q + 2;
-                s0 = s0 - 2 < 0 ? s0 - 2 + n : s0 - 2;
-                s1 = s1 - 2 < 0 ? s1 - 2 + n : s1 - 2;
-            }
-        } else if (C.npack > 0) {
-            // 33-64 atoms: the pairs packed up to 63 per step (LigSetDev::pack). Lane l scores the pair
-            // {i, j} of its entry from the coordinate tile, and atom l collects +p from the (at most
-            // two) lanes where it is i and -p from those where it is j; lane 63 scores nothing and
-            // stands for no lane. The next step's entry is loaded while this one is scored.
-            const uint2* pk = C.L->pack + (size_t)C.pack_off * kWave + ln;
-            uint2 t = pk[0];
+            // up to 32 atoms: two folded diagonals per step, lanes 0-31 the pairs {a, (a + d) mod natom} of
+            // diagonal d, lanes 32-63 those of d + 1, a the lane mod 32; lane a collects its atom's own share
+            // from lane a + 32 and the partner shares of both diagonals
+            const float4 xa = lx4[ln & 31];
+            const uint32_t own = 4u * uint32_t((ln & 31) + 32);
 #pragma unroll 1
             for (int st = 0; st < C.npack; st++) {
-                const uint2 tn = pk[(st + 1 < C.npack ? st + 1 : st) * kWave];
+                at += uint32_t(sizeof(uint4)) * kWave;
+                const uint4 tn = *reinterpret_cast<const uint4*>(pk + at);
                 float px = 0.0f, py = 0.0f, pz = 0.0f;
-                if (t.x >> 31) {
-                    const float4 xi = lx4[t.x & 0xff], xj = lx4[(t.x >> 8) & 0xff];
-                    e += pair_core(xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, xi.w + xj.w, int(t.x >> 16) & 3, v_cap,
-                                   px, py, pz);
-                }
-                const int s0 = int(t.y & 0xffu), s1 = int((t.y >> 8) & 0xffu);
-                const int s2 = int((t.y >> 16) & 0xffu), s3 = int(t.y >> 24);
-                // the twelve lane reads go out together, then the sums (one LDS round trip per step)
-                const float a0x = bperm(s0, px), a0y = bperm(s0, py), a0z = bperm(s0, pz);
-                const float a1x = bperm(s1, px), a1y = bperm(s1, py), a1z = bperm(s1, pz);
-                const float b0x = bperm(s2, px), b0y = bperm(s2, py), b0z = bperm(s2, pz);
-                const float b1x = bperm(s3, px), b1y = bperm(s3, py), b1z = bperm(s3, pz);
-                __builtin_amdgcn_sched_group_barrier(0x0080, 12, 0);
-                __builtin_amdgcn_sched_group_barrier(0x0002, 16, 0);
-                ax += (a0x + a1x) - (b0x + b1x);
-                ay += (a0y + a1y) - (b0y + b1y);
-                az += (a0z + a1z) - (b0z + b1z);
+                const float4 xj = *reinterpret_cast<const float4*>(tile + (t.x & 0xffffu));
+                const float rx = xa.x - xj.x, ry = xa.y - xj.y, rz = xa.z - xj.z;
+                const float rr = sq_dist(rx, ry, rz), rs = opaque(xa.w + xj.w);
+                if (__uint_as_float(t.z) < kRampNoPair && rr < kR2Cut)
+                    e += pair_core(rx, ry, rz, rr, rs, __uint_as_float(t.z), __uint_as_float(t.w), v_cap, px,
+                                   py, pz);
+                share_put(C.lf, ln, px, py, pz);
+                const float3 o = share_get(C.lf, own), b0 = share_get(C.lf, t.y & 0xffu),
+                             b1 = share_get(C.lf, (t.y >> 8) & 0xffu);
+                ax += (px + o.x) - (b0.x + b1.x);
+                ay += (py + o.y) - (b0.y + b1.y);
+                az += (pz + o.z) - (b0.z + b1.z);
                 t = tn;
             }
         } else {
-            // one diagonal per step (33-64 atoms without packed steps: a ligand with no scored pairs)
-            int q = ln + 1 >= n ? ln + 1 - n : ln + 1;       // partner on diagonal 1 (ln <= 63 < 2 n)
-            int src = ln - 1 < 0 ? n - 1 : (ln - 1 >= n ? ln - 1 - n : ln - 1);
+            // 33-64 atoms: up to 63 pairs {i, j} of a step, lane l scores the one of its entry, and atom l
+            // collects +p from the (at most two) lanes where it is i and -p from those where it is j; lane
+            // 63 scores nothing and stands for no lane
 #pragma unroll 1
-            for (int dg = 1; dg <= C.nfold; dg++) {
-                const unsigned long long m = uload(fm + dg - 1);
+            for (int st = 0; st < C.npack; st++) {
+                at += uint32_t(sizeof(uint4)) * kWave;
+                const uint4 tn = *reinterpret_cast<const uint4*>(pk + at);
                 float px = 0.0f, py = 0.0f, pz = 0.0f;
-                if (__builtin_amdgcn_inverse_ballot_w64(m))
-                    e += pair_grad(P.x[0], P.y[0], P.z[0], C.rad[0], C.lut[0], lx4[q], lfl[q], v_cap, px, py, pz);
-                const int b = lane_addr(src);
-                const float bx = bperm(b, px), by = bperm(b, py), bz = bperm(b, pz);
-                ax += px - bx;
-                ay += py - by;
-                az += pz - bz;
-                q = q + 1 == n ? 0 : q + 1;
-                src = src == 0 ? n - 1 : src - 1;
+                const float4 xi = *reinterpret_cast<const float4*>(tile + (t.x & 0xffffu)),
+                             xj = *reinterpret_cast<const float4*>(tile + (t.x >> 16));
+                const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
+                // the radii with the coordinates, as 16-byte loads (12 bytes take the LDS pipe longer than 16)
+                const float rr = sq_dist(rx, ry, rz), rs = opaque(xi.w + xj.w);
+                if (__uint_as_float(t.z) < kRampNoPair && rr < kR2Cut)
+                    e += pair_core(rx, ry, rz, rr, rs, __uint_as_float(t.z), __uint_as_float(t.w), v_cap, px,
+                                   py, pz);
+                share_put(C.lf, ln, px, py, pz);
+                const float3 a0 = share_get(C.lf, t.y & 0xffu), a1 = share_get(C.lf, (t.y >> 8) & 0xffu);
+                const float3 b0 = share_get(C.lf, (t.y >> 16) & 0xffu), b1 = share_get(C.lf, t.y >> 24);
+                ax += (a0.x + a1.x) - (b0.x + b1.x);
+                ay += (a0.y + a1.y) - (b0.y + b1.y);
+                az += (a0.z + a1.z) - (b0.z + b1.z);
+                t = tn;
             }
         }
         fx[0] += ax; fy[0] += ay; fz[0] += az;

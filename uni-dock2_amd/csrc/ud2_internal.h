@@ -25,6 +25,14 @@ __host__ __device__ constexpr int mc_variant_tw(int v) { return v == kMcWhole ? 
 constexpr int kMcHeads = kMcVariants + kMaxApl - 1;
 constexpr int kNumTypes = 21;
 
+// A pair's flag terms as two constants of eval_ramps: kh is 1.5 for a hydrophobic pair, else so low that the
+// hydrophobic ramp clamp(kh - d) is zero at any distance; kb is -1 / 0.7 for a hydrogen-bond pair,
+// else 0, and the ramp clamp(kb d) with it.
+constexpr float kRampHyd = 1.5f, kRampNone = -1e30f, kRampHb = -(1.0f / 0.7f);
+constexpr float kRampNoPair = 4.0f;  // kh of a lane that scores no pair (packed steps)
+__host__ __device__ constexpr float ramp_hyd(int flags) { return (flags & 1) ? kRampHyd : kRampNone; }
+__host__ __device__ constexpr float ramp_hb(int flags) { return (flags & 2) ? kRampHb : 0.0f; }
+
 // One ligand of a ligand set on the device.
 struct DevLig {
     int32_t natom, ntors, npair, nheavy;
@@ -55,13 +63,16 @@ struct LigSetDev {
     // pair (for even natom, diagonal natom / 2 only for atoms below natom / 2, so every pair
     // appears once).
     const unsigned long long* fold_mask;
-    // Packed pair steps of ligands of 33-64 atoms: per step one entry per lane, .x = i | j << 8 |
-    // pair flags << 16 | 1 << 31 when lane l scores the pair {i, j} (gradient +p on i, -p on j) in this
-    // step (lanes 0 .. 62 only), .y = four byte addresses (lane * 4) of the lanes whose p atom l
-    // collects: bytes 0-1 lanes where l is i (+p), bytes 2-3 lanes where l is j (-p); lane 63, which
-    // scores nothing, stands for none. Every atom is i of at most two pairs and j of at most two per
-    // step.
-    const uint2* pack;
+    // Pair steps of the one-atom-per-lane ligands, one entry per lane and step. Lane l scores the pair {i, j}
+    // (gradient +p on i, -p on j) of .x = 16 i | 16 j << 16 (their LDS offsets), with the flag constants
+    // kh = .z and kb = .w (ramp_hyd, ramp_hb; kh = kRampNoPair: no pair), and collects the p of the lanes
+    // whose byte offsets 4 * lane .y holds.
+    // 33-64 atoms: up to 63 pairs per step in any order, lanes 0 .. 62; every atom is i of at most two and j of at
+    // most two: bytes 0-1 of .y the lanes where atom l is i, bytes 2-3 those where it is j, lane 63, which
+    // scores nothing, for none.
+    // Up to 32 atoms: the folded diagonals 2 s + 1 (lanes 0-31) and 2 s + 2 (lanes 32-63) in step s, i the lane mod
+    // 32 and .x = 16 j; bytes 0-1 of .y the two lanes where atom l is j.
+    const uint4* pack;
     // Bias sites (FlexParamVina::inds_bias / params_bias, E/src/cuda/task.cu:157-168)
     // and the task options that change the search (DockParam, E/src/model/model.h:151-168).
     const int32_t* bias_start;             // [atoms + 1] CSR over the set's atoms; null: no sites
