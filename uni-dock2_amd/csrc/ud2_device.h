@@ -115,7 +115,11 @@ __device__ __forceinline__ float uni(float v) {
 
 // Lane index within the tile, and the tile's first lane in the wave.
 template <int TW>
-__device__ __forceinline__ int tlane() { return TW == kWave ? __lane_id() : (__lane_id() & (TW - 1)); }
+__device__ __forceinline__ int tlane() {
+    int l = __lane_id();
+    asm volatile("" : "+v"(l));
+    return TW == kWave ? l : (l & (TW - 1));
+}
 template <int TW>
 __device__ __forceinline__ int tbase() { return TW == kWave ? 0 : (__lane_id() & ~(TW - 1)); }
 
@@ -186,6 +190,30 @@ template <int TW>
 __device__ __forceinline__ unsigned long long tmask(unsigned long long m) {
     if constexpr (TW == kWave) return m;
     else return (m & 0xffffffffull) | (m << 32);
+}
+
+// A kernel's arguments, read where they are used. Taken by value, the compiler loads them all at the kernel's
+// entry, and with the addresses and constants that it also forms there, they overflow the 102 SGPRs
+// into lanes of vector registers and those into scratch memory (the six-wave learned search kernel: 246 SGPRs and
+// 90 VGPRs spilled, 2 TB/s of HBM traffic mostly for them). reread() makes the compiler forget a value's
+// origin, so that nothing read through it is hoisted out of the function (tlane does the same for LDS
+// addresses): 20 and 36 spilled, the 1,024-ligand learned search 371 -> 331 ms, the MC kernel's SGPR spills
+// 157 -> 0 and its registers without spills 123 -> 95.
+template <class T>
+using Karg = const __attribute__((address_space(4))) T;
+using KHead = Karg<ArgHead>;
+using KLig = Karg<DevLig>;
+using LigArg = Karg<LigSetDev>;
+using SceneArg = Karg<SceneDev>;
+
+template <class T>
+__device__ __forceinline__ T reread(T v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+template <class T>
+__device__ __forceinline__ Karg<T>* kernel_args() {
+    return (Karg<T>*)__builtin_amdgcn_kernarg_segment_ptr();
 }
 
 // Dynamic LDS of a launch; every wave owns a slice of it.
@@ -284,7 +312,7 @@ struct Reach {
     bool whole;
 };
 
-__device__ __forceinline__ Reach reach_of(const SceneDev& S, float px, float py, float pz) {
+__device__ __forceinline__ Reach reach_of(SceneArg& S, float px, float py, float pz) {
     const float gx = (px - S.rorigin[0]) * S.rinv, gy = (py - S.rorigin[1]) * S.rinv, gz = (pz - S.rorigin[2]) * S.rinv;
     Reach r{0, 0, false};
     if (gx >= 0.0f && gx < float(S.rn[0]) && gy >= 0.0f && gy < float(S.rn[1]) && gz >= 0.0f && gz < float(S.rn[2])) {
@@ -305,7 +333,7 @@ __device__ __forceinline__ Reach reach_of(const SceneDev& S, float px, float py,
 // 57-atom ligand 1,266 -> 238 us, the re-score and decomposition of 10,210 poses 982 -> 152 us, a
 // direct-mode search of 8 ligands 745 -> 43 ms.
 template <class F>
-__device__ __forceinline__ void for_reach(const SceneDev& S, const Reach& r, F f) {
+__device__ __forceinline__ void for_reach(SceneArg& S, const Reach& r, F f) {
     for (int j = r.begin; j < r.end; j += kReachPad) {
         float4 q[kReachPad];
 #pragma unroll
@@ -419,7 +447,7 @@ __device__ __forceinline__ float3 orient_grad(float v0, float v1, float v2, floa
 }
 
 // Trilinear value and gradient of map `slot` at p; clamped axes have zero derivative.
-__device__ __forceinline__ float grid_eval(const SceneDev& S, int slot, float px, float py, float pz, float& gx,
+__device__ __forceinline__ float grid_eval(SceneArg& S, int slot, float px, float py, float pz, float& gx,
                                           float& gy, float& gz) {
     float g[3] = {(px - S.gorigin[0]) * S.ginv, (py - S.gorigin[1]) * S.ginv, (pz - S.gorigin[2]) * S.ginv};
     int i0[3];
@@ -464,51 +492,70 @@ struct WPose {
     float e;            // energy (uniform)
 };
 
-// Per-tile constants of the ligand being processed. The tile's LDS slice
+// Per-tile constants of the ligand being processed: its descriptor and the kernel's arguments are read
+// where they are used (see reread), the lane's own values are kept. The tile's LDS slice
 // (offsets in floats into s_lds) holds: lx float4 coordinates [TW*APL], lf
 // pair-force tile [3][TW*APL], lo a saved pose, lt the ligand's torsion table,
 // lh the inverse Hessian (row i at lh + i * ld).
-template <int APL, int TW = kWave>
+template <int APL, int TW = kWave, bool LAZY = true>
 struct Ctx {
-    int natom, ntors, npair, nheavy, dim;
-    int atom_off, tors_off, pair_off;
-    int leaf_first;     // the torsion table's order is leaf-first (see apply_update)
-    int nfold, fold_off;  // folded pair diagonals (one-slot ligands)
-    int npack, pack_off;  // packed pair steps (ligands of 33-64 atoms)
+    KHead* K;
+    KLig* lig;
+    int base, ld;
     int type[APL];      // XS type; -1 for lanes beyond natom
     int slot[APL];      // grid map of the atom's type
     float rad[APL];     // vdW radius of the atom's type (0 beyond natom)
     uint32_t lut[APL];  // pair flags with a partner of doubled type flags f: (lut >> f) & 3 (see pair_lut)
-    int lx, lf, lo, lfl, lt, lh, ld;
-    const LigSetDev* L;
-    const SceneDev* S;
     int mode;
     mutable int evals;  // energy evaluations of the current work item
     bool stage;         // pose updates may stage torsion steps in the coordinate / pair-force area
+
+    // LAZY: read where used; else left to the compiler to load once and keep, which a kernel that has
+    // registers to spare and no other waves to hide a scalar load behind runs faster with.
+    template <class T>
+    static __device__ __forceinline__ T lazy(T v) {
+        if constexpr (LAZY) return reread(v);
+        else return v;
+    }
+    __device__ __forceinline__ LigArg& L() const { return lazy(K)->L; }
+    __device__ __forceinline__ SceneArg& S() const { return lazy(K)->S; }
+    __device__ __forceinline__ KLig& d() const { return *lazy(lig); }
+    __device__ __forceinline__ bool biased() const {
+        LigArg& l = L();
+        return l.bias_type != 0 && l.bias_start;
+    }
+    __device__ __forceinline__ int natom() const { return d().natom; }
+    __device__ __forceinline__ int ntors() const { return d().ntors; }
+    __device__ __forceinline__ int npair() const { return d().npair; }
+    __device__ __forceinline__ int nheavy() const { return d().nheavy; }
+    __device__ __forceinline__ int dim() const { return 6 + d().ntors; }
+    __device__ __forceinline__ int lx() const {
+        if constexpr (TW == kWave) return lazy(base);
+        else return base;
+    }
+    __device__ __forceinline__ int lf() const { return lx() + 4 * TW * APL; }
+    __device__ __forceinline__ int lo() const { return lx() + 7 * TW * APL; }
+    __device__ __forceinline__ int lfl() const { return lx() + lds_flags_offset(APL, TW); }
+    __device__ __forceinline__ int lt() const { return lx() + lds_fixed_floats(APL, TW); }
+    __device__ __forceinline__ int lh() const { return lx() + lds_head_floats(APL, ld, TW); }
 };
 
-template <int APL, int TW>
-__device__ __forceinline__ void load_ctx(Ctx<APL, TW>& C, const LigSetDev& L, const SceneDev& S, int lig, int mode,
-                                         int base, int ld) {
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void load_ctx(Ctx<APL, TW, LAZY>& C, KHead* K, int lig, int mode, int base, int ld) {
     static_assert(TW == kWave || APL == 1, "a tile narrower than the wave holds one atom per lane");
     const int tl = tlane<TW>();
-    const DevLig d = L.ligs[lig];
-    C.natom = d.natom; C.ntors = d.ntors; C.npair = d.npair; C.nheavy = d.nheavy;
-    C.dim = 6 + d.ntors;
-    C.atom_off = d.atom_off; C.tors_off = d.tors_off; C.pair_off = d.pair_off;
-    C.leaf_first = d.leaf_first;
-    C.nfold = d.nfold; C.fold_off = d.fold_off;
-    C.npack = d.npack; C.pack_off = d.pack_off;
-    C.L = &L; C.S = &S; C.mode = mode;
+    // the same for every lane of the wave (base: of the tile)
+    C.K = K;
+    C.lig = (KLig*)(K->L.ligs + __builtin_amdgcn_readfirstlane(lig));
+    C.base = TW == kWave ? __builtin_amdgcn_readfirstlane(base) : base;
+    C.ld = ld;
+    C.mode = mode;
     C.evals = 0;
     C.stage = true;
-    C.lx = base;
-    C.lf = base + 4 * TW * APL;
-    C.lo = base + 7 * TW * APL;
-    C.lfl = base + lds_flags_offset(APL, TW);
-    C.lt = base + lds_fixed_floats(APL, TW);
-    C.lh = base + lds_head_floats(APL, ld, TW);
-    C.ld = ld;
+    LigArg& L = C.L();
+    SceneArg& S = C.S();
+    KLig& d = C.d();
+    const int lfl = C.lfl(), lt = C.lt();
 #pragma unroll
     for (int k = 0; k < APL; k++) {
         int a = tl + TW * k;
@@ -519,7 +566,7 @@ __device__ __forceinline__ void load_ctx(Ctx<APL, TW>& C, const LigSetDev& L, co
         C.lut[k] = pair_lut(fa);
         // the atom's doubled type flags, read by its pair partners; this part of the slice is not
         // overlaid by anything else, so it is written once per work item
-        reinterpret_cast<int*>(s_lds + C.lfl)[a] = 2 * fa;
+        reinterpret_cast<int*>(s_lds + lfl)[a] = 2 * fa;
     }
     // torsion table: lane t copies torsion t once, so the kinematics and the gradient read
     // the torsion tree from LDS instead of global memory on every step
@@ -528,7 +575,7 @@ __device__ __forceinline__ void load_ctx(Ctx<APL, TW>& C, const LigSetDev& L, co
         const int2 ax = L.tors_axis[tg];
         const int2 rr = L.tors_range[tg];
         const float2 r0 = L.ranges[rr.x];
-        float* e = s_lds + C.lt + tl * tors_entry_floats(APL);
+        float* e = s_lds + lt + tl * tors_entry_floats(APL);
         // from | to << 8 | order << 16 | rank << 24 (atoms < 256, torsions < 64)
         const int word = (ax.x & 0xff) | ((ax.y & 0xff) << 8) | (((ax.y >> 16) & 0xff) << 16) | (((ax.x >> 16) & 0xff) << 24);
         *reinterpret_cast<float4*>(e) = make_float4(__int_as_float(word), __int_as_float(rr.y), r0.x, r0.y);
@@ -549,9 +596,9 @@ struct TorsEnt {
     float lo, hi;
 };
 
-template <int APL, int TW>
-__device__ __forceinline__ TorsEnt tors_ent(const Ctx<APL, TW>& C, int t) {
-    const float4 h = *reinterpret_cast<const float4*>(s_lds + C.lt + t * tors_entry_floats(APL));
+template <int APL>
+__device__ __forceinline__ TorsEnt tors_ent_at(int lt, int t) {
+    const float4 h = *reinterpret_cast<const float4*>(s_lds + lt + t * tors_entry_floats(APL));
     const int ax = __float_as_int(h.x);
     TorsEnt e;
     e.from = ax & 0xff;
@@ -564,17 +611,24 @@ __device__ __forceinline__ TorsEnt tors_ent(const Ctx<APL, TW>& C, int t) {
     return e;
 }
 
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ TorsEnt tors_ent(const Ctx<APL, TW, LAZY>& C, int t) { return tors_ent_at<APL>(C.lt(), t); }
+
 // Rotated-atom mask of torsion t over atom slot k (bit l = atom l + 64 k).
-template <int APL, int TW>
-__device__ __forceinline__ unsigned long long tors_mask(const Ctx<APL, TW>& C, int t, int k) {
-    const float2 m = *reinterpret_cast<const float2*>(s_lds + C.lt + t * tors_entry_floats(APL) + 4 + 2 * k);
+template <int APL>
+__device__ __forceinline__ unsigned long long tors_mask_at(int lt, int t, int k) {
+    const float2 m = *reinterpret_cast<const float2*>(s_lds + lt + t * tors_entry_floats(APL) + 4 + 2 * k);
     return (unsigned long long)__float_as_uint(m.x) | ((unsigned long long)__float_as_uint(m.y) << 32);
 }
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ unsigned long long tors_mask(const Ctx<APL, TW, LAZY>& C, int t, int k) {
+    return tors_mask_at<APL>(C.lt(), t, k);
+}
 
-template <int APL, int TW>
-__device__ __forceinline__ bool heavy(const Ctx<APL, TW>& C, int k) { return C.type[k] > kTypeH; }
-template <int APL, int TW>
-__device__ __forceinline__ bool valid(const Ctx<APL, TW>& C, int k) { return C.type[k] >= 0; }
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ bool heavy(const Ctx<APL, TW, LAZY>& C, int k) { return C.type[k] > kTypeH; }
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ bool valid(const Ctx<APL, TW, LAZY>& C, int k) { return C.type[k] >= 0; }
 
 // Position of atom a (tile lane a % TW, slot a / TW), a the same for every lane of the tile.
 template <int TW, int APL>
@@ -587,13 +641,13 @@ __device__ __forceinline__ float3 atom_pos(const WPose<APL>& P, int a) {
     return r;
 }
 
-template <int APL, int TW>
-__device__ __forceinline__ void centroid(const Ctx<APL, TW>& C, WPose<APL>& P) {
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void centroid(const Ctx<APL, TW, LAZY>& C, WPose<APL>& P) {
     float sx = 0.0f, sy = 0.0f, sz = 0.0f;
 #pragma unroll
     for (int k = 0; k < APL; k++)
         if (valid(C, k)) { sx += P.x[k]; sy += P.y[k]; sz += P.z[k]; }
-    const float inv = 1.0f / float(C.natom);
+    const float inv = 1.0f / float(C.natom());
     P.c0 = tuni<TW>(tsum<TW>(sx) * inv);
     P.c1 = tuni<TW>(tsum<TW>(sy) * inv);
     P.c2 = tuni<TW>(tsum<TW>(sz) * inv);
@@ -602,13 +656,13 @@ __device__ __forceinline__ void centroid(const Ctx<APL, TW>& C, WPose<APL>& P) {
 // Pose slots in the wave's LDS slice: slot 0 parks the BFGS start pose, slot 1
 // the accepted MC pose. A slot holds x, y, z per atom and the dihedrals per lane,
 // then c, rot_vec and the energy.
-template <int APL, int TW>
-__device__ __forceinline__ int pose_slot(const Ctx<APL, TW>& C, int slot) {
-    return C.lo + slot * (TW * (3 * APL + 1) + 8);
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ int pose_slot(const Ctx<APL, TW, LAZY>& C, int slot) {
+    return C.lo() + slot * (TW * (3 * APL + 1) + 8);
 }
 
-template <int APL, int TW>
-__device__ __forceinline__ void save_pose(const Ctx<APL, TW>& C, const WPose<APL>& P, int slot = 0) {
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void save_pose(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& P, int slot = 0) {
     const int ln = tlane<TW>();
     const int lo = pose_slot(C, slot);
 #pragma unroll
@@ -626,8 +680,8 @@ __device__ __forceinline__ void save_pose(const Ctx<APL, TW>& C, const WPose<APL
     }
 }
 
-template <int APL, int TW>
-__device__ __forceinline__ void restore_pose(const Ctx<APL, TW>& C, WPose<APL>& P, int slot = 0) {
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void restore_pose(const Ctx<APL, TW, LAZY>& C, WPose<APL>& P, int slot = 0) {
     wave_lds_fence();
     const int ln = tlane<TW>();
     const int lo = pose_slot(C, slot);
@@ -645,7 +699,7 @@ __device__ __forceinline__ void restore_pose(const Ctx<APL, TW>& C, WPose<APL>& 
 }
 
 // clamp_by_ranges (E/src/myutils/mymath.h:133-158) over the torsion's ranges.
-__device__ __forceinline__ float clamp_ranges(const LigSetDev& L, int tg, float ang) {
+__device__ __forceinline__ float clamp_ranges(LigArg& L, int tg, float ang) {
     const int2 rr = L.tors_range[tg];
     for (int i = 0; i < rr.y; i++) {
         const float2 r = L.ranges[rr.x + i];
@@ -662,9 +716,9 @@ __device__ __forceinline__ float clamp_ranges(const LigSetDev& L, int tg, float 
 }
 
 // clamp_ranges of torsion t from its table entry: one allowed range inline, more from global memory.
-template <int APL, int TW>
-__device__ __forceinline__ float clamp_tors(const Ctx<APL, TW>& C, const TorsEnt& e, int tg, float ang) {
-    if (e.nrange != 1) return clamp_ranges(*C.L, tg, ang);
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ float clamp_tors(const Ctx<APL, TW, LAZY>& C, const TorsEnt& e, int tg, float ang) {
+    if (e.nrange != 1) return clamp_ranges(C.L(), tg, ang);
     if (ang >= e.lo && ang <= e.hi) return ang;
     const float dl = fabsf(ang - e.lo), dh = fabsf(ang - e.hi);
     float best = ang, md = 100.0f;
@@ -676,9 +730,9 @@ __device__ __forceinline__ float clamp_tors(const Ctx<APL, TW>& C, const TorsEnt
 // One torsion step, apply_grad_update_dihe_tile (E/src/cuda/bfgs.cuh:443-527);
 // the centroid is refreshed by the caller after the last torsion (only the
 // final centroid is ever read, bfgs.cuh:531-548, 576-578).
-template <int APL, int TW>
-__device__ __forceinline__ void apply_torsion(const Ctx<APL, TW>& C, WPose<APL>& P, int t, float inc_raw) {
-    const int tg = C.tors_off + t;
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void apply_torsion(const Ctx<APL, TW, LAZY>& C, WPose<APL>& P, int t, float inc_raw) {
+    const int tg = C.d().tors_off + t;
     const TorsEnt te = tors_ent(C, t);
     const float dt = tread<TW>(P.dihe, t);
     float inc = normalize_angle(inc_raw);
@@ -709,8 +763,8 @@ __device__ __forceinline__ void apply_torsion(const Ctx<APL, TW>& C, WPose<APL>&
 }
 
 // Rigid rotation about o by q, then translation so that o maps to n.
-template <int APL, int TW>
-__device__ __forceinline__ void rigid_move(const Ctx<APL, TW>& C, WPose<APL>& P, float4 q, float ox, float oy, float oz,
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void rigid_move(const Ctx<APL, TW, LAZY>& C, WPose<APL>& P, float4 q, float ox, float oy, float oz,
                                            float nx, float ny, float nz) {
     Mat3 R = quat_to_mat(q);
 #pragma unroll
@@ -753,22 +807,22 @@ static_assert(tstage_cap<1, kTileNarrow>() == kTileNarrowTors, "narrow tiles tak
 // steps are staged in LDS in application order and the rotations then read them with broadcast LDS
 // loads (no VALU work per value), each masked atom moved as R (x - p) + p. Ligands with more
 // torsions than the stage holds read the steps from the torsion lanes instead.
-template <int APL, int TW>
-__device__ __forceinline__ void apply_torsions_leaf_first(const Ctx<APL, TW>& C, WPose<APL>& P, float dir, float alpha) {
-    const int ln = tlane<TW>();
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void apply_torsions_leaf_first(const Ctx<APL, TW, LAZY>& C, WPose<APL>& P, float dir, float alpha) {
+    const int ln = tlane<TW>(), nt = C.ntors();
     const float inc_raw = tshfl<TW>(dir, ln + 6) * alpha;  // torsion components sit on lanes 6 + t
     // every lane reads an entry (lanes past ntors read entry 0) and gathers its axis atoms
-    const TorsEnt te = tors_ent(C, ln < C.ntors ? ln : 0);
+    const TorsEnt te = tors_ent(C, ln < nt ? ln : 0);
     const float3 xt = lane_gather<TW>(P, te.to), xf = lane_gather<TW>(P, te.from);
     float px = 0.0f, py = 0.0f, pz = 0.0f, ux = 1.0f, uy = 0.0f, uz = 0.0f, c = 1.0f, s = 0.0f;
     int ord = 0;
     uint32_t mlo[APL], mhi[APL];
 #pragma unroll
     for (int k = 0; k < APL; k++) mlo[k] = mhi[k] = 0u;
-    if (ln < C.ntors) {
+    if (ln < nt) {
         ord = te.ord;
         float inc = normalize_angle(inc_raw);
-        const float nw = clamp_tors(C, te, C.tors_off + ln, normalize_angle(P.dihe + inc));
+        const float nw = clamp_tors(C, te, C.d().tors_off + ln, normalize_angle(P.dihe + inc));
         inc = nw - P.dihe;
         P.dihe = nw;
         px = xt.x; py = xt.y; pz = xt.z;
@@ -786,12 +840,13 @@ __device__ __forceinline__ void apply_torsions_leaf_first(const Ctx<APL, TW>& C,
             mhi[k] = uint32_t(m >> 32);
         }
     }
-    if (C.stage && C.ntors <= tstage_cap<APL, TW>()) {
+    if (C.stage && nt <= tstage_cap<APL, TW>()) {
         constexpr int SE = tstage_floats<APL>();
-        if (ln < C.ntors) {
+        const int lx = C.lx();
+        if (ln < nt) {
             // Rodrigues: R = c I + s [u]x + (1 - c) u u^T
             const float oc = 1.0f - c;
-            float* st = s_lds + C.lx + te.rank * SE;
+            float* st = s_lds + lx + te.rank * SE;
             const float ox = oc * ux, oy = oc * uy, oz = oc * uz;
             reinterpret_cast<float4*>(st)[0] =
                 make_float4(fmaf_(ox, ux, c), msub2(ox, uy, s, uz), madd2(ox, uz, s, uy), madd2(oy, ux, s, uz));
@@ -806,8 +861,8 @@ __device__ __forceinline__ void apply_torsions_leaf_first(const Ctx<APL, TW>& C,
         }
         wave_lds_fence();
 #pragma unroll 1
-        for (int q = 0; q < C.ntors; q++) {
-            const float* st = s_lds + C.lx + q * SE;
+        for (int q = 0; q < nt; q++) {
+            const float* st = s_lds + lx + q * SE;
             const float4 r0 = reinterpret_cast<const float4*>(st)[0], r1 = reinterpret_cast<const float4*>(st)[1],
                          r2 = reinterpret_cast<const float4*>(st)[2];
 #pragma unroll
@@ -827,7 +882,7 @@ __device__ __forceinline__ void apply_torsions_leaf_first(const Ctx<APL, TW>& C,
         return;
     }
 #pragma unroll 1
-    for (int q = 0; q < C.ntors; q++) {
+    for (int q = 0; q < nt; q++) {
         if constexpr (TW == kWave) {
             const int t = rdl_i(ord, q);
             const float tx = rdl(px, t), ty = rdl(py, t), tz = rdl(pz, t);
@@ -868,16 +923,17 @@ __device__ __forceinline__ void apply_torsions_leaf_first(const Ctx<APL, TW>& C,
 // ligand's torsion tree allows it, else in index order), then centre += alpha *
 // dir[0..2] and a rotation by q(alpha * dir[3..5]) about the old centre;
 // rot_vec := alpha * dir[3..5]. dir is lane-distributed.
-template <int APL, int TW>
-__device__ __forceinline__ void apply_update(const Ctx<APL, TW>& C, WPose<APL>& P, float dir, float alpha) {
-    if (C.leaf_first) {
-        if (C.ntors > 0) apply_torsions_leaf_first(C, P, dir, alpha);
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void apply_update(const Ctx<APL, TW, LAZY>& C, WPose<APL>& P, float dir, float alpha) {
+    const int nt = C.ntors();
+    if (C.d().leaf_first) {
+        if (nt > 0) apply_torsions_leaf_first(C, P, dir, alpha);
     } else {
 #pragma unroll 1
-        for (int t = 0; t < C.ntors; t++) apply_torsion(C, P, t, trdl<TW>(dir, 6 + t) * alpha);
+        for (int t = 0; t < nt; t++) apply_torsion(C, P, t, trdl<TW>(dir, 6 + t) * alpha);
     }
-    if (C.ntors > 0) centroid(C, P);
-    if (C.L->constraint) return;  // constraint docking: no rigid step (bfgs.cuh:571)
+    if (nt > 0) centroid(C, P);
+    if (C.L().constraint) return;  // constraint docking: no rigid step (bfgs.cuh:571)
     const float o0 = P.c0, o1 = P.c1, o2 = P.c2;
     P.c0 = tuni<TW>(o0 + alpha * trdl<TW>(dir, 0));
     P.c1 = tuni<TW>(o1 + alpha * trdl<TW>(dir, 1));
@@ -919,14 +975,14 @@ __device__ __forceinline__ float bias_site_energy(int bias_type, float bias_k, f
 
 // Bias sites of every atom (hydrogens included), uncurled (the bias block of
 // cal_e_f_tile, bfgs.cuh:355-388): returns this lane's energy and adds dE/dx to F.
-template <int APL, int TW>
-__device__ __forceinline__ float bias_forces(const Ctx<APL, TW>& C, const WPose<APL>& P, Forces<APL>& F) {
-    const LigSetDev& L = *C.L;
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ float bias_forces(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& P, Forces<APL>& F) {
+    LigArg& L = C.L();
     float e = 0.0f;
 #pragma unroll
     for (int k = 0; k < APL; k++) {
         if (!valid(C, k)) continue;
-        const int a = C.atom_off + tlane<TW>() + TW * k;
+        const int a = C.d().atom_off + tlane<TW>() + TW * k;
         const int j1 = L.bias_start[a + 1];
         for (int j = L.bias_start[a]; j < j1; j++) {
             const float4 b = L.bias_site[j];
@@ -995,11 +1051,12 @@ __device__ __forceinline__ float pair_grad(float xi, float yi, float zi, float r
 
 // cal_e_f_tile (bfgs.cuh:221-394): energy under the curl cap v_cap and the
 // per-atom gradient F.
-template <int APL, int TW>
-__device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPose<APL>& P, float v_cap, float slope, Forces<APL>& F) {
-    const SceneDev& S = *C.S;
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ float energy_forces(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& P, float v_cap, float slope, Forces<APL>& F) {
+    SceneArg& S = C.S();
     const int ln = tlane<TW>();
     const int n3 = TW * APL;
+    const int lx = C.lx(), lf = lx + 4 * TW * APL;
     float* fx = F.fx;
     float* fy = F.fy;
     float* fz = F.fz;
@@ -1009,7 +1066,7 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
 #pragma unroll
     for (int k = 0; k < APL; k++) {
         const int a = ln + TW * k;
-        reinterpret_cast<float4*>(s_lds + C.lx)[a] = make_float4(P.x[k], P.y[k], P.z[k], C.rad[k]);
+        reinterpret_cast<float4*>(s_lds + lx)[a] = make_float4(P.x[k], P.y[k], P.z[k], C.rad[k]);
     }
     // inter-molecular term with the per-atom curl, and the box penalty
 #pragma unroll
@@ -1053,10 +1110,10 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
     }
     wave_lds_fence();
     // The diagonals' masks are uniform: scalar loads, used as the lane condition directly.
-    const unsigned long long* fm = C.L->fold_mask + C.fold_off;
-    const float4* lx4 = reinterpret_cast<const float4*>(s_lds + C.lx);
-    const int* lfl = reinterpret_cast<const int*>(s_lds + C.lfl);
-    const int n = C.natom;
+    const unsigned long long* fm = C.L().fold_mask + C.d().fold_off;
+    const float4* lx4 = reinterpret_cast<const float4*>(s_lds + lx);
+    const int* lfl = reinterpret_cast<const int*>(s_lds + C.lfl());
+    const int n = C.natom(), nfold = C.d().nfold;
     if constexpr (TW < kWave) {
         // A 32-lane tile (at most 32 atoms): the two diagonals dg and dg + 1 of a step are scored one
         // after the other by the same lanes, with the sums the whole-wave path forms over its two
@@ -1076,9 +1133,9 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
         const int tb = tbase<TW>();
         float ax = 0.0f, ay = 0.0f, az = 0.0f, e1 = 0.0f;
 #pragma unroll 1
-        for (int dg = 1; dg <= C.nfold; dg += 2) {
+        for (int dg = 1; dg <= nfold; dg += 2) {
             const unsigned long long m0 = uload(fm + dg - 1);
-            const unsigned long long m1 = dg < C.nfold ? uload(fm + dg) : 0ull;
+            const unsigned long long m1 = dg < nfold ? uload(fm + dg) : 0ull;
             float px0 = 0.0f, py0 = 0.0f, pz0 = 0.0f, px1 = 0.0f, py1 = 0.0f, pz1 = 0.0f;
             if (__builtin_amdgcn_inverse_ballot_w64(tmask<TW>(m0)))
                 e += pair_grad(xa.x, xa.y, xa.z, xa.w, C.lut[0], lx4[q0], lfl[q0], v_cap, px0, py0, pz0);
@@ -1096,7 +1153,7 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
             s1 = s1 - 2 < 0 ? s1 - 2 + n : s1 - 2;
         }
         fx[0] += ax; fy[0] += ay; fz[0] += az;
-        if (C.L->bias_type != 0 && C.L->bias_start) e += bias_forces(C, P, F);
+        if (C.biased()) e += bias_forces(C, P, F);
         const float r0 = row_sum(e), r1 = row_sum(e1);
         const float lo = ((rdl(r0, 0) + rdl(r0, 16)) + rdl(r1, 0)) + rdl(r1, 16);
         const float hi = ((rdl(r0, 32) + rdl(r0, 48)) + rdl(r1, 32)) + rdl(r1, 48);
@@ -1111,8 +1168,9 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
         // constants, so that nothing is decoded or selected per pair, and twelve (nine) ds_bpermute per
         // step, at 6 cycles of the LDS pipe each, are three writes and paired reads.
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
-        const char* tile = reinterpret_cast<const char*>(s_lds + C.lx);
-        const char* pk = reinterpret_cast<const char*>(C.L->pack + (size_t)C.pack_off * kWave);
+        const char* tile = reinterpret_cast<const char*>(s_lds + lx);
+        const char* pk = reinterpret_cast<const char*>(C.L().pack + (size_t)C.d().pack_off * kWave);
+        const int npack = C.d().npack;
         uint32_t at = uint32_t(sizeof(uint4)) * uint32_t(ln);
         uint4 t = *reinterpret_cast<const uint4*>(pk + at);
         if (n <= kWave / 2) {
@@ -1122,7 +1180,7 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
             const float4 xa = lx4[ln & 31];
             const uint32_t own = 4u * uint32_t((ln & 31) + 32);
 #pragma unroll 1
-            for (int st = 0; st < C.npack; st++) {
+            for (int st = 0; st < npack; st++) {
                 at += uint32_t(sizeof(uint4)) * kWave;
                 const uint4 tn = *reinterpret_cast<const uint4*>(pk + at);
                 float px = 0.0f, py = 0.0f, pz = 0.0f;
@@ -1132,9 +1190,9 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
                 if (__uint_as_float(t.z) < kRampNoPair && rr < kR2Cut)
                     e += pair_core(rx, ry, rz, rr, rs, __uint_as_float(t.z), __uint_as_float(t.w), v_cap, px,
                                    py, pz);
-                share_put(C.lf, ln, px, py, pz);
-                const float3 o = share_get(C.lf, own), b0 = share_get(C.lf, t.y & 0xffu),
-                             b1 = share_get(C.lf, (t.y >> 8) & 0xffu);
+                share_put(lf, ln, px, py, pz);
+                const float3 o = share_get(lf, own), b0 = share_get(lf, t.y & 0xffu),
+                             b1 = share_get(lf, (t.y >> 8) & 0xffu);
                 ax += (px + o.x) - (b0.x + b1.x);
                 ay += (py + o.y) - (b0.y + b1.y);
                 az += (pz + o.z) - (b0.z + b1.z);
@@ -1145,7 +1203,7 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
             // collects +p from the (at most two) lanes where it is i and -p from those where it is j; lane
             // 63 scores nothing and stands for no lane
 #pragma unroll 1
-            for (int st = 0; st < C.npack; st++) {
+            for (int st = 0; st < npack; st++) {
                 at += uint32_t(sizeof(uint4)) * kWave;
                 const uint4 tn = *reinterpret_cast<const uint4*>(pk + at);
                 float px = 0.0f, py = 0.0f, pz = 0.0f;
@@ -1157,9 +1215,9 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
                 if (__uint_as_float(t.z) < kRampNoPair && rr < kR2Cut)
                     e += pair_core(rx, ry, rz, rr, rs, __uint_as_float(t.z), __uint_as_float(t.w), v_cap, px,
                                    py, pz);
-                share_put(C.lf, ln, px, py, pz);
-                const float3 a0 = share_get(C.lf, t.y & 0xffu), a1 = share_get(C.lf, (t.y >> 8) & 0xffu);
-                const float3 b0 = share_get(C.lf, (t.y >> 16) & 0xffu), b1 = share_get(C.lf, t.y >> 24);
+                share_put(lf, ln, px, py, pz);
+                const float3 a0 = share_get(lf, t.y & 0xffu), a1 = share_get(lf, (t.y >> 8) & 0xffu);
+                const float3 b0 = share_get(lf, (t.y >> 16) & 0xffu), b1 = share_get(lf, t.y >> 24);
                 ax += (a0.x + a1.x) - (b0.x + b1.x);
                 ay += (a0.y + a1.y) - (b0.y + b1.y);
                 az += (a0.z + a1.z) - (b0.z + b1.z);
@@ -1167,7 +1225,7 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
             }
         }
         fx[0] += ax; fy[0] += ay; fz[0] += az;
-        if (C.L->bias_type != 0 && C.L->bias_start) e += bias_forces(C, P, F);
+        if (C.biased()) e += bias_forces(C, P, F);
         return uni(wave_sum(e));
     }
     // intra-molecular pairs with the per-pair curl, each pair once, as folded diagonals over the
@@ -1180,7 +1238,7 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
 #pragma unroll
         for (int k = 0; k < APL; k++) ax[k] = ay[k] = az[k] = 0.0f;
 #pragma unroll 1
-        for (int dg = 1; dg <= C.nfold; dg++) {
+        for (int dg = 1; dg <= nfold; dg++) {
 #pragma unroll
             for (int k = 0; k < APL; k++) {
                 const unsigned long long m = uload(fm + (dg - 1) * APL + k);
@@ -1191,9 +1249,9 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
                     e += pair_grad(P.x[k], P.y[k], P.z[k], C.rad[k], C.lut[k], lx4[q], lfl[q], v_cap, px, py, pz);
                 }
                 ax[k] += px; ay[k] += py; az[k] += pz;
-                s_lds[C.lf + a] = px;
-                s_lds[C.lf + n3 + a] = py;
-                s_lds[C.lf + 2 * n3 + a] = pz;
+                s_lds[lf + a] = px;
+                s_lds[lf + n3 + a] = py;
+                s_lds[lf + 2 * n3 + a] = pz;
             }
             wave_lds_fence();
 #pragma unroll
@@ -1201,9 +1259,9 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
                 const int c = ln + TW * k;
                 if (c < n) {
                     const int src = c - dg >= 0 ? c - dg : c - dg + n;
-                    ax[k] -= s_lds[C.lf + src];
-                    ay[k] -= s_lds[C.lf + n3 + src];
-                    az[k] -= s_lds[C.lf + 2 * n3 + src];
+                    ax[k] -= s_lds[lf + src];
+                    ay[k] -= s_lds[lf + n3 + src];
+                    az[k] -= s_lds[lf + 2 * n3 + src];
                 }
             }
             wave_lds_fence();
@@ -1213,14 +1271,14 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW>& C, const WPos
             fx[k] += ax[k]; fy[k] += ay[k]; fz[k] += az[k];
         }
     }
-    if (C.L->bias_type != 0 && C.L->bias_start) e += bias_forces(C, P, F);
+    if (C.biased()) e += bias_forces(C, P, F);
     return uni(wave_sum(e));
 }
 
 // cal_grad_tile (bfgs.cuh:69-193): the pose gradient from the per-atom gradient,
 // returned lane-distributed (lane k = component k).
-template <int APL, int TW>
-__device__ __forceinline__ float pose_grad(const Ctx<APL, TW>& C, const WPose<APL>& P, const Forces<APL>& F) {
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ float pose_grad(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& P, const Forces<APL>& F) {
     const int ln = tlane<TW>();
     const float* fx = F.fx;
     const float* fy = F.fy;
@@ -1250,10 +1308,11 @@ __device__ __forceinline__ float pose_grad(const Ctx<APL, TW>& C, const WPose<AP
     }
     // the axis atoms from the LDS coordinate tile, which still holds this pose (the energy of P was
     // the last evaluation): broadcast loads instead of lane reads
-    const float4* lx4 = reinterpret_cast<const float4*>(s_lds + C.lx);
+    const float4* lx4 = reinterpret_cast<const float4*>(s_lds + C.lx());
+    const int nt = C.ntors(), lt = C.lt();
 #pragma unroll 1
-    for (int t = 0; t < C.ntors; t++) {
-        const TorsEnt te = tors_ent(C, t);
+    for (int t = 0; t < nt; t++) {
+        const TorsEnt te = tors_ent_at<APL>(lt, t);
         const float4 xt = lx4[te.to], xf = lx4[te.from];
         float ux = xt.x - xf.x, uy = xt.y - xf.y, uz = xt.z - xf.z;
         const float inv = frsq(sq_dist(ux, uy, uz));
@@ -1261,7 +1320,7 @@ __device__ __forceinline__ float pose_grad(const Ctx<APL, TW>& C, const WPose<AP
         float st = 0.0f;
 #pragma unroll
         for (int k = 0; k < APL; k++) {
-            if (((tors_mask(C, t, k) >> ln) & 1ull) && heavy(C, k)) {
+            if (((tors_mask_at<APL>(lt, t, k) >> ln) & 1ull) && heavy(C, k)) {
                 const float lx = P.x[k] - xt.x, ly = P.y[k] - xt.y, lz = P.z[k] - xt.z;
                 const float cx = msub2(ly, fz[k], lz, fy[k]), cy = msub2(lz, fx[k], lx, fz[k]),
                             cz = msub2(lx, fy[k], ly, fx[k]);
@@ -1273,13 +1332,13 @@ __device__ __forceinline__ float pose_grad(const Ctx<APL, TW>& C, const WPose<AP
     }
     // constraint docking (bfgs.cuh:176): the rigid components are never written and
     // keep the zeros the reference's gradient buffers start with
-    if (C.L->constraint && ln < 6) gout = 0.0f;
+    if (C.L().constraint && ln < 6) gout = 0.0f;
     return gout;
 }
 
 // cal_e_grad_tile (bfgs.cuh:397-410).
-template <int APL, int TW>
-__device__ __forceinline__ float energy_grad(const Ctx<APL, TW>& C, const WPose<APL>& P, float v_cap, float slope,
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ float energy_grad(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& P, float v_cap, float slope,
                                              float& g) {
     Forces<APL> F;
     const float e = energy_forces(C, P, v_cap, slope, F);
@@ -1292,9 +1351,9 @@ __device__ __forceinline__ float energy_grad(const Ctx<APL, TW>& C, const WPose<
 // the receptor (every receptor heavy atom at its most attractive distance: the gauss, hydrophobic and
 // hydrogen-bond terms together stay below 0.67 kcal/mol per pair, and a grid value interpolates such
 // sums) and any intra pair can add (the curl only shrinks repulsion).
-template <int APL, int TW>
-__device__ __forceinline__ float energy_lower_bound(const Ctx<APL, TW>& C, const WPose<APL>& P, float slope) {
-    const SceneDev& S = *C.S;
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ float energy_lower_bound(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& P, float slope) {
+    SceneArg& S = C.S();
     float pen = 0.0f;
 #pragma unroll
     for (int k = 0; k < APL; k++) {
@@ -1303,7 +1362,7 @@ __device__ __forceinline__ float energy_lower_bound(const Ctx<APL, TW>& C, const
         pen += fmaxf(S.box_lo[1] - P.y[k], 0.0f) + fmaxf(P.y[k] - S.box_hi[1], 0.0f);
         pen += fmaxf(S.box_lo[2] - P.z[k], 0.0f) + fmaxf(P.z[k] - S.box_hi[2], 0.0f);
     }
-    return tuni<TW>(tsum<TW>(pen) * slope - 0.67f * (float(S.nrec) * float(C.nheavy) + float(C.npair)));
+    return tuni<TW>(tsum<TW>(pen) * slope - 0.67f * (float(S.nrec) * float(C.nheavy()) + float(C.npair())));
 }
 
 // line_search_tile (bfgs.cuh:623-670). A trial whose energy is certain to fail the sufficient-decrease
@@ -1319,8 +1378,8 @@ __device__ __forceinline__ float energy_lower_bound(const Ctx<APL, TW>& C, const
 // where FP32 rounds bonded atoms onto one point: a torsion axis of zero length turns its gradient and
 // its rotated atoms into NaN. The reference searches on, and can keep a pose of NaN coordinates, which
 // every energy term skips (their comparisons fail), so it scores finite; hydrogens are never scored.
-template <int APL, int TW>
-__device__ __forceinline__ bool pose_finite(const Ctx<APL, TW>& C, const WPose<APL>& P) {
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ bool pose_finite(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& P) {
     bool bad = false;
 #pragma unroll
     for (int k = 0; k < APL; k++)
@@ -1329,8 +1388,8 @@ __device__ __forceinline__ bool pose_finite(const Ctx<APL, TW>& C, const WPose<A
     return tballot<TW>(bad) == 0ull;
 }
 
-template <int APL, int TW>
-__device__ __forceinline__ bool line_search(const Ctx<APL, TW>& C, const WPose<APL>& x, float g, float p, float e0, float v_cap,
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ bool line_search(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& x, float g, float p, float e0, float v_cap,
                             float slope, WPose<APL>& x_new, float& g_new, float& e_out, float& alpha_out) {
     const float pg = tuni<TW>(tsum<TW>(p * g));
     const auto fail = [&]() {
@@ -1341,7 +1400,7 @@ __device__ __forceinline__ bool line_search(const Ctx<APL, TW>& C, const WPose<A
         return false;
     };
     if (!__builtin_isfinite(pg)) return fail();
-    const bool screen = pg < -1e4f && !(C.L->bias_type != 0 && C.L->bias_start);
+    const bool screen = pg < -1e4f && !(C.biased());
     float alpha = 1.0f, e_new = 0.0f;
     Forces<APL> F;
     for (int trial = 0; trial < 10; trial++) {
@@ -1377,8 +1436,8 @@ __device__ __forceinline__ void stage_vec(int o, float v) { s_lds[o + tlane<TW>(
 // components: four columns per pass with independent partial sums, the vector's four components by
 // one broadcast load, so the reads are in flight together. Every lane reads a real row (callers mask
 // lanes past dim).
-template <int APL, int TW>
-__device__ __forceinline__ float hess_row_dot(const Ctx<APL, TW>& C, int hrow, int dim, int vo) {
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ float hess_row_dot(const Ctx<APL, TW, LAZY>& C, int hrow, int dim, int vo) {
     float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
     int j = 0;
     for (; j + 4 <= dim; j += 4) {
@@ -1397,30 +1456,31 @@ __device__ __forceinline__ float hess_row_dot(const Ctx<APL, TW>& C, int hrow, i
 // tile (lane i owns row i) and the start pose is parked in LDS for the
 // restore at the end (the energy went up, or a line search failed). The vectors the Hessian products read (g, y, p, -Hy) are staged in
 // the coordinate tile, idle between a line search and the next one.
-template <int APL, int TW>
-__device__ __forceinline__ void bfgs(const Ctx<APL, TW>& C, WPose<APL>& x, int max_steps, float v_cap, float slope) {
-    const int ln = tlane<TW>(), dim = C.dim;
-    const int hrow = C.lh + ln * C.ld;
-    const int hrow_rd = C.lh + (row_lane_clamped(ln, dim)) * C.ld;  // lanes past dim read the last row
-    const bool row = ln < dim;
-    const int v0 = C.lx, vp = C.lx + TW, vm = C.lx + 2 * TW;
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void bfgs(const Ctx<APL, TW, LAZY>& C, WPose<APL>& x, int max_steps, float v_cap, float slope) {
     float g;
     const float E_ori = energy_grad(C, x, v_cap, slope, g);
     float E = E_ori, E1 = 0.0f, alpha = 0.0f;
-    if (row)
-        for (int j = 0; j < dim; j++) s_lds[hrow + j] = (j == ln) ? 1.0f : 0.0f;
+    {
+        const int ln = tlane<TW>(), dim = C.dim(), hrow = C.lh() + ln * C.ld;
+        if (ln < dim)
+            for (int j = 0; j < dim; j++) s_lds[hrow + j] = (j == ln) ? 1.0f : 0.0f;
+    }
     float g_new = g;
     WPose<APL> x_new = x;
     save_pose(C, x);
     float p = g;
     bool failed = false;
     for (int step = 0; step < max_steps; step++) {
-        // rows beyond dim are masked
-        stage_vec<TW>(v0, g);
-        wave_lds_fence();
-        const float s = hess_row_dot(C, hrow_rd, dim, v0);
-        p = row ? -s : 0.0f;
-        wave_lds_fence();
+        // rows beyond dim are masked: their lanes read the last row
+        {
+            const int ln = tlane<TW>(), dim = C.dim(), v0 = C.lx();
+            stage_vec<TW>(v0, g);
+            wave_lds_fence();
+            const float s = hess_row_dot(C, C.lh() + row_lane_clamped(ln, dim) * C.ld, dim, v0);
+            p = ln < dim ? -s : 0.0f;
+            wave_lds_fence();
+        }
         if (!line_search(C, x, g, p, E, v_cap, slope, x_new, g_new, E1, alpha)) {
             failed = true;
             break;
@@ -1431,6 +1491,9 @@ __device__ __forceinline__ void bfgs(const Ctx<APL, TW>& C, WPose<APL>& x, int m
         const float gg = tsum<TW>(g * g);
         if (sqrtf(gg) < 1e-5f) break;
         g = g_new;
+        const int ln = tlane<TW>(), dim = C.dim(), hrow = C.lh() + ln * C.ld;
+        const int v0 = C.lx(), vp = v0 + TW, vm = v0 + 2 * TW;
+        const bool row = ln < dim;
         if (step == 0) {
             const float yy = tuni<TW>(tsum<TW>(y * y));
             if (fabsf(yy) > kEps) {
@@ -1442,7 +1505,7 @@ __device__ __forceinline__ void bfgs(const Ctx<APL, TW>& C, WPose<APL>& x, int m
         if (alpha * yp < kEps) continue;
         stage_vec<TW>(v0, y);
         wave_lds_fence();
-        const float hy = hess_row_dot(C, hrow_rd, dim, v0);
+        const float hy = hess_row_dot(C, C.lh() + row_lane_clamped(ln, dim) * C.ld, dim, v0);
         const float mhy = row ? -hy : 0.0f;
         const float yhy = -tsum<TW>(y * mhy);
         const float r = 1.0f / (alpha * yp);
@@ -1514,8 +1577,8 @@ __device__ __forceinline__ float3 rand_in_ball(Rng& rng) {
 }
 
 // gyration_radius (common.cuh:106-122).
-template <int APL, int TW>
-__device__ __forceinline__ float gyration(const Ctx<APL, TW>& C, const WPose<APL>& P) {
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ float gyration(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& P) {
     float s = 0.0f;
 #pragma unroll
     for (int k = 0; k < APL; k++)
@@ -1524,7 +1587,7 @@ __device__ __forceinline__ float gyration(const Ctx<APL, TW>& C, const WPose<APL
             s += sq_dist(dx, dy, dz);
         }
     s = tsum<TW>(s);
-    const float r = C.nheavy > 0 ? sqrtf(s / float(C.nheavy)) : 0.0f;
+    const float r = C.nheavy() > 0 ? sqrtf(s / float(C.nheavy())) : 0.0f;
     return tuni<TW>(r > 0.0f ? r : 1.0f);
 }
 
@@ -1538,14 +1601,14 @@ struct Move {
 };
 
 // mutate_pose_tile (E/src/cuda/mc.cu:146-256).
-template <int APL, int TW>
-__device__ __forceinline__ Move mutate(const Ctx<APL, TW>& C, WPose<APL>& P, Rng& rng) {
-    const SceneDev& S = *C.S;
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ Move mutate(const Ctx<APL, TW, LAZY>& C, WPose<APL>& P, Rng& rng) {
+    SceneArg& S = C.S();
     const uint4 b = rng.next();
     // constraint docking draws a torsion only; a rigid ligand then stays put (mc.cu:159-166)
     int which;
-    if (C.L->constraint) which = C.ntors > 0 ? 2 + int(b.x % uint32_t(C.ntors)) : -1;
-    else which = int(b.x % uint32_t(2 + C.ntors));
+    if (C.L().constraint) which = C.ntors() > 0 ? 2 + int(b.x % uint32_t(C.ntors())) : -1;
+    else which = int(b.x % uint32_t(2 + C.ntors()));
     Move mv;
     if (which < 0) {
         mv.kind = 2;
@@ -1580,7 +1643,7 @@ __device__ __forceinline__ Move mutate(const Ctx<APL, TW>& C, WPose<APL>& P, Rng
         int i = int(ceilf(__fsub_rn(__fmul_rn(u01(bb.x), float(te.nrange)), 1.0f)));
         i = i < 0 ? 0 : (i > te.nrange - 1 ? te.nrange - 1 : i);
         float2 r = make_float2(te.lo, te.hi);
-        if (i > 0) r = C.L->ranges[C.L->tors_range[C.tors_off + t].x + i];
+        if (i > 0) r = C.L().ranges[C.L().tors_range[C.d().tors_off + t].x + i];
         const float target = r.x + (r.y - r.x) * u01(bb.y);
         const float inc = target - tread<TW>(P.dihe, t);
         apply_torsion(C, P, t, inc);
@@ -1590,7 +1653,7 @@ __device__ __forceinline__ Move mutate(const Ctx<APL, TW>& C, WPose<APL>& P, Rng
         for (int k = 0; k < APL; k++) nmoved += __popcll(tors_mask(C, t, k) & tballot<TW>(heavy(C, k)));
         mv.kind = 2;
         mv.mag = fabsf(normalize_angle(inc)) * (1.0f / kPi);
-        mv.moved = C.nheavy > 0 ? float(nmoved) / float(C.nheavy) : 0.0f;
+        mv.moved = C.nheavy() > 0 ? float(nmoved) / float(C.nheavy()) : 0.0f;
     }
     return mv;
 }
@@ -1600,9 +1663,9 @@ __device__ __forceinline__ Move mutate(const Ctx<APL, TW>& C, WPose<APL>& P, Rng
 // applied through apply_update with alpha = 1. Constraint docking keeps centre
 // and orientation (:27-35), the align bias keeps the centre (:36-39); the centre
 // block is drawn either way.
-template <int APL, int TW>
-__device__ __forceinline__ void randomize(const Ctx<APL, TW>& C, WPose<APL>& P, Rng& rng, int idx, int n) {
-    const SceneDev& S = *C.S;
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void randomize(const Ctx<APL, TW, LAZY>& C, WPose<APL>& P, Rng& rng, int idx, int n) {
+    SceneArg& S = C.S();
     const int ln = tlane<TW>();
     const uint4 b = rng.next();
     const float gc0 = (S.box_lo[0] + (S.box_hi[0] - S.box_lo[0]) * u01(b.x)) - P.c0;
@@ -1619,19 +1682,19 @@ __device__ __forceinline__ void randomize(const Ctx<APL, TW>& C, WPose<APL>& P, 
     const float3 rv = quat_to_rotvec(make_float4(r * sa, r * ca, R * sb, R * cb));
     // torsion t draws block (draw + t) on lane t: a range, then a value in it
     float tv = 0.0f;
-    if (ln < C.ntors) {
+    if (ln < C.ntors()) {
         const uint4 bt = rng.at(rng.draw + ln);
-        const int2 rr = C.L->tors_range[C.tors_off + ln];
+        const int2 rr = C.L().tors_range[C.d().tors_off + ln];
         int j = int(__fmul_rn(u01(bt.x), float(rr.y)));
         j = j > rr.y - 1 ? rr.y - 1 : j;
-        const float2 rg = C.L->ranges[rr.x + j];
+        const float2 rg = C.L().ranges[rr.x + j];
         tv = (rg.x + (rg.y - rg.x) * u01(bt.y)) - P.dihe;
     }
-    rng.draw += C.ntors;
+    rng.draw += C.ntors();
     // direction vector: lanes 0..5 rigid part, lane 6 + t torsion t
     const float sh = tshfl<TW>(tv, ln - 6);
-    float d = (ln >= 6 && ln < 6 + C.ntors) ? sh : 0.0f;
-    const bool keep_c = C.L->constraint || C.L->bias_type == 2, keep_o = C.L->constraint;
+    float d = (ln >= 6 && ln < 6 + C.ntors()) ? sh : 0.0f;
+    const bool keep_c = C.L().constraint || C.L().bias_type == 2, keep_o = C.L().constraint;
     d = ln == 0 ? (keep_c ? 0.0f : gc0) : d;
     d = ln == 1 ? (keep_c ? 0.0f : gc1) : d;
     d = ln == 2 ? (keep_c ? 0.0f : gc2) : d;
@@ -1643,47 +1706,50 @@ __device__ __forceinline__ void randomize(const Ctx<APL, TW>& C, WPose<APL>& P, 
 
 // ---------------------------------------------------------- pose buffers
 template <int APL>
-__device__ __forceinline__ void load_pose(const LigSetDev& L, const PoseBufs& B, int lig, int chain, WPose<APL>& P) {
-    const DevLig d = L.ligs[lig];
-    const size_t xo = ((size_t)d.atom_off * B.nchain + (size_t)chain * d.natom) * 3;
-    const size_t po = (size_t)lig * B.nchain + chain;
+__device__ __forceinline__ void load_pose(const Ctx<APL>& C, Karg<PoseBufs>& B, int lig, int chain, WPose<APL>& P) {
+    KLig& d = C.d();
+    const int natom = d.natom, ntors = d.ntors, nchain = B.nchain;
+    const size_t xo = ((size_t)d.atom_off * nchain + (size_t)chain * natom) * 3;
+    const size_t po = (size_t)lig * nchain + chain;
 #pragma unroll
     for (int k = 0; k < APL; k++) {
         const int a = lane() + kWave * k;
-        if (a < d.natom) { P.x[k] = B.x[xo + 3 * a]; P.y[k] = B.x[xo + 3 * a + 1]; P.z[k] = B.x[xo + 3 * a + 2]; }
+        if (a < natom) { P.x[k] = B.x[xo + 3 * a]; P.y[k] = B.x[xo + 3 * a + 1]; P.z[k] = B.x[xo + 3 * a + 2]; }
         else { P.x[k] = P.y[k] = P.z[k] = 0.0f; }
     }
     P.c0 = B.c[po * 3]; P.c1 = B.c[po * 3 + 1]; P.c2 = B.c[po * 3 + 2];
     P.r0 = B.rv[po * 3]; P.r1 = B.rv[po * 3 + 1]; P.r2 = B.rv[po * 3 + 2];
-    const size_t dof = (size_t)d.tors_off * B.nchain + (size_t)chain * d.ntors;
-    P.dihe = lane() < d.ntors ? B.dihe[dof + lane()] : 0.0f;
+    const size_t dof = (size_t)d.tors_off * nchain + (size_t)chain * ntors;
+    P.dihe = lane() < ntors ? B.dihe[dof + lane()] : 0.0f;
     P.e = B.e[po];
 }
 
-template <int APL, int TW = kWave>
-__device__ __forceinline__ void store_pose(const LigSetDev& L, const PoseBufs& B, int lig, int chain,
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void store_pose(const Ctx<APL, TW, LAZY>& C, Karg<PoseBufs>& B, int lig, int chain,
                                            const WPose<APL>& P) {
-    const DevLig d = L.ligs[lig];
-    const size_t xo = ((size_t)d.atom_off * B.nchain + (size_t)chain * d.natom) * 3;
-    const size_t po = (size_t)lig * B.nchain + chain;
+    KLig& d = C.d();
+    const int natom = d.natom, ntors = d.ntors, nchain = B.nchain;
+    const size_t xo = ((size_t)d.atom_off * nchain + (size_t)chain * natom) * 3;
+    const size_t po = (size_t)lig * nchain + chain;
     const int ln = tlane<TW>();
 #pragma unroll
     for (int k = 0; k < APL; k++) {
         const int a = ln + TW * k;
-        if (a < d.natom) { B.x[xo + 3 * a] = P.x[k]; B.x[xo + 3 * a + 1] = P.y[k]; B.x[xo + 3 * a + 2] = P.z[k]; }
+        if (a < natom) { B.x[xo + 3 * a] = P.x[k]; B.x[xo + 3 * a + 1] = P.y[k]; B.x[xo + 3 * a + 2] = P.z[k]; }
     }
     if (ln == 0) { B.c[po * 3] = P.c0; B.rv[po * 3] = P.r0; B.e[po] = P.e; }
     if (ln == 1) { B.c[po * 3 + 1] = P.c1; B.rv[po * 3 + 1] = P.r1; }
     if (ln == 2) { B.c[po * 3 + 2] = P.c2; B.rv[po * 3 + 2] = P.r2; }
-    const size_t dof = (size_t)d.tors_off * B.nchain + (size_t)chain * d.ntors;
-    if (ln < d.ntors) B.dihe[dof + ln] = P.dihe;
+    const size_t dof = (size_t)d.tors_off * nchain + (size_t)chain * ntors;
+    if (ln < ntors) B.dihe[dof + ln] = P.dihe;
 }
 
 // Input conformation of a ligand: coordinates, dihedrals, centroid, rot_vec = 0,
 // energy 999 (E/src/cuda/task.cu:94-108).
-template <int APL, int TW>
-__device__ __forceinline__ void initial_pose(const Ctx<APL, TW>& C, const LigSetDev& L, int lig, WPose<APL>& P) {
-    const DevLig d = L.ligs[lig];
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ void initial_pose(const Ctx<APL, TW, LAZY>& C, WPose<APL>& P) {
+    KLig& d = C.d();
+    LigArg& L = C.L();
     const int ln = tlane<TW>();
 #pragma unroll
     for (int k = 0; k < APL; k++) {

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace ud2 {
@@ -118,6 +119,12 @@ struct PoseBufs {
 };
 
 enum InterMode : int32_t { kDirect = 0, kGrid = 1 };
+
+// What the arguments of every kernel that works on poses begin with.
+struct ArgHead {
+    LigSetDev L;
+    SceneDev S;
+};
 
 struct McArgs {
     LigSetDev L;
@@ -306,6 +313,12 @@ struct FeatArgs {
     int32_t lds_floats_per_wave;
     int32_t hdim_ld;         // sizes the torsion table (>= 6 + ntors of every selected ligand)
 };
+
+template <class T>
+constexpr bool begins_with_head() { return offsetof(T, L) == offsetof(ArgHead, L) && offsetof(T, S) == offsetof(ArgHead, S); }
+static_assert(begins_with_head<McArgs>() && begins_with_head<OptArgs>() && begins_with_head<PoseVecArgs>() &&
+                  begins_with_head<LmcArgs>() && begins_with_head<FeatArgs>(),
+              "kernels read the ligand set and the scene through ArgHead");
 
 // Launchers (ud2_kernels.hip); each returns a hipError_t.
 hipError_t launch_grid_build(const GridArgs& a, hipStream_t s);

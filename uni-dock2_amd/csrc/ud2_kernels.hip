@@ -15,10 +15,9 @@ namespace ud2 {
 // chain and stores nothing. The best pose goes to the pose buffers whenever it improves (the
 // reference copies it to out_pose at the same points, mc.cu:389-392).
 // OCC is the occupancy hint (waves per SIMD the register allocation must allow). One-atom-per-lane
-// ligands fit six waves per SIMD in LDS; the whole-wave kernel runs at six (80 VGPRs, about 60
-// spilled), which measured 6 % faster than four waves with 128 VGPRs and few spills, bit for bit:
-// the search is bound by latency (dependent LDS round trips and transcendental chains) more than by
-// VALU issue. The half-wave kernel needs about 180 VGPRs without spills, so it comes at 4
+// ligands fit six waves per SIMD in LDS; the whole-wave kernel runs at six (80 VGPRs, 31 spilled): five
+// waves with 96 VGPRs and none spilled measure the same on 256 ligands, and the learned kernel 3 % slower.
+// The search is bound by VALU issue, the LDS pipe and latency together. The half-wave kernel needs about 180 VGPRs without spills, so it comes at 4
 // (spilling), 3 and 2 waves. The two-slot kernel runs at three waves per SIMD (168 VGPRs, a few spilled;
 // its LDS allows three blocks per CU), the three- and four-slot kernels at two: on ligands of 65-80
 // atoms three waves measured 25 % faster than the two that an unconstrained allocation (239 VGPRs)
@@ -26,15 +25,17 @@ namespace ud2 {
 // MODE is the inter term: the grid builds hold nothing of the direct sum and the other way round.
 template <int APL, int TW, int OCC, int MODE>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) __attribute__((amdgpu_waves_per_eu(OCC)))
-void mc_kernel(McArgs A) {
+void mc_kernel(McArgs) {
+    Karg<McArgs>* const K = kernel_args<McArgs>();
     constexpr int CPW = kWave / TW;  // chains per wave
     const int w = threadIdx.x / kWave;
     const int h = CPW == 1 ? 0 : __lane_id() / TW;
-    const int base = w * A.lds_floats_per_wave + h * (A.lds_floats_per_wave / CPW);
-    const int nchain = A.P.nchain;
-    const int ngroup = (nchain + CPW - 1) / CPW;
-    const int n_items = A.n_order * ngroup;
     for (;;) {
+        Karg<McArgs>& A = *reread(K);
+        const int base = w * A.lds_floats_per_wave + h * (A.lds_floats_per_wave / CPW);
+        const int nchain = A.P.nchain;
+        const int ngroup = (nchain + CPW - 1) / CPW;
+        const int n_items = A.n_order * ngroup;
         int item = 0;
         if (lane() == 0) item = atomicAdd(A.counter, 1);
         item = __builtin_amdgcn_readfirstlane(item);
@@ -43,52 +44,54 @@ void mc_kernel(McArgs A) {
         const int c = CPW * (item % ngroup) + h;
         const bool real = CPW == 1 || c < nchain;
         const int chain = real ? c : nchain - 1;
-        Ctx<APL, TW> C;
-        load_ctx(C, A.L, A.S, lig, MODE, base, A.hdim_ld);
+        Ctx<APL, TW, (OCC > 2)> C;
+        load_ctx(C, (KHead*)K, lig, MODE, base, A.hdim_ld);
         Rng rng{A.seed, uint32_t(lig + A.lig_index_base), uint32_t(chain), 0u};
         WPose<APL> acc;
-        initial_pose(C, A.L, lig, acc);
+        initial_pose(C, acc);
         if (A.randomize) randomize(C, acc, rng, chain, nchain);
         if (A.mc_steps == 0) {
             Forces<APL> F;
             acc.e = energy_forces(C, acc, kVCap, kSlope, F);
-            if (real) store_pose<APL, TW>(A.L, A.P, lig, chain, acc);
+            if (real) store_pose(C, reread(K)->P, lig, chain, acc);
             continue;
         }
-        if (real) store_pose<APL, TW>(A.L, A.P, lig, chain, acc);
+        if (real) store_pose(C, reread(K)->P, lig, chain, acc);
         save_pose(C, acc, 1);  // the accepted pose lives in LDS between steps
         float best = 1e9f;
         C.evals = 0;
-        for (int step = 0; step < A.mc_steps; step++) {
+        for (int step = 0; step < reread(K)->mc_steps; step++) {
             WPose<APL> cand;
             restore_pose(C, cand, 1);
             const float acc_e = cand.e;
             mutate(C, cand, rng);
-            if (A.opt_steps == 0) {
+            const int opt_steps = reread(K)->opt_steps;
+            if (opt_steps == 0) {
                 float gd;
                 cand.e = energy_grad(C, cand, kVCap, kSlope, gd);
             } else {
-                bfgs(C, cand, A.opt_steps, kVCap, kSlope);
+                bfgs(C, cand, opt_steps, kVCap, kSlope);
             }
             const uint4 b = rng.next();
             const bool accepted = (cand.e < acc_e) || (u01(b.x) < __expf((acc_e - cand.e) / 1.2f));
             if (step == 0 || accepted) {
                 if (cand.e < best) {
-                    if (A.opt_steps > 0) bfgs(C, cand, A.opt_steps, kVCapAuth, kSlope);
+                    if (opt_steps > 0) bfgs(C, cand, opt_steps, kVCapAuth, kSlope);
                     if (cand.e < best) {
-                        if (real) store_pose<APL, TW>(A.L, A.P, lig, chain, cand);
+                        if (real) store_pose(C, reread(K)->P, lig, chain, cand);
                         best = cand.e;
                     }
                 }
                 save_pose(C, cand, 1);
             }
         }
-        if (A.stats && tlane<TW>() == 0 && real) {
+        unsigned long long* stats = reread(K)->stats;
+        if (stats && tlane<TW>() == 0 && real) {
             const unsigned long long ev = (unsigned long long)C.evals;
-            atomicAdd(&A.stats[0], ev);
-            atomicAdd(&A.stats[1], ev * 32ull * (unsigned long long)C.nheavy);
-            atomicAdd(&A.stats[2], ev * (unsigned long long)C.npair);
-            atomicAdd(&A.stats[3], 1ull);
+            atomicAdd(&stats[0], ev);
+            atomicAdd(&stats[1], ev * 32ull * (unsigned long long)C.nheavy());
+            atomicAdd(&stats[2], ev * (unsigned long long)C.npair());
+            atomicAdd(&stats[3], 1ull);
         }
     }
 }
@@ -98,7 +101,9 @@ void mc_kernel(McArgs A) {
 // (line_search_one_gpu, E/src/cuda/bfgs_wrapper.cu:12-48), or a reset to the
 // input conformation.
 template <int APL, int MODE>
-__global__ __launch_bounds__(kWave* kWavesPerBlock) void opt_kernel(OptArgs A) {
+__global__ __launch_bounds__(kWave* kWavesPerBlock) void opt_kernel(OptArgs) {
+    Karg<OptArgs>* const K = kernel_args<OptArgs>();
+    Karg<OptArgs>& A = *K;
     const int w = threadIdx.x / kWave;
     const int s = blockIdx.x * kWavesPerBlock + w;
     if (s >= A.n_sel) return;
@@ -106,39 +111,39 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void opt_kernel(OptArgs A) {
     const int lig = pid / A.P.nchain, chain = pid % A.P.nchain;
     const int o = A.pos ? A.pos[s] : s;
     Ctx<APL> C;
-    load_ctx(C, A.L, A.S, lig, MODE, w * A.lds_floats_per_wave, A.hdim_ld);
+    load_ctx(C, (KHead*)K, lig, MODE, w * A.lds_floats_per_wave, A.hdim_ld);
     WPose<APL> P;
     const int ln = lane();
     if (A.op == 4) {
-        initial_pose(C, A.L, lig, P);
-        store_pose(A.L, A.P, lig, chain, P);
+        initial_pose(C, P);
+        store_pose(C, A.P, lig, chain, P);
         return;
     }
-    load_pose(A.L, A.P, lig, chain, P);
+    load_pose(C, A.P, lig, chain, P);
     if (A.op == 0) {
         bfgs(C, P, A.max_steps, A.v_cap, A.slope);
-        store_pose(A.L, A.P, lig, chain, P);
+        store_pose(C, A.P, lig, chain, P);
         if (A.out_e && ln == 0) A.out_e[o] = P.e;
     } else if (A.op == 1) {
         float g;
         const float e = energy_grad(C, P, A.v_cap, A.slope, g);
         if (A.out_e && ln == 0) A.out_e[o] = e;
-        if (A.out_g && ln < C.dim) A.out_g[(size_t)o * kWave + ln] = g;
+        if (A.out_g && ln < C.dim()) A.out_g[(size_t)o * kWave + ln] = g;
     } else if (A.op == 2) {
-        const float d = ln < C.dim ? A.dir[(size_t)o * kWave + ln] : 0.0f;
+        const float d = ln < C.dim() ? A.dir[(size_t)o * kWave + ln] : 0.0f;
         apply_update(C, P, d, A.alpha);
-        store_pose(A.L, A.P, lig, chain, P);
+        store_pose(C, A.P, lig, chain, P);
     } else {
         float g;
         const float e0 = energy_grad(C, P, A.v_cap, A.slope, g);
-        const float p = ln < C.dim ? -g : 0.0f;
+        const float p = ln < C.dim() ? -g : 0.0f;
         WPose<APL> xn;
         float gn, e1, al;
         line_search(C, P, g, p, e0, A.v_cap, A.slope, xn, gn, e1, al);
         xn.e = e1;
-        store_pose(A.L, A.P, lig, chain, xn);
+        store_pose(C, A.P, lig, chain, xn);
         if (A.out_e && ln == 0) A.out_e[o] = al;
-        if (A.out_g && ln < C.dim) A.out_g[(size_t)o * kWave + ln] = gn;
+        if (A.out_g && ln < C.dim()) A.out_g[(size_t)o * kWave + ln] = gn;
     }
 }
 
@@ -147,21 +152,23 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void opt_kernel(OptArgs A) {
 // the conformer rotated by q about its centroid and moved to the centre;
 // rot_vec = rotvec(q).
 template <int APL, int MODE>
-__global__ __launch_bounds__(kWave* kWavesPerBlock) void posevec_kernel(PoseVecArgs A) {
+__global__ __launch_bounds__(kWave* kWavesPerBlock) void posevec_kernel(PoseVecArgs) {
+    Karg<PoseVecArgs>* const K = kernel_args<PoseVecArgs>();
+    Karg<PoseVecArgs>& A = *K;
     const int w = threadIdx.x / kWave;
     Ctx<APL> C;
-    load_ctx(C, A.L, A.S, A.lig, MODE, w * A.lds_floats_per_wave, A.hdim_ld);
+    load_ctx(C, (KHead*)K, A.lig, MODE, w * A.lds_floats_per_wave, A.hdim_ld);
     WPose<APL> P0;
-    initial_pose(C, A.L, A.lig, P0);
+    initial_pose(C, P0);
     const int ln = lane();
-    const int dimv = 7 + C.ntors, dimg = 6 + C.ntors;
+    const int nt = C.ntors(), dimv = 7 + nt, dimg = 6 + nt;
     const int64_t stride = (int64_t)gridDim.x * kWavesPerBlock;
     for (int64_t i = (int64_t)blockIdx.x * kWavesPerBlock + w; i < A.n; i += stride) {
         const float* pv = A.pv + i * dimv;
         const float mine = ln < dimv ? pv[ln] : 0.0f;
         WPose<APL> P = P0;
-        for (int t = 0; t < C.ntors; t++) apply_torsion(C, P, t, rdl(mine, 7 + t) - rdl(P.dihe, t));
-        if (C.ntors > 0) centroid(C, P);
+        for (int t = 0; t < nt; t++) apply_torsion(C, P, t, rdl(mine, 7 + t) - rdl(P.dihe, t));
+        if (nt > 0) centroid(C, P);
         const float4 q = make_float4(rdl(mine, 3), rdl(mine, 4), rdl(mine, 5), rdl(mine, 6));
         const float n0 = rdl(mine, 0), n1 = rdl(mine, 1), n2 = rdl(mine, 2);
         rigid_move(C, P, q, P.c0, P.c1, P.c2, n0, n1, n2);
@@ -449,8 +456,8 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void final_score_kernel(Scor
     const int lig = pid / A.nchain, chain = pid % A.nchain;
     const DevLig d = A.L.ligs[lig];
     const float* xb = A.x + ((size_t)d.atom_off * A.nchain + (size_t)chain * d.natom) * 3;
-    const SceneDev& S = A.S;
-    const LigSetDev& L = A.L;
+    SceneArg& S = kernel_args<ScoreArgs>()->S;
+    LigArg& L = kernel_args<ScoreArgs>()->L;
     const int ln = lane();
     float e_inter = 0.0f, e_pen = 0.0f, e_intra = 0.0f, e_bias = 0.0f;
 #pragma unroll

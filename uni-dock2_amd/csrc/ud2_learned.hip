@@ -37,8 +37,8 @@ static __constant__ int c_fclass[kNumTypes] = {-1, 1, 0, 1, 2, 3, 4, 3, 5, 6, 5,
 template <int APL>
 __device__ __forceinline__ void pose_features(const Ctx<APL>& C, const WPose<APL>& P, const Move& mv, float e_acc, int sc,
                               uint16_t* xrow) {
-    const SceneDev& S = *C.S;
-    const int ln = lane();
+    SceneArg& S = C.S();
+    const int ln = tlane<kWave>(), natom = C.natom();
     float curl = 0.0f;
 #pragma unroll
     for (int k = 0; k < APL; k++) {
@@ -64,7 +64,7 @@ __device__ __forceinline__ void pose_features(const Ctx<APL>& C, const WPose<APL
             p7 = e > 0.0f ? gc : 0.0f;
             curl += e > 0.0f ? e / (1.0f + e) : e;
         }
-        if (a < C.natom) {
+        if (a < natom) {
             float* r = s_lds + sc + 8 * a;
             r[0] = cls; r[1] = p1; r[2] = p2; r[3] = p3; r[4] = p4; r[5] = p5; r[6] = p6; r[7] = p7;
         }
@@ -74,7 +74,7 @@ __device__ __forceinline__ void pose_features(const Ctx<APL>& C, const WPose<APL
     const int st = ln & 7;
     float f = 0.0f;
 #pragma unroll 4
-    for (int a = 0; a < C.natom; a++) {
+    for (int a = 0; a < natom; a++) {
         const float c = s_lds[sc + 8 * a];
         const float v = st == 0 ? 1.0f : s_lds[sc + 8 * a + st];
         f += c == my_cls ? v : 0.0f;
@@ -87,14 +87,22 @@ __device__ __forceinline__ void pose_features(const Ctx<APL>& C, const WPose<APL
         if (ln == 1) g = mv.kind == 1 ? 1.0f : 0.0f;
         if (ln == 2) g = mv.kind == 2 ? 1.0f : 0.0f;
         if (ln == 3) g = mv.mag;
-        if (ln == 4) g = float(C.nheavy) / 64.0f;
-        if (ln == 5) g = float(C.ntors) / 16.0f;
+        if (ln == 4) g = float(C.nheavy()) / 64.0f;
+        if (ln == 5) g = float(C.ntors()) / 16.0f;
         if (ln == 6) g = fminf(fmaxf(e_acc, -20.0f), 20.0f) / 10.0f;
         if (ln == 7) g = mv.moved;
         if (ln == 8) g = fminf(fmaxf(curl, -20.0f), 20.0f) / 10.0f;
         xrow[kPooled + ln] = f2bf(g);
     }
     wave_lds_fence();
+}
+
+__device__ __forceinline__ MlpDev network(Karg<MlpDev>& w) {
+    MlpDev W;
+    W.w1t = w.w1t; W.w2t = w.w2t; W.w2p = w.w2p; W.w2 = w.w2;
+    W.b1 = w.b1; W.b2 = w.b2; W.w3 = w.w3; W.b3 = w.b3;
+    W.mu = w.mu; W.inv_sigma = w.inv_sigma;
+    return W;
 }
 
 // Persistent learned-proposal MC kernel. One-atom-per-lane ligands fit six
@@ -109,47 +117,48 @@ __device__ __forceinline__ void pose_features(const Ctx<APL>& C, const WPose<APL
 // three waves per SIMD (two slots) or two (three and four), as the MC kernel does.
 template <int APL, int POL>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) __attribute__((amdgpu_waves_per_eu(APL == 1 ? 6 : APL == 2 ? 3 : 2)))
-void lmc_kernel(LmcArgs A) {
-    const int policy = POL >= 0 ? POL : A.policy;
+void lmc_kernel(LmcArgs) {
+    Karg<LmcArgs>* const K = kernel_args<LmcArgs>();
+    const int policy = POL >= 0 ? POL : K->policy;
     const int w = threadIdx.x / kWave;
-    const int base = w * A.lds_floats_per_wave;
-    const int nchain = A.P.nchain;
-    const int n_items = A.n_order * nchain;
+    const int base = w * reread(K)->lds_floats_per_wave;
+    const int nchain = reread(K)->P.nchain;
+    const int n_items = reread(K)->n_order * nchain;
     const int ln = lane();
-    uint16_t* xl = reinterpret_cast<uint16_t*>(s_lds + base + A.lfeat);
-    uint16_t* a1l = reinterpret_cast<uint16_t*>(s_lds + base + A.la1);
-    uint16_t* a1lb = reinterpret_cast<uint16_t*>(s_lds + base + A.la1b);
+    uint16_t* xl = reinterpret_cast<uint16_t*>(s_lds + base + reread(K)->lfeat);
+    uint16_t* a1l = reinterpret_cast<uint16_t*>(s_lds + base + reread(K)->la1);
+    uint16_t* a1lb = reinterpret_cast<uint16_t*>(s_lds + base + reread(K)->la1b);
     for (;;) {
         int item = 0;
-        if (ln == 0) item = atomicAdd(A.counter, 1);
+        if (ln == 0) item = atomicAdd(reread(K)->counter, 1);
         item = __builtin_amdgcn_readfirstlane(item);
         if (item >= n_items) break;
-        const int lig = A.order[item / nchain];
+        const int lig = reread(K)->order[item / nchain];
         const int chain = item % nchain;
         const size_t pid = (size_t)lig * nchain + chain;
         Ctx<APL> C;
-        load_ctx(C, A.L, A.S, lig, POL >= 0 ? int(kGrid) : A.mode, base, A.hdim_ld);
-        Rng rng{A.seed, uint32_t(lig + A.lig_index_base), uint32_t(chain), 0u};
+        load_ctx(C, (KHead*)K, lig, POL >= 0 ? int(kGrid) : reread(K)->mode, base, reread(K)->hdim_ld);
+        Rng rng{reread(K)->seed, uint32_t(lig + reread(K)->lig_index_base), uint32_t(chain), 0u};
         C.evals = 0;
         int n_feat = 0;
         WPose<APL> acc;
-        initial_pose(C, A.L, lig, acc);
+        initial_pose(C, acc);
         // step -1 is the start pre-screen: n_start randomised starts (super-Fibonacci
         // orientations spread over n_start * nchain) go through the same candidate code
         // as the MC steps' mutations, and the chain starts from the best one (network,
         // or exact energy for the plain / exact policies)
-        const int ns = A.n_start;
-        const bool prescreen = A.randomize && ns > 1;
-        if (A.randomize && !prescreen) randomize(C, acc, rng, chain, nchain);
-        store_pose(A.L, A.P, lig, chain, acc);
+        const int ns = reread(K)->n_start;
+        const bool prescreen = reread(K)->randomize && ns > 1;
+        if (reread(K)->randomize && !prescreen) randomize(C, acc, rng, chain, nchain);
+        store_pose(C, reread(K)->P, lig, chain, acc);
         save_pose(C, acc, 1);  // the accepted pose lives in LDS between steps
         float best = 1e9f;
-        for (int step = prescreen ? -1 : 0; step < A.mc_steps; step++) {
+        for (int step = prescreen ? -1 : 0; step < reread(K)->mc_steps; step++) {
             const bool pre = step < 0;
             WPose<APL> cand;
             restore_pose(C, cand, 1);
             const float acc_e = cand.e;
-            const size_t crow = ((size_t)(pre ? 0 : step) * A.n_pose + pid) * kGroup;
+            const size_t crow = ((size_t)(pre ? 0 : step) * reread(K)->n_pose + pid) * kGroup;
             if (pre && policy != kPolicyLearned) {
                 float be = INFINITY;
                 uint32_t bs = rng.draw;
@@ -166,7 +175,7 @@ void lmc_kernel(LmcArgs A) {
                 Rng r3 = rng;
                 r3.draw = bs;
                 randomize(C, cand, r3, chain * ns + bk, nchain * ns);
-                store_pose(A.L, A.P, lig, chain, cand);
+                store_pose(C, reread(K)->P, lig, chain, cand);
                 save_pose(C, cand, 1);
                 continue;
             }
@@ -175,7 +184,7 @@ void lmc_kernel(LmcArgs A) {
             } else if (policy == kPolicyExact) {
                 float be = INFINITY;
                 uint32_t bs = rng.draw;
-                for (int c = 0; c < A.n_cand; c++) {
+                for (int c = 0; c < reread(K)->n_cand; c++) {
                     const uint32_t start = rng.draw;
                     WPose<APL> t;
                     restore_pose(C, t, 1);
@@ -190,7 +199,7 @@ void lmc_kernel(LmcArgs A) {
                 mutate(C, cand, r3);
             } else {
                 // candidate c starts at Philox block my_start of lane c
-                const int nc = pre ? ns : A.n_cand;
+                const int nc = pre ? ns : reread(K)->n_cand;
                 uint32_t my_start = 0;
                 // the candidate rows sit in the coordinate / pair-force area: randomised starts must
                 // not stage their torsion steps there
@@ -206,14 +215,15 @@ void lmc_kernel(LmcArgs A) {
                     } else {
                         mv = mutate(C, t, rng);
                     }
-                    uint16_t* dst = policy == kPolicyCollect ? A.collect_x + (crow + c) * kFeat : xl + c * kFeat;
-                    pose_features(C, t, mv, pre ? 999.0f : acc_e, base + A.lscr, dst);
+                    uint16_t* dst = policy == kPolicyCollect ? reread(K)->collect_x + (crow + c) * kFeat : xl + c * kFeat;
+                    pose_features(C, t, mv, pre ? 999.0f : acc_e, base + reread(K)->lscr, dst);
                 }
                 n_feat += nc;
                 C.stage = true;  // no pose update until the network has read the rows
                 if (policy == kPolicyLearned) {
                     wave_lds_fence();
-                    float p = mlp_group_scores_lds(A.W, xl, a1l, a1lb, A.a1_split, A.a1_rows);  // lane 16 q + r: score of candidate r
+                    const MlpDev W = network(reread(K)->W);
+                    float p = mlp_group_scores_lds(W, xl, a1l, a1lb, reread(K)->a1_split, reread(K)->a1_rows);  // lane 16 q + r: score of candidate r
                     p = (ln < nc && p == p) ? p : INFINITY;
                     int rank = 0;
                     float pmin = INFINITY;
@@ -232,13 +242,13 @@ void lmc_kernel(LmcArgs A) {
                         r3.draw = bs;
                         restore_pose(C, cand, 1);
                         randomize(C, cand, r3, chain * ns + pick, nchain * ns);
-                        store_pose(A.L, A.P, lig, chain, cand);
+                        store_pose(C, reread(K)->P, lig, chain, cand);
                         save_pose(C, cand, 1);
                         continue;
                     }
-                    if (A.sel_temp > 0.0f) {
+                    if (reread(K)->sel_temp > 0.0f) {
                         // one candidate drawn with p ~ exp(-(score - min) / T); no exact rescoring
-                        const float w = (ln < nc && pmin < INFINITY) ? __expf(-(p - pmin) / A.sel_temp) : 0.0f;
+                        const float w = (ln < nc && pmin < INFINITY) ? __expf(-(p - pmin) / reread(K)->sel_temp) : 0.0f;
                         float wsum = 0.0f;
                         for (int j = 0; j < nc; j++) wsum += rdl(w, j);
                         const float target = u01(rng.next().x) * wsum;
@@ -250,7 +260,7 @@ void lmc_kernel(LmcArgs A) {
                         pick = pick < nc ? pick : nc - 1;
                         bs = uint32_t(rdl_i(int(my_start), pick));
                     }
-                    for (int r = 0; A.sel_temp <= 0.0f && r < A.top_k; r++) {
+                    for (int r = 0; reread(K)->sel_temp <= 0.0f && r < reread(K)->top_k; r++) {
                         const unsigned long long m = __ballot(ln < nc && rank == r);
                         const int c = __ffsll((long long)m) - 1;
                         const uint32_t start = uint32_t(rdl_i(int(my_start), c));
@@ -275,71 +285,73 @@ void lmc_kernel(LmcArgs A) {
                         WPose<APL> t;
                         restore_pose(C, t, 1);
                         mutate(C, t, r2);
-                        if (A.collect_e0) {
+                        if (reread(K)->collect_e0) {
                             Forces<APL> F;
                             const float e0 = energy_forces(C, t, kVCap, kSlope, F);
-                            if (ln == 0) A.collect_e0[crow + c] = e0;
+                            if (ln == 0) reread(K)->collect_e0[crow + c] = e0;
                         }
-                        bfgs(C, t, A.opt_steps, kVCap, kSlope);
-                        if (ln == 0) A.collect_y[crow + c] = t.e;
+                        bfgs(C, t, reread(K)->opt_steps, kVCap, kSlope);
+                        if (ln == 0) reread(K)->collect_y[crow + c] = t.e;
                     }
                     Rng r2 = rng;
                     r2.draw = uint32_t(rdl_i(int(my_start), 0));
                     restore_pose(C, cand, 1);
                     mutate(C, cand, r2);
-                    if (A.collect_e0) {
+                    if (reread(K)->collect_e0) {
                         Forces<APL> F;
                         const float e0 = energy_forces(C, cand, kVCap, kSlope, F);
-                        if (ln == 0) A.collect_e0[crow] = e0;
+                        if (ln == 0) reread(K)->collect_e0[crow] = e0;
                     }
                 }
             }
-            if (A.opt_steps == 0) {
+            if (reread(K)->opt_steps == 0) {
                 float gd;
                 cand.e = energy_grad(C, cand, kVCap, kSlope, gd);
             } else {
-                bfgs(C, cand, A.opt_steps, kVCap, kSlope);
+                bfgs(C, cand, reread(K)->opt_steps, kVCap, kSlope);
             }
-            if (policy == kPolicyCollect && ln == 0) A.collect_y[crow] = cand.e;
+            if (policy == kPolicyCollect && ln == 0) reread(K)->collect_y[crow] = cand.e;
             const uint4 b = rng.next();
             const bool accepted = (cand.e < acc_e) || (u01(b.x) < __expf((acc_e - cand.e) / 1.2f));
             if (step == 0 || accepted) {
                 if (cand.e < best) {
-                    if (A.opt_steps > 0) bfgs(C, cand, A.opt_steps, kVCapAuth, kSlope);
+                    if (reread(K)->opt_steps > 0) bfgs(C, cand, reread(K)->opt_steps, kVCapAuth, kSlope);
                     if (cand.e < best) {
-                        store_pose(A.L, A.P, lig, chain, cand);
+                        store_pose(C, reread(K)->P, lig, chain, cand);
                         best = cand.e;
                     }
                 }
                 save_pose(C, cand, 1);
             }
         }
-        if (A.stats && ln == 0) {
+        if (reread(K)->stats && ln == 0) {
             const unsigned long long ev = (unsigned long long)C.evals;
-            const unsigned long long nh = (unsigned long long)C.nheavy;
-            atomicAdd(&A.stats[0], ev);
-            atomicAdd(&A.stats[1], (ev + (unsigned long long)n_feat) * 32ull * nh);
-            atomicAdd(&A.stats[2], ev * (unsigned long long)C.npair);
-            atomicAdd(&A.stats[3], 1ull);
+            const unsigned long long nh = (unsigned long long)C.nheavy();
+            atomicAdd(&reread(K)->stats[0], ev);
+            atomicAdd(&reread(K)->stats[1], (ev + (unsigned long long)n_feat) * 32ull * nh);
+            atomicAdd(&reread(K)->stats[2], ev * (unsigned long long)C.npair());
+            atomicAdd(&reread(K)->stats[3], 1ull);
         }
     }
 }
 
 // Features of selected poses (no move: kind -1, accepted energy 0).
 template <int APL>
-__global__ __launch_bounds__(kWave* kWavesPerBlock) void features_kernel(FeatArgs A) {
+__global__ __launch_bounds__(kWave* kWavesPerBlock) void features_kernel(FeatArgs) {
+    Karg<FeatArgs>* const K = kernel_args<FeatArgs>();
+    Karg<FeatArgs>& A = *K;
     const int w = threadIdx.x / kWave;
     const int s = blockIdx.x * kWavesPerBlock + w;
     if (s >= A.n_sel) return;
     const int pid = A.sel[s];
     const int lig = pid / A.P.nchain, chain = pid % A.P.nchain;
     Ctx<APL> C;
-    load_ctx(C, A.L, A.S, lig, kGrid, w * A.lds_floats_per_wave, A.hdim_ld);
+    load_ctx(C, (KHead*)K, lig, kGrid, w * A.lds_floats_per_wave, A.hdim_ld);
     WPose<APL> p;
-    load_pose<APL>(A.L, A.P, lig, chain, p);
+    load_pose<APL>(C, A.P, lig, chain, p);
     Move mv;
     mv.kind = -1; mv.mag = 0.0f; mv.moved = 0.0f;
-    pose_features(C, p, mv, 0.0f, C.lh, A.x + (size_t)s * kFeat);
+    pose_features(C, p, mv, 0.0f, C.lh(), A.x + (size_t)s * kFeat);
 }
 
 // ------------------------------------------------------------- launchers
