@@ -1597,27 +1597,27 @@ struct ud2_mlp {
     float* d_params = nullptr;  // canonical FP32 parameters, then mu and inv_sigma
     float* d_m = nullptr;       // Adam moments
     float* d_v = nullptr;
-    float* d_grad = nullptr;
-    uint16_t* d_w1t = nullptr;
+    uint16_t* d_w1 = nullptr;
+    uint16_t* d_w1s = nullptr;
     uint16_t* d_w2t = nullptr;
-    uint16_t* d_w2p = nullptr;
+    uint16_t* d_w2s = nullptr;
     uint16_t* d_w2 = nullptr;
     float* d_w3r = nullptr;
     int32_t step = 0;
     // training scratch, sized for cap_groups groups
     int32_t cap_groups = 0;
-    float* d_yhat = nullptr;
-    float* d_dy = nullptr;
-    uint16_t* d_fm = nullptr;   // xn, a1, dz1, dz2 feature-major
+    uint16_t* d_fm = nullptr;   // xn, a1, dz1, dz2 (MlpTrain)
     float* d_part = nullptr;
     float* d_gpart = nullptr;   // split-K partials of the weight-gradient GEMMs
-    float* d_lparts = nullptr;
+
+    MlpPack pack() const { return MlpPack{d_w1, d_w1s, d_w2t, d_w2s, d_w2, d_w3r}; }
 
     MlpDev view() const {
         MlpDev w;
-        w.w1t = d_w1t;
+        w.w1 = d_w1;
+        w.w1s = d_w1s;
         w.w2t = d_w2t;
-        w.w2p = d_w2p;
+        w.w2s = d_w2s;
         w.w2 = d_w2;
         w.b1 = d_params + kOffB1;
         w.b2 = d_params + kOffB2;
@@ -1631,13 +1631,13 @@ struct ud2_mlp {
 
 namespace {
 
+// Ranges of the weight-gradient GEMMs' rows: 16 ranges of 40 tiles are 640 waves.
 constexpr int kGemmSplits = 16;
 
 void free_train(ud2_mlp* m) {
-    for (void* p : {(void*)m->d_yhat, (void*)m->d_dy, (void*)m->d_fm, (void*)m->d_part, (void*)m->d_gpart,
-                    (void*)m->d_lparts})
+    for (void* p : {(void*)m->d_fm, (void*)m->d_part, (void*)m->d_gpart})
         if (p) (void)hipFree(p);
-    m->d_yhat = m->d_dy = m->d_part = m->d_gpart = m->d_lparts = nullptr;
+    m->d_part = m->d_gpart = nullptr;
     m->d_fm = nullptr;
     m->cap_groups = 0;
 }
@@ -1646,12 +1646,9 @@ int ensure_train(ud2_mlp* m, int32_t n_groups) {
     if (n_groups <= m->cap_groups) return UD2_OK;
     free_train(m);
     const size_t rows = size_t(n_groups) * kGroup;
-    UD2_HIP(hipMalloc(reinterpret_cast<void**>(&m->d_yhat), rows * sizeof(float)));
-    UD2_HIP(hipMalloc(reinterpret_cast<void**>(&m->d_dy), rows * sizeof(float)));
     UD2_HIP(hipMalloc(reinterpret_cast<void**>(&m->d_fm), rows * size_t(kFeat + 3 * kHidden) * sizeof(uint16_t)));
     UD2_HIP(hipMalloc(reinterpret_cast<void**>(&m->d_part), size_t(n_groups) * kPartStride * sizeof(float)));
-    UD2_HIP(hipMalloc(reinterpret_cast<void**>(&m->d_gpart), size_t(kGemmSplits) * kHidden * kHidden * sizeof(float)));
-    UD2_HIP(hipMalloc(reinterpret_cast<void**>(&m->d_lparts), size_t(n_groups) * sizeof(float)));
+    UD2_HIP(hipMalloc(reinterpret_cast<void**>(&m->d_gpart), size_t(kGemmSplits) * kGradW * sizeof(float)));
     m->cap_groups = n_groups;
     return UD2_OK;
 }
@@ -1663,9 +1660,10 @@ int check_mlp_inputs(const uint16_t* x_d, int32_t n_groups) {
     return UD2_OK;
 }
 
-// Backward pass and gradient reductions of the minibatch whose d loss / d y_hat is in dy.
-int mlp_grads(ud2_mlp* m, const uint16_t* x_d, const int32_t* groups_d, int32_t n_groups, const float* dy,
-              hipStream_t st) {
+// The minibatch's partial sums (dy null: of the loss to label_d; else for the given d loss / d y_hat), then the
+// gradient into grad, or the Adam step O where grad is null.
+int mlp_step(ud2_mlp* m, const uint16_t* x_d, const float* label_d, const int32_t* groups_d, int32_t n_groups,
+             const float* dy, float* grad, const MlpAdam& O, hipStream_t st) {
     int rc = ensure_train(m, n_groups);
     if (rc) return rc;
     const size_t rows = size_t(n_groups) * kGroup;
@@ -1673,19 +1671,17 @@ int mlp_grads(ud2_mlp* m, const uint16_t* x_d, const int32_t* groups_d, int32_t 
     T.x = x_d;
     T.groups = groups_d;
     T.n_groups = n_groups;
+    T.label = label_d;
     T.dy = dy;
-    T.xn_fm = m->d_fm;
-    T.a1_fm = T.xn_fm + rows * kFeat;
-    T.dz1_fm = T.a1_fm + rows * kHidden;
-    T.dz2_fm = T.dz1_fm + rows * kHidden;
+    T.xn = m->d_fm;
+    T.a1 = T.xn + rows * kFeat;
+    T.dz1 = T.a1 + rows * kHidden;
+    T.dz2 = T.dz1 + rows * kHidden;
     T.part = m->d_part;
-    UD2_HIP(launch_mlp_backward(m->view(), T, st));
     int splits = kGemmSplits;
     while (splits > 1 && n_groups % splits) splits >>= 1;
-    // dW1[f][h] = sum_r xn[r][f] dz1[r][h]; dW2[h][o] = sum_r a1[r][h] dz2[r][o]
-    UD2_HIP(launch_gemm_nt(T.xn_fm, T.dz1_fm, kFeat, kHidden, int(rows), splits, m->d_gpart, m->d_grad + kOffW1, st));
-    UD2_HIP(launch_gemm_nt(T.a1_fm, T.dz2_fm, kHidden, kHidden, int(rows), splits, m->d_gpart, m->d_grad + kOffW2, st));
-    UD2_HIP(launch_mlp_reduce_parts(m->d_part, n_groups, m->d_grad, st));
+    UD2_HIP(launch_mlp_train(m->view(), T, splits, m->d_gpart, st));
+    UD2_HIP(launch_mlp_update(m->d_gpart, splits, m->d_part, n_groups, grad, O, m->pack(), st));
     return UD2_OK;
 }
 
@@ -1705,10 +1701,10 @@ int ud2_mlp_create(const float* params_h, ud2_mlp** out) {
     al(reinterpret_cast<void**>(&m->d_params), (np + kMlpNNorm) * sizeof(float));
     al(reinterpret_cast<void**>(&m->d_m), np * sizeof(float));
     al(reinterpret_cast<void**>(&m->d_v), np * sizeof(float));
-    al(reinterpret_cast<void**>(&m->d_grad), np * sizeof(float));
-    al(reinterpret_cast<void**>(&m->d_w1t), size_t(kFeat) * kHidden * sizeof(uint16_t));
+    al(reinterpret_cast<void**>(&m->d_w1), size_t(kFeat) * kHidden * sizeof(uint16_t));
+    al(reinterpret_cast<void**>(&m->d_w1s), size_t(kW1sSize) * sizeof(uint16_t));
     al(reinterpret_cast<void**>(&m->d_w2t), size_t(kHidden) * kHidden * sizeof(uint16_t));
-    al(reinterpret_cast<void**>(&m->d_w2p), size_t(kHidden) * kHidden * sizeof(uint16_t));
+    al(reinterpret_cast<void**>(&m->d_w2s), size_t(kHidden) * kHidden * sizeof(uint16_t));
     al(reinterpret_cast<void**>(&m->d_w2), size_t(kHidden) * kHidden * sizeof(uint16_t));
     al(reinterpret_cast<void**>(&m->d_w3r), size_t(kHidden) * sizeof(float));
     if (rc == UD2_OK) rc = ud2_mlp_set_params(m, params_h);
@@ -1730,7 +1726,8 @@ int ud2_mlp_set_params(ud2_mlp* m, const float* params_h) {
     UD2_HIP(hipMemset(m->d_m, 0, size_t(kMlpNParam) * sizeof(float)));
     UD2_HIP(hipMemset(m->d_v, 0, size_t(kMlpNParam) * sizeof(float)));
     m->step = 0;
-    UD2_HIP(launch_mlp_pack(m->d_params, m->d_w1t, m->d_w2t, m->d_w2p, m->d_w2, m->d_w3r, nullptr));
+    UD2_HIP(hipMemset(m->d_w1s, 0, size_t(kW1sSize) * sizeof(uint16_t)));  // the features past 79 of the last K block
+    UD2_HIP(launch_mlp_pack(m->d_params, m->pack(), nullptr));
     UD2_HIP(hipDeviceSynchronize());
     return UD2_OK;
 }
@@ -1745,8 +1742,8 @@ int ud2_mlp_get_params(const ud2_mlp* m, float* params_h) {
 int ud2_mlp_destroy(ud2_mlp* m) {
     if (!m) return UD2_OK;
     free_train(m);
-    for (void* p : {(void*)m->d_params, (void*)m->d_m, (void*)m->d_v, (void*)m->d_grad, (void*)m->d_w1t,
-                    (void*)m->d_w2t, (void*)m->d_w2p, (void*)m->d_w2, (void*)m->d_w3r})
+    for (void* p : {(void*)m->d_params, (void*)m->d_m, (void*)m->d_v, (void*)m->d_w1, (void*)m->d_w1s,
+                    (void*)m->d_w2t, (void*)m->d_w2s, (void*)m->d_w2, (void*)m->d_w3r})
         if (p) (void)hipFree(p);
     delete m;
     return UD2_OK;
@@ -1766,11 +1763,7 @@ int ud2_mlp_backward(ud2_mlp* m, const uint16_t* x_d, const int32_t* groups_d, i
     if (!m || !dy_d || !grad_d) return fail(UD2_ERR_ARG, "null argument");
     int rc = check_mlp_inputs(x_d, n_groups);
     if (rc) return rc;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    rc = mlp_grads(m, x_d, groups_d, n_groups, dy_d, st);
-    if (rc) return rc;
-    UD2_HIP(hipMemcpyAsync(grad_d, m->d_grad, size_t(kMlpNParam) * sizeof(float), hipMemcpyDeviceToDevice, st));
-    return UD2_OK;
+    return mlp_step(m, x_d, nullptr, groups_d, n_groups, dy_d, grad_d, MlpAdam{}, static_cast<hipStream_t>(stream));
 }
 
 int ud2_mlp_train_step(ud2_mlp* m, const uint16_t* x_d, const float* label_d, const int32_t* groups_d,
@@ -1781,21 +1774,22 @@ int ud2_mlp_train_step(ud2_mlp* m, const uint16_t* x_d, const float* label_d, co
     if (!(opt->lr > 0.0f) || !(opt->beta1 >= 0.0f && opt->beta1 < 1.0f) || !(opt->beta2 >= 0.0f && opt->beta2 < 1.0f) ||
         !(opt->eps > 0.0f))
         return fail(UD2_ERR_ARG, "invalid Adam settings");
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    rc = ensure_train(m, n_groups);
-    if (rc) return rc;
-    UD2_HIP(launch_mlp_forward(m->view(), x_d, groups_d, n_groups, m->d_yhat, st));
-    float* loss = loss_d ? loss_d : m->d_lparts;  // without a loss output the partials' slot 0 takes the sum
-    UD2_HIP(launch_group_loss(m->d_yhat, label_d, groups_d, n_groups, m->d_dy, m->d_lparts, loss, st));
-    rc = mlp_grads(m, x_d, groups_d, n_groups, m->d_dy, st);
-    if (rc) return rc;
-    m->step++;
-    const float c1 = 1.0f - std::pow(opt->beta1, float(m->step));
-    const float c2 = 1.0f - std::pow(opt->beta2, float(m->step));
-    UD2_HIP(launch_adam(m->d_params, m->d_m, m->d_v, m->d_grad, kMlpNParam, opt->lr, opt->beta1, opt->beta2, opt->eps,
-                        c1, c2, st));
-    UD2_HIP(launch_mlp_pack(m->d_params, m->d_w1t, m->d_w2t, m->d_w2p, m->d_w2, m->d_w3r, st));
-    return UD2_OK;
+    const int32_t step = m->step + 1;
+    MlpAdam O;
+    O.p = m->d_params;
+    O.m = m->d_m;
+    O.v = m->d_v;
+    O.lr = opt->lr;
+    O.beta1 = opt->beta1;
+    O.beta2 = opt->beta2;
+    O.eps = opt->eps;
+    O.c1 = 1.0f - std::pow(opt->beta1, float(step));
+    O.c2 = 1.0f - std::pow(opt->beta2, float(step));
+    O.loss = loss_d;
+    O.loss_scale = 1.0f / (float(n_groups) * kGroup);
+    rc = mlp_step(m, x_d, label_d, groups_d, n_groups, nullptr, nullptr, O, static_cast<hipStream_t>(stream));
+    if (rc == UD2_OK) m->step = step;
+    return rc;
 }
 
 int ud2_features(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P, const int32_t* sel_d, int32_t n_sel,

@@ -13,6 +13,7 @@ constexpr int kMaxApl = 4;                  // atoms per lane: natom <= 256
 constexpr int kMaxAtoms = kWave * kMaxApl;  // pair records pack atom indices in 8 bits
 constexpr int kMaxTors = 57;                // 7 + ntors <= 64: one pose-vector / BFGS component per lane
 constexpr int kWavesPerBlock = 4;
+constexpr int kXcds = 8;                    // blocks are dealt round the chip's XCDs, each with its own L2 cache
 // The narrow tile of the MC search: two chains of a ligand per wave, one per 32 lanes, for ligands of
 // at most kTileNarrow atoms and kTileNarrowTors torsions (every torsion step of a pose update staged
 // in the tile's LDS, as a whole wave stages them, so both round alike).
@@ -245,12 +246,24 @@ constexpr int kMlpNNorm = 2 * kFeat;
 constexpr int kOffW1 = 0, kOffB1 = kFeat * kHidden, kOffW2 = kOffB1 + kHidden, kOffB2 = kOffW2 + kHidden * kHidden,
               kOffW3 = kOffB2 + kHidden, kOffB3 = kOffW3 + kHidden;
 
+// Place of A[row][k] of a weight matrix in its fragments of 16 rows by 16 or 32 k, nk fragments along k: lane l of a
+// fragment holds row l % 16 and the 4 or 8 k from 4 (l / 16) or 8 (l / 16) on.
+__host__ __device__ constexpr int frag16(int row, int k, int nk) {
+    return ((row / 16 * nk + k / 16) * kWave + 16 * (k % 16 / 4) + row % 16) * 4 + k % 4;
+}
+__host__ __device__ constexpr int frag32(int row, int k, int nk) {
+    return ((row / 16 * nk + k / 32) * kWave + 16 * (k % 32 / 8) + row % 16) * 8 + k % 8;
+}
+
 // Device copies of the network used by the MFMA kernels.
 struct MlpDev {
-    const uint16_t* w1t;  // [256][80] bf16, W1 transposed (hidden-major)
-    const uint16_t* w2t;  // [256 out][256 in] bf16
-    const uint16_t* w2p;  // [256 out][256 in] bf16, the in-units in the K = 32 order of the scoring MFMAs (k32_slot)
-    const uint16_t* w2;   // [256 in][256 out] bf16 (backward)
+    // bf16 weights as A operands, fragment by fragment: the 64 lanes' values of one MFMA lie together, in the
+    // order of the lanes (frag16, frag32), so that a wave's load is 512 or 1,024 consecutive bytes
+    const uint16_t* w1;   // [16 tiles][5 K blocks] 16x16x16 fragments of W1 transposed (rows: hidden units)
+    const uint16_t* w1s;  // [16][3] 16x16x32 fragments of it, zero past feature 79 (scoring)
+    const uint16_t* w2t;  // [16][16] 16x16x16 fragments of W2 transposed (rows: out-units)
+    const uint16_t* w2s;  // [16][8] 16x16x32 fragments of it, the in-units in the K = 32 order (k32_slot) (scoring)
+    const uint16_t* w2;   // [16][16] 16x16x16 fragments of W2 (rows: in-units) (backward)
     const float* b1;      // [256]
     const float* b2;      // [256]
     const float* w3;      // [256], values rounded to bf16
@@ -264,14 +277,34 @@ struct MlpTrain {
     const uint16_t* x;       // dataset features [*][80]
     const int32_t* groups;   // dataset group of each minibatch group (null: identity)
     int32_t n_groups;
-    const float* dy;         // [rows] d loss / d y_hat
-    uint16_t* xn_fm;         // [80][rows] normalised inputs, feature-major
-    uint16_t* a1_fm;         // [256][rows]
-    uint16_t* dz1_fm;        // [256][rows]
-    uint16_t* dz2_fm;        // [256][rows]
-    float* part;             // [n_groups][kPartStride]: dw3, db2, db1, db3 partial sums
+    const float* label;      // dataset labels [*], for the loss
+    const float* dy;         // [rows] d loss / d y_hat; null: of the loss
+    // operands of the weight-gradient GEMMs in bf16: 16x16x16 fragments [tiles of 16 units][groups] with the units as
+    // rows and the group's 16 candidates as k (frag16)
+    uint16_t* xn;            // normalised inputs, 5 tiles
+    uint16_t* a1;            // 16 tiles each
+    uint16_t* dz1;
+    uint16_t* dz2;
+    float* part;             // [n_groups][kPartStride]: partial sums of dw3, db2, db1, db3 and the loss
 };
-constexpr int kPartStride = 3 * kHidden + 4;
+constexpr int kPartStride = 3 * kHidden + 16;  // whole blocks of 16 sums
+constexpr int kGradW = kFeat * kHidden + kHidden * kHidden;  // weights with GEMM gradients: W1, then W2
+
+constexpr int kW1sSize = kHidden * 96;  // W1's 16x16x32 fragments: three K blocks
+
+// bf16 copies of the weights that an update writes (MlpDev).
+struct MlpPack {
+    uint16_t *w1, *w1s, *w2t, *w2s, *w2;
+    float* w3r;
+};
+
+// Adam's state and settings, and where the loss goes (may be null).
+struct MlpAdam {
+    float *p, *m, *v;
+    float lr, beta1, beta2, eps, c1, c2;
+    float* loss;
+    float loss_scale;
+};
 
 enum LmcPolicy : int32_t { kPolicyPlain = 0, kPolicyExact = 1, kPolicyLearned = 2, kPolicyCollect = 3 };
 
@@ -363,15 +396,9 @@ hipError_t launch_features(FeatArgs a, int apl, hipStream_t s);
 int lmc_blocks_per_cu(int apl, int policy, int mode, int lds_bytes_per_block);
 hipError_t launch_mlp_forward(const MlpDev& W, const uint16_t* x, const int32_t* groups, int64_t n_groups, float* y,
                               hipStream_t s);
-hipError_t launch_mlp_backward(const MlpDev& W, const MlpTrain& T, hipStream_t s);
-hipError_t launch_gemm_nt(const uint16_t* A, const uint16_t* B, int M, int N, int K, int splits, float* part,
-                          float* C, hipStream_t s);
-hipError_t launch_mlp_reduce_parts(const float* part, int n_groups, float* grad, hipStream_t s);
-hipError_t launch_group_loss(const float* yhat, const float* label, const int32_t* groups, int n_groups, float* dy,
-                             float* loss_parts, float* loss, hipStream_t s);
-hipError_t launch_adam(float* p, float* m, float* v, const float* g, int n, float lr, float beta1, float beta2,
-                       float eps, float c1, float c2, hipStream_t s);
-hipError_t launch_mlp_pack(const float* params, uint16_t* w1t, uint16_t* w2t, uint16_t* w2p, uint16_t* w2,
-                           float* w3r, hipStream_t s);
+hipError_t launch_mlp_train(const MlpDev& W, const MlpTrain& T, int splits, float* gpart, hipStream_t s);
+hipError_t launch_mlp_update(const float* gpart, int splits, const float* part, int n_groups, float* grad,
+                             const MlpAdam& O, const MlpPack& D, hipStream_t s);
+hipError_t launch_mlp_pack(const float* params, const MlpPack& D, hipStream_t s);
 
 }  // namespace ud2

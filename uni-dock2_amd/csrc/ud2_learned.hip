@@ -99,7 +99,7 @@ __device__ __forceinline__ void pose_features(const Ctx<APL>& C, const WPose<APL
 
 __device__ __forceinline__ MlpDev network(Karg<MlpDev>& w) {
     MlpDev W;
-    W.w1t = w.w1t; W.w2t = w.w2t; W.w2p = w.w2p; W.w2 = w.w2;
+    W.w1 = w.w1; W.w1s = w.w1s; W.w2t = w.w2t; W.w2s = w.w2s; W.w2 = w.w2;
     W.b1 = w.b1; W.b2 = w.b2; W.w3 = w.w3; W.b3 = w.b3;
     W.mu = w.mu; W.inv_sigma = w.inv_sigma;
     return W;

@@ -13,7 +13,7 @@
 // candidate l % 16 on lane l; the two tiles 2 kb and 2 kb + 1 together give lane
 // l the 8 hidden units 32 kb + 4 (l / 16) + {0..3, 16..19}, which is the B
 // operand of the next layer's K block kb when that layer's weights take the
-// same order of k (w2p, packed so), so hidden activations never leave the
+// same order of k (w2s, packed so), so hidden activations never leave the
 // registers. Layer 1 has K = 80: three 32-wide blocks, the last one zero past
 // k = 80 (lanes 32-63 hold zeros): a chain of accumulating MFMAs keeps one
 // opcode (an accumulator written by one MFMA opcode and read by another as
@@ -35,18 +35,18 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float(uint32_t(b) << 16); }
 __device__ __forceinline__ float bf2f_s(short b) { return bf2f(uint16_t(b)); }
 
-// Round to nearest even; NaN stays NaN (quietened), overflow rounds to inf.
-__device__ __forceinline__ uint16_t f2bf(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7F800000u) == 0x7F800000u) {
-        if (u & 0x007FFFFFu) u |= 0x00400000u;
-        return uint16_t(u >> 16);
-    }
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return uint16_t(u >> 16);
-}
+// Round to nearest even; NaN stays NaN (quietened), overflow rounds to inf: v_cvt_pk_bf16_f32, whose result is that
+// of the integer rounding for every float. A conversion in integer operations with a branch for infinities and NaN cut
+// the training kernel into a hundred basic blocks, each waiting for its own loads.
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f)); }
 
-__device__ __forceinline__ bf16x4 ld4(const uint16_t* p) { return *reinterpret_cast<const bf16x4*>(p); }
+// Loads of what no kernel that uses them writes (weights, and in the weight-gradient GEMMs the operands), through the
+// constant address space, so that they may be issued ahead of barriers and stores.
+template <class T>
+__device__ __forceinline__ T cload(const void* p) {
+    return *(const __attribute__((address_space(4))) T*)(p);
+}
+__device__ __forceinline__ bf16x4 ld4(const uint16_t* p) { return cload<bf16x4>(p); }
 
 __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
@@ -56,24 +56,36 @@ typedef short bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ bf16x8 ld8(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
+__device__ __forceinline__ bf16x8 ldw8(const uint16_t* p) { return cload<bf16x8>(p); }
 
 __device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
                                                    0, 0, 0);
 }
 
-// Place of hidden unit h in the K = 32 order of layer 2 (w2p and the staged hidden rows): h = 32 kb +
+// Place of hidden unit h in the K = 32 order of layer 2 (w2s and the staged hidden rows): h = 32 kb +
 // 16 t + 4 q + i goes to 32 kb + 8 q + 4 t + i.
 __host__ __device__ constexpr int k32_slot(int h) {
     return (h & ~31) + 8 * ((h >> 2) & 3) + 4 * ((h >> 4) & 1) + (h & 3);
 }
 
-// Sum over the 16 lanes of a lane row (lanes 16 q .. 16 q + 15).
+// Sum and minimum over the 16 lanes of a lane row (lanes 16 q .. 16 q + 15), by DPP row exchanges.
+template <int CTRL>
+__device__ __forceinline__ float row16_dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
 __device__ __forceinline__ float row16_sum(float v) {
-    v += __shfl_xor(v, 1);
-    v += __shfl_xor(v, 2);
-    v += __shfl_xor(v, 4);
-    v += __shfl_xor(v, 8);
+    v += row16_dpp<0xB1>(v);
+    v += row16_dpp<0x4E>(v);
+    v += row16_dpp<0x141>(v);
+    v += row16_dpp<0x140>(v);
+    return v;
+}
+__device__ __forceinline__ float row16_min(float v) {
+    v = fminf(v, row16_dpp<0xB1>(v));
+    v = fminf(v, row16_dpp<0x4E>(v));
+    v = fminf(v, row16_dpp<0x141>(v));
+    v = fminf(v, row16_dpp<0x140>(v));
     return v;
 }
 
@@ -90,25 +102,24 @@ __device__ __forceinline__ void load_inputs(const MlpDev& W, const uint16_t* xr,
     }
 }
 
-// Layer 1: a1 tiles (hidden 16 mt + 4 q + i of candidate `row` on this lane).
-__device__ __forceinline__ void layer1(const MlpDev& W, const bf16x4 xb[5], int row, int q, bf16x4 a1[16]) {
+// Layer-1 tile mt: hidden units 16 mt + 4 q + i of candidate `row`, after bias and ReLU, in bf16.
+__device__ __forceinline__ bf16x4 layer1_tile(const MlpDev& W, const bf16x4 xb[5], int mt, int row, int q) {
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    const uint16_t* wf = W.w1 + (mt * 5 * kWave + 16 * q + row) * 4;
 #pragma unroll
-    for (int mt = 0; mt < 16; mt++) {
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        const uint16_t* wr = W.w1t + (16 * mt + row) * kFeat + 4 * q;
+    for (int ks = 0; ks < 5; ks++) acc = mfma16(ld4(wf + ks * kWave * 4), xb[ks], acc);
+    bf16x4 h;
 #pragma unroll
-        for (int ks = 0; ks < 5; ks++) acc = mfma16(ld4(wr + 16 * ks), xb[ks], acc);
-#pragma unroll
-        for (int i = 0; i < 4; i++) a1[mt][i] = short(f2bf(fmaxf(acc[i] + W.b1[16 * mt + 4 * q + i], 0.0f)));
-    }
+    for (int i = 0; i < 4; i++) h[i] = short(f2bf(fmaxf(acc[i] + W.b1[16 * mt + 4 * q + i], 0.0f)));
+    return h;
 }
 
 // z2 tile ot (outputs 16 ot + 4 q + i of candidate `row`), before bias.
 __device__ __forceinline__ f32x4 layer2_tile(const MlpDev& W, const bf16x4 a1[16], int ot, int row, int q) {
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const uint16_t* wr = W.w2t + (16 * ot + row) * kHidden + 4 * q;
+    const uint16_t* wf = W.w2t + (ot * 16 * kWave + 16 * q + row) * 4;
 #pragma unroll
-    for (int kt = 0; kt < 16; kt++) acc = mfma16(ld4(wr + 16 * kt), a1[kt], acc);
+    for (int kt = 0; kt < 16; kt++) acc = mfma16(ld4(wf + kt * kWave * 4), a1[kt], acc);
     return acc;
 }
 
@@ -130,13 +141,10 @@ __device__ __forceinline__ void load_inputs32(const MlpDev& W, const uint16_t* x
 // Layer-1 tile mt in the scoring form: hidden units 16 mt + 4 q + i of candidate `row`, after bias and
 // ReLU, in bf16.
 __device__ __forceinline__ bf16x4 layer1_tile32(const MlpDev& W, const bf16x8 xb[3], int mt, int row, int q) {
-    const uint16_t* wr = W.w1t + (16 * mt + row) * kFeat;
-    const bf16x8 w2 = ld8(wr + 64 + 8 * (q & 1));  // in the row for every lane; zero for q >= 2
-    const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    const uint16_t* wf = W.w1s + (mt * 3 * kWave + 16 * q + row) * 8;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    acc = mfma32(ld8(wr + 8 * q), xb[0], acc);
-    acc = mfma32(ld8(wr + 32 + 8 * q), xb[1], acc);
-    acc = mfma32(q < 2 ? w2 : zero, xb[2], acc);
+#pragma unroll
+    for (int kb = 0; kb < 3; kb++) acc = mfma32(ldw8(wf + kb * kWave * 8), xb[kb], acc);
     bf16x4 h;
 #pragma unroll
     for (int i = 0; i < 4; i++) h[i] = short(f2bf(fmaxf(acc[i] + W.b1[16 * mt + 4 * q + i], 0.0f)));
@@ -170,9 +178,9 @@ __device__ __forceinline__ float mlp_group_scores(const MlpDev& W, const uint16_
 #pragma unroll 2
     for (int ot = 0; ot < 16; ot++) {
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        const uint16_t* wr = W.w2p + (16 * ot + row) * kHidden + 8 * q;
+        const uint16_t* wf = W.w2s + (ot * 8 * kWave + l) * 8;
 #pragma unroll
-        for (int kb = 0; kb < 8; kb++) acc = mfma32(ld8(wr + 32 * kb), a1[kb], acc);
+        for (int kb = 0; kb < 8; kb++) acc = mfma32(ldw8(wf + kb * kWave * 8), a1[kb], acc);
         yp += layer3_part(W, acc, ot, q);
     }
     yp += __shfl_xor(yp, 16);
@@ -209,9 +217,9 @@ __device__ __forceinline__ float mlp_group_scores_lds(const MlpDev& W, const uin
     const uint16_t* ar = a1row + 8 * q;
     for (int ot = 0; ot < 16; ot++) {
         f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        const uint16_t* wr = W.w2p + (16 * ot + row) * kHidden + 8 * q;
+        const uint16_t* wf = W.w2s + (ot * 8 * kWave + l) * 8;
 #pragma unroll 4
-        for (int kb = 0; kb < 8; kb++) acc = mfma32(ld8(wr + 32 * kb), ld8(ar + 32 * kb), acc);
+        for (int kb = 0; kb < 8; kb++) acc = mfma32(ldw8(wf + kb * kWave * 8), ld8(ar + 32 * kb), acc);
         yp += layer3_part(W, acc, ot, q);
     }
     yp += __shfl_xor(yp, 16);
