@@ -502,13 +502,20 @@ McArgs mc_args(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P, co
     return A;
 }
 
+// Searches of up to this many chains per CU, over all their launches, run each chain on a team of four waves (see
+// Team in ud2_device.h): a team evaluates 1.7 times what one wave would, on a chip that is idle otherwise. Both sides, plain searches at 128 chains per ligand, ms with one wave per chain / with a team: grid 128 chains 9.2 /
+// 5.9, 1,024 11.3 / 7.1, 2,048 15.4 / 12.6, 3,072 17.9 / 14.4, 4,096 19.2 / 18.0, 6,144 18.6 / 23.8; direct 128
+// 10.8 / 8.9, 1,024 14.1 / 10.2, 1,536 18.4 / 13.1, 2,048 16.3 / 16.8, 3,072 24.4 / 25.3 (256 CUs).
+constexpr int kTeamMaxApl = 2, kTeamPerCuGrid = 12, kTeamPerCuDirect = 6;
+
 // One persistent MC launch over n ligands of the work order at order (atoms-per-lane class apl, kernel
 // variant, largest 6 + ntors dmax), its queue head at counter.
+// chains: those of the whole search, with its other launches.
 // shared: the launch runs beside the one-slot class of the same search. A wider class then takes one block
 // per CU less than it could alone, so one-slot waves fit beside it (three two-slot waves of 168 VGPRs fill
 // a SIMD's register file, and the one-slot launch would wait for the whole two-slot queue to drain).
 int launch_mc_part(McArgs A, int apl, int variant, const int32_t* order, int n, int32_t* counter, int dmax,
-                   int nchain, hipStream_t st, bool shared = false) {
+                   int nchain, hipStream_t st, int64_t chains, bool shared = false) {
     if (n <= 0) return UD2_OK;
     // in direct mode the sum over the receptor outweighs what two chains per wave share: whole waves only
     if (A.mode == kDirect) variant = kMcWhole;
@@ -522,6 +529,13 @@ int launch_mc_part(McArgs A, int apl, int variant, const int32_t* order, int n, 
     const int lds_bytes = A.lds_floats_per_wave * kWavesPerBlock * int(sizeof(float));
     if (lds_bytes > 160 * 1024) return fail(UD2_ERR_LIMIT, "per-block LDS exceeds 160 KB");
     const int64_t items = int64_t(n) * ((nchain + cpw - 1) / cpw);
+    const int team_per_cu = A.mode == kDirect ? kTeamPerCuDirect : kTeamPerCuGrid;
+    if (variant == kMcWhole && apl <= kTeamMaxApl && A.mc_steps > 0 && A.opt_steps > 0 &&
+        chains <= int64_t(team_per_cu) * n_cus() &&
+        lds_bytes + team_floats(apl) * int(sizeof(float)) <= 160 * 1024) {
+        UD2_HIP(launch_mc_team(A, apl, int(items), st));
+        return UD2_OK;
+    }
     const int64_t need = (items + kWavesPerBlock - 1) / kWavesPerBlock;
     int bpc = mc_blocks_per_cu(apl, variant, A.mode, lds_bytes);
     if (shared && apl > 1) bpc = std::max(1, bpc - 1);
@@ -604,7 +618,7 @@ int launch_mc_classes(const ud2_ligset* ls, const ud2_poses* P, McArgs A, int32_
             used[k] = true;
         }
         rc = launch_mc_part(A, p.apl, p.variant, p.order, p.n, p.head, p.dmax, P->nchain, s,
-                            S != nullptr && ls->cls_cnt[1] > 0);
+                            int64_t(ls->n_lig) * P->nchain, S != nullptr && ls->cls_cnt[1] > 0);
         if (rc) return rc;
     }
     for (int k = 0; S && k < kMcSide; k++)
@@ -1425,7 +1439,7 @@ int ud2_autotune(const ud2_scene* sc, const ud2_ligset* ls, const ud2_mc_params*
         // probe searches with the caller's parameters: each bucket's ligands, repeated until the launch
         // holds two rounds of the chip's resident whole-wave chains, searched with every variant (each
         // variant run once untimed first); a half-wave variant replaces whole waves only when it is at
-        // least 2% faster. Repeated ligands write the same pose slots (the probe's poses are discarded).
+        // least 2% faster (in direct mode every variant runs whole waves). Repeated ligands write the same pose slots (the probe's poses are discarded).
         const DevLig& last = ls->h_ligs.back();
         const int64_t n_atoms = int64_t(last.atom_off) + last.natom, n_tors = int64_t(last.tors_off) + last.ntors;
         float *x = nullptr, *c = nullptr, *rv = nullptr, *dh = nullptr, *e = nullptr;
@@ -1465,7 +1479,8 @@ int ud2_autotune(const ud2_scene* sc, const ud2_ligset* ls, const ud2_mc_params*
                     for (int v = 0; v < kMcVariants; v++) {
                         UD2_HIP(launch_fill_i32(head, 0, 1, st));
                         UD2_HIP(hipEventRecord(ev0, st));
-                        const int r = launch_mc_part(A, 1, v, ord, reps, head, dmax, nchain, st);
+                        const int r = launch_mc_part(A, 1, v, ord, reps, head, dmax, nchain, st,
+                                                     int64_t(reps) * nchain);
                         if (r) return r;
                         UD2_HIP(hipEventRecord(ev1, st));
                         UD2_HIP(hipEventSynchronize(ev1));
@@ -1480,7 +1495,7 @@ int ud2_autotune(const ud2_scene* sc, const ud2_ligset* ls, const ud2_mc_params*
                     ms[b][v] = best[v];
                     if (v != kMcWhole && best[v] < best[fast]) fast = v;
                 }
-                choice[b] = int8_t(best[fast] < 0.98f * best[kMcWhole] ? fast : kMcWhole);
+                choice[b] = int8_t(prm->mode != kDirect && best[fast] < 0.98f * best[kMcWhole] ? fast : kMcWhole);
             }
             return UD2_OK;
         };

@@ -1365,6 +1365,19 @@ __device__ __forceinline__ float energy_lower_bound(const Ctx<APL, TW, LAZY>& C,
     return tuni<TW>(tsum<TW>(pen) * slope - 0.67f * (float(S.nrec) * float(C.nheavy()) + float(C.npair())));
 }
 
+// How many waves run a chain. Solo: one. Team: the four of a block, each with the chain's whole state in its own
+// registers and LDS slice and computing the same bits, so that they take the same branches; a line search
+// evaluates four trial steps at a time, one per wave, and every wave goes on with the one the sequential
+// search would have ended on. sh: the block's shared area in LDS (floats).
+struct Solo {};
+struct Team {
+    int wave, sh;      // team_floats(APL) at sh: two sets of codes, the queue item, then a pose, its gradient and energy
+    mutable int flip;  // which of the two sets of trial codes the next round uses
+};
+// Trial codes: how a trial of the line search ended.
+constexpr int kTrialRejected = 0, kTrialScreened = 1, kTrialTaken = 2, kTrialNotFinite = 3, kTrialLast = 4;
+constexpr int kTrials = 10;
+
 // line_search_tile (bfgs.cuh:623-670). A trial whose energy is certain to fail the sufficient-decrease
 // test is not evaluated: when the gradient is dominated by the box penalty (p . g below -1e4, a pose
 // partly outside the box at slope 1e6), the trial pose's penalty alone can exceed the test's bound by
@@ -1390,7 +1403,8 @@ __device__ __forceinline__ bool pose_finite(const Ctx<APL, TW, LAZY>& C, const W
 
 template <int APL, int TW, bool LAZY>
 __device__ __forceinline__ bool line_search(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& x, float g, float p, float e0, float v_cap,
-                            float slope, WPose<APL>& x_new, float& g_new, float& e_out, float& alpha_out) {
+                            float slope, WPose<APL>& x_new, float& g_new, float& e_out, float& alpha_out,
+                            const Solo& = Solo()) {
     const float pg = tuni<TW>(tsum<TW>(p * g));
     const auto fail = [&]() {
         x_new = x;
@@ -1426,6 +1440,115 @@ __device__ __forceinline__ bool line_search(const Ctx<APL, TW, LAZY>& C, const W
     return true;
 }
 
+// line_search by a team. The trials of a round are independent; what is counted as evaluated is what the sequential
+// search evaluates.
+template <int APL, int TW, bool LAZY>
+__device__ __forceinline__ bool line_search(const Ctx<APL, TW, LAZY>& C, const WPose<APL>& x, float g, float p, float e0,
+                                            float v_cap, float slope, WPose<APL>& x_new, float& g_new, float& e_out,
+                                            float& alpha_out, const Team& T) {
+    static_assert(TW == kWave, "a team's chain takes whole waves");
+    const int ln = tlane<TW>();
+    const float pg = uni(wave_sum(p * g));
+    const int ev0 = C.evals;
+    int ev = 0, first = 0, code = 0, winner = 0;
+    float e_new = 0.0f;
+    Forces<APL> F;
+    bool failed = !__builtin_isfinite(pg);
+    if (!failed) {
+        const bool screen = pg < -1e4f && !C.biased();
+        for (; ; first += kWavesPerBlock) {
+            const int trial = first + T.wave;
+            int mine = kTrialScreened;  // past the last trial: never looked at
+            if (trial < kTrials) {
+                const float alpha = __uint_as_float(uint32_t(127 - trial) << 23);  // 2^-trial
+                x_new = x;
+                apply_update(C, x_new, p, alpha);
+                bool skip = false;
+                if (!pose_finite(C, x_new)) {
+                    mine = kTrialNotFinite;
+                } else {
+                    if (screen && trial < kTrials - 1) {
+                        const float bound = 1e-4f * alpha * pg;
+                        const float lb = energy_lower_bound(C, x_new, slope);
+                        skip = (lb - e0) - bound > 1e-4f * (fabsf(lb) + fabsf(e0) + fabsf(bound)) + 1.0f;
+                    }
+                    if (!skip) {
+                        e_new = energy_forces(C, x_new, v_cap, slope, F);
+                        mine = e_new - e0 < 1e-4f * alpha * pg ? kTrialTaken
+                               : trial == kTrials - 1          ? kTrialLast
+                                                               : kTrialRejected;
+                    }
+                }
+            }
+            int* codes = reinterpret_cast<int*>(s_lds + T.sh) + kWavesPerBlock * T.flip;
+            T.flip ^= 1;
+            if (ln == 0) codes[T.wave] = mine;
+            __syncthreads();
+            winner = -1;
+#pragma unroll
+            for (int w = 0; w < kWavesPerBlock; w++) {
+                const int c = __builtin_amdgcn_readfirstlane(codes[w]);
+                if (winner < 0) {
+                    ev += c != kTrialScreened && c != kTrialNotFinite;
+                    if (c >= kTrialTaken) {
+                        winner = w;
+                        code = c;
+                    }
+                }
+            }
+            if (winner >= 0) break;
+        }
+        failed = code == kTrialNotFinite;
+    }
+    C.evals = ev0 + ev;
+    if (failed) {
+        x_new = x;
+        g_new = g;
+        e_out = e0;
+        alpha_out = 0.0f;
+        return false;
+    }
+    float* s = s_lds + T.sh + 12;
+    if (T.wave == winner) {
+        g_new = pose_grad(C, x_new, F);
+#pragma unroll
+        for (int k = 0; k < APL; k++) {
+            s[(3 * k) * kWave + ln] = x_new.x[k];
+            s[(3 * k + 1) * kWave + ln] = x_new.y[k];
+            s[(3 * k + 2) * kWave + ln] = x_new.z[k];
+        }
+        s[3 * APL * kWave + ln] = x_new.dihe;
+        s[(3 * APL + 1) * kWave + ln] = g_new;
+        float* u = s + (3 * APL + 2) * kWave;
+        if (ln == 0) {
+            u[0] = x_new.c0; u[1] = x_new.c1; u[2] = x_new.c2;
+            u[3] = x_new.r0; u[4] = x_new.r1; u[5] = x_new.r2;
+            u[6] = e_new;
+        }
+    }
+    __syncthreads();
+    if (T.wave != winner) {
+#pragma unroll
+        for (int k = 0; k < APL; k++) {
+            x_new.x[k] = s[(3 * k) * kWave + ln];
+            x_new.y[k] = s[(3 * k + 1) * kWave + ln];
+            x_new.z[k] = s[(3 * k + 2) * kWave + ln];
+        }
+        x_new.dihe = s[3 * APL * kWave + ln];
+        g_new = s[(3 * APL + 1) * kWave + ln];
+        const float* u = s + (3 * APL + 2) * kWave;
+        x_new.c0 = uni(u[0]); x_new.c1 = uni(u[1]); x_new.c2 = uni(u[2]);
+        x_new.r0 = uni(u[3]); x_new.r1 = uni(u[4]); x_new.r2 = uni(u[5]);
+        x_new.e = x.e;
+        e_new = uni(u[6]);
+    }
+    const int taken = first + winner;
+    e_out = e_new;
+    // after the last trial failed, the step is halved once more
+    alpha_out = __uint_as_float(uint32_t(127 - taken - (code == kTrialLast ? 1 : 0)) << 23);
+    return true;
+}
+
 __device__ __forceinline__ int row_lane_clamped(int ln, int dim) { return ln < dim ? ln : dim - 1; }
 
 // A lane-distributed vector (component k on lane k) written to LDS at offset o, for broadcast reads.
@@ -1456,8 +1579,9 @@ __device__ __forceinline__ float hess_row_dot(const Ctx<APL, TW, LAZY>& C, int h
 // tile (lane i owns row i) and the start pose is parked in LDS for the
 // restore at the end (the energy went up, or a line search failed). The vectors the Hessian products read (g, y, p, -Hy) are staged in
 // the coordinate tile, idle between a line search and the next one.
-template <int APL, int TW, bool LAZY>
-__device__ __forceinline__ void bfgs(const Ctx<APL, TW, LAZY>& C, WPose<APL>& x, int max_steps, float v_cap, float slope) {
+template <int APL, int TW, bool LAZY, class Crew = Solo>
+__device__ __forceinline__ void bfgs(const Ctx<APL, TW, LAZY>& C, WPose<APL>& x, int max_steps, float v_cap, float slope,
+                                     const Crew& crew = Crew()) {
     float g;
     const float E_ori = energy_grad(C, x, v_cap, slope, g);
     float E = E_ori, E1 = 0.0f, alpha = 0.0f;
@@ -1481,7 +1605,7 @@ __device__ __forceinline__ void bfgs(const Ctx<APL, TW, LAZY>& C, WPose<APL>& x,
             p = ln < dim ? -s : 0.0f;
             wave_lds_fence();
         }
-        if (!line_search(C, x, g, p, E, v_cap, slope, x_new, g_new, E1, alpha)) {
+        if (!line_search(C, x, g, p, E, v_cap, slope, x_new, g_new, E1, alpha, crew)) {
             failed = true;
             break;
         }

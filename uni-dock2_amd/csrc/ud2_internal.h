@@ -362,6 +362,7 @@ hipError_t launch_gather_probe(const float4* cells, uint32_t span, uint32_t seed
                                hipStream_t s);
 hipError_t launch_valu_probe(float* out, int iters, int64_t n_threads, hipStream_t s);
 hipError_t launch_mc(McArgs a, int apl, int variant, int n_blocks, int waves, hipStream_t s);
+hipError_t launch_mc_team(McArgs a, int apl, int n_blocks, hipStream_t s);
 hipError_t launch_opt(OptArgs a, int apl, hipStream_t s);
 hipError_t launch_posevec(PoseVecArgs a, int apl, int n_blocks, hipStream_t s);
 hipError_t launch_cluster(const ClusterArgs& a, hipStream_t s);
@@ -384,6 +385,8 @@ __host__ __device__ constexpr int lds_tors_floats(int apl, int ld) { return (ld 
 __host__ __device__ constexpr int lds_head_floats(int apl, int ld, int tw = kWave) {
     return lds_fixed_floats(apl, tw) + lds_tors_floats(apl, ld);
 }
+// Shared area of a block whose four waves run one chain, after their slices (Team).
+__host__ __device__ constexpr int team_floats(int apl) { return 12 + kWave * (3 * apl + 2) + 8; }
 // Per-wave slices are rounded to 4 floats so every slice starts 16-byte aligned.
 __host__ __device__ constexpr int lds_round4(int n) { return (n + 3) & ~3; }
 int posevec_blocks_per_cu(int apl, int mode, int lds_bytes_per_block);

@@ -2,6 +2,8 @@
 // per-pose optimisation hooks, pose-vector scoring, grid-map build, clustering
 // and final scoring. The device building blocks and the execution model are
 // described in ud2_device.h.
+#include <type_traits>
+
 #include "ud2_device.h"
 
 namespace ud2 {
@@ -23,28 +25,43 @@ namespace ud2 {
 // atoms three waves measured 25 % faster than the two that an unconstrained allocation (239 VGPRs)
 // allowed.
 // MODE is the inter term: the grid builds hold nothing of the direct sum and the other way round.
-template <int APL, int TW, int OCC, int MODE>
+// TEAM: the four waves of a block run one chain (see Team). A search of few chains leaves most of the chip's 1,024
+// SIMDs idle and lasts as long as one chain's serial work, 2.4 energies per line search; a team's rounds of four
+// trials make that 1.2, with two barriers each: one ligand of 24 atoms at 128 chains 22.8 -> 14.0 ms, 8 ligands in
+// direct mode 41.6 -> 23.6 ms, a three-stage pipeline of 16 ligands 61.9 -> 47.0 ms.
+template <int APL, int TW, int OCC, int MODE, bool TEAM = false>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) __attribute__((amdgpu_waves_per_eu(OCC)))
 void mc_kernel(McArgs) {
     Karg<McArgs>* const K = kernel_args<McArgs>();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    using Crew = std::conditional_t<TEAM, Team, Solo>;
+    Crew crew;
+    if constexpr (TEAM) crew = Team{wave, kWavesPerBlock * K->lds_floats_per_wave, 0};
     constexpr int CPW = kWave / TW;  // chains per wave
-    const int w = threadIdx.x / kWave;
     const int h = CPW == 1 ? 0 : __lane_id() / TW;
     for (;;) {
         Karg<McArgs>& A = *reread(K);
-        const int base = w * A.lds_floats_per_wave + h * (A.lds_floats_per_wave / CPW);
+        const int base = wave * A.lds_floats_per_wave + h * (A.lds_floats_per_wave / CPW);
         const int nchain = A.P.nchain;
         const int ngroup = (nchain + CPW - 1) / CPW;
         const int n_items = A.n_order * ngroup;
         int item = 0;
-        if (lane() == 0) item = atomicAdd(A.counter, 1);
+        if constexpr (TEAM) {
+            int* slot = reinterpret_cast<int*>(s_lds + crew.sh) + 2 * kWavesPerBlock;
+            __syncthreads();  // every wave has read the last item
+            if (threadIdx.x == 0) *slot = atomicAdd(A.counter, 1);
+            __syncthreads();
+            item = *slot;
+        } else {
+            if (lane() == 0) item = atomicAdd(A.counter, 1);
+        }
         item = __builtin_amdgcn_readfirstlane(item);
         if (item >= n_items) break;
         const int lig = A.order[item / ngroup];
         const int c = CPW * (item % ngroup) + h;
-        const bool real = CPW == 1 || c < nchain;
-        const int chain = real ? c : nchain - 1;
-        Ctx<APL, TW, (OCC > 2)> C;
+        const bool real = CPW == 1 ? !TEAM || wave == 0 : c < nchain;  // who stores
+        const int chain = CPW == 1 || real ? c : nchain - 1;
+        Ctx<APL, TW, (OCC > 2) && !TEAM> C;
         load_ctx(C, (KHead*)K, lig, MODE, base, A.hdim_ld);
         Rng rng{A.seed, uint32_t(lig + A.lig_index_base), uint32_t(chain), 0u};
         WPose<APL> acc;
@@ -70,13 +87,13 @@ void mc_kernel(McArgs) {
                 float gd;
                 cand.e = energy_grad(C, cand, kVCap, kSlope, gd);
             } else {
-                bfgs(C, cand, opt_steps, kVCap, kSlope);
+                bfgs(C, cand, opt_steps, kVCap, kSlope, crew);
             }
             const uint4 b = rng.next();
             const bool accepted = (cand.e < acc_e) || (u01(b.x) < __expf((acc_e - cand.e) / 1.2f));
             if (step == 0 || accepted) {
                 if (cand.e < best) {
-                    if (opt_steps > 0) bfgs(C, cand, opt_steps, kVCapAuth, kSlope);
+                    if (opt_steps > 0) bfgs(C, cand, opt_steps, kVCapAuth, kSlope, crew);
                     if (cand.e < best) {
                         if (real) store_pose(C, reread(K)->P, lig, chain, cand);
                         best = cand.e;
@@ -683,10 +700,24 @@ static hipError_t launch_mc_t(const McArgs& a, int n_blocks, hipStream_t s) {
     return hipGetLastError();
 }
 
+// A team launch (n_blocks chains at a time, four waves each) of a one- or two-slot class; lds_floats_per_wave as ever,
+// the team's shared area after the four slices.
+hipError_t launch_mc_team(McArgs a, int apl, int n_blocks, hipStream_t s) {
+    const size_t lds = ((size_t)a.lds_floats_per_wave * kWavesPerBlock + team_floats(apl)) * sizeof(float);
+    const dim3 grid(n_blocks), block(kWave * kWavesPerBlock);
+    const bool direct = a.mode == kDirect;
+    if (apl == 1 && !direct) hipLaunchKernelGGL((mc_kernel<1, kWave, 4, kGrid, true>), grid, block, lds, s, a);
+    else if (apl == 1) hipLaunchKernelGGL((mc_kernel<1, kWave, 4, kDirect, true>), grid, block, lds, s, a);
+    else if (apl == 2 && !direct) hipLaunchKernelGGL((mc_kernel<2, kWave, 3, kGrid, true>), grid, block, lds, s, a);
+    else if (apl == 2) hipLaunchKernelGGL((mc_kernel<2, kWave, 3, kDirect, true>), grid, block, lds, s, a);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
 // waves: the most waves per SIMD the launch can keep resident (2, 4 or more). The one-slot whole-wave
-// search runs the build held to that many: with no other waves to hide its latency behind, a chain is
-// faster with fewer spills (one ligand of 24 atoms at 128 chains, 32 blocks: 32.4 ligands/s on the
-// six-wave build, 33.9 on the four-wave one, 34.9 on the two-wave one, which spills nothing).
+// search runs the build held to that many: with few other waves to hide its latency behind, a chain is
+// faster with fewer spills (128 chains, one wave each: 32.4 ligands/s on the six-wave build, 33.9 on the
+// four-wave one). Grid searches that fill only two waves per SIMD go to teams.
 hipError_t launch_mc(McArgs a, int apl, int variant, int n_blocks, int waves, hipStream_t s) {
     if (variant != kMcWhole && apl != 1) return hipErrorInvalidValue;
     if (a.mode == kDirect) {  // whole waves at two or four waves per SIMD (one slot), as below otherwise
@@ -710,9 +741,8 @@ hipError_t launch_mc(McArgs a, int apl, int variant, int n_blocks, int waves, hi
     }
     switch (apl) {
         case 1:
-            return waves <= 2   ? launch_mc_t<1, kWave, 2>(a, n_blocks, s)
-                   : waves <= 4 ? launch_mc_t<1, kWave, 4>(a, n_blocks, s)
-                                : launch_mc_t<1, kWave, 6>(a, n_blocks, s);
+            return waves <= 4 ? launch_mc_t<1, kWave, 4>(a, n_blocks, s)
+                              : launch_mc_t<1, kWave, 6>(a, n_blocks, s);
         case 2: return launch_mc_t<2, kWave, 3>(a, n_blocks, s);
         case 3: return launch_mc_t<3, kWave, 2>(a, n_blocks, s);
         case 4: return launch_mc_t<4, kWave, 2>(a, n_blocks, s);
