@@ -156,6 +156,36 @@ __device__ __forceinline__ float tsum(float v) {
     }
 }
 
+// Sums of four values over the tile's lanes: lane l (ln: tlane) gets that of v[l % 4], in the bits of tsum. The first two
+// exchanges of row_sum halve the values in flight instead of repeating themselves for each (a lane adds up the
+// values of its own place in the quad), the row sums are exchanged by two lane swaps instead of four lane reads per
+// value: 21 VALU instructions for what takes four tsum 48.
+template <int TW>
+__device__ __forceinline__ float tsum4(int ln, float v0, float v1, float v2, float v3) {
+    const bool odd = ln & 1, up = ln & 2;
+    const float a = (odd ? v1 : v0) + dpp_f<0xB1>(odd ? v0 : v1);
+    const float b = (odd ? v3 : v2) + dpp_f<0xB1>(odd ? v2 : v3);
+    float c = (up ? b : a) + dpp_f<0x4E>(up ? a : b);
+    c += dpp_f<0x1B>(dpp_f<0x141>(c));  // lane ^ 4: the half row mirrored, then each quad
+    c += dpp_f<0x128>(c);               // lane ^ 8: the row rotated by 8
+    const auto swap16 = [](float v, float& r0, float& r1) {  // the rows of each half: its first everywhere, its second
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        r0 = __uint_as_float(r[0]);
+        r1 = __uint_as_float(r[1]);
+    };
+    if constexpr (TW == kWave) {
+        const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(c), __float_as_uint(c), false, false);
+        float r0, r1, r2, r3;
+        swap16(__uint_as_float(h[0]), r0, r1);
+        swap16(__uint_as_float(h[1]), r2, r3);
+        return ((r0 + r1) + r2) + r3;
+    } else {
+        float r0, r1;
+        swap16(c, r0, r1);
+        return r0 + r1;
+    }
+}
+
 // Lane l of the tile, l the same for every lane of the wave (a constant or a wave-uniform index).
 template <int TW>
 __device__ __forceinline__ float trdl(float v, int l) {
@@ -648,9 +678,10 @@ __device__ __forceinline__ void centroid(const Ctx<APL, TW, LAZY>& C, WPose<APL>
     for (int k = 0; k < APL; k++)
         if (valid(C, k)) { sx += P.x[k]; sy += P.y[k]; sz += P.z[k]; }
     const float inv = 1.0f / float(C.natom());
-    P.c0 = tuni<TW>(tsum<TW>(sx) * inv);
-    P.c1 = tuni<TW>(tsum<TW>(sy) * inv);
-    P.c2 = tuni<TW>(tsum<TW>(sz) * inv);
+    const float c = tsum4<TW>(tlane<TW>(), sx, sy, sz, 0.0f) * inv;
+    P.c0 = trdl<TW>(c, 0);
+    P.c1 = trdl<TW>(c, 1);
+    P.c2 = trdl<TW>(c, 2);
 }
 
 // Pose slots in the wave's LDS slice: slot 0 parks the BFGS start pose, slot 1
@@ -1296,40 +1327,83 @@ __device__ __forceinline__ float pose_grad(const Ctx<APL, TW, LAZY>& C, const WP
         tqy += msub2(wz, fx[k], wx, fz[k]);
         tqz += msub2(wx, fy[k], wy, fx[k]);
     }
-    float gout = 0.0f, v;
-    v = tsum<TW>(sgx); gout = ln == 0 ? v : gout;
-    v = tsum<TW>(sgy); gout = ln == 1 ? v : gout;
-    v = tsum<TW>(sgz); gout = ln == 2 ? v : gout;
+    const float rg = tsum4<TW>(ln, sgx, sgy, sgz, tqx), rt = tsum4<TW>(ln, tqy, tqz, tqy, tqz);
+    float gout = rg;  // lanes 0-2
     {
-        const float3 og = orient_grad(P.r0, P.r1, P.r2, tsum<TW>(tqx), tsum<TW>(tqy), tsum<TW>(tqz));
+        const float3 og = orient_grad(P.r0, P.r1, P.r2, trdl<TW>(rg, 3), trdl<TW>(rt, 0), trdl<TW>(rt, 1));
         gout = ln == 3 ? og.x : gout;
         gout = ln == 4 ? og.y : gout;
         gout = ln == 5 ? og.z : gout;
     }
-    // the axis atoms from the LDS coordinate tile, which still holds this pose (the energy of P was
-    // the last evaluation): broadcast loads instead of lane reads
+    // Torsions. Lane t forms torsion t's unit axis from the LDS coordinate tile, which still holds this pose (the
+    // energy of P was the last evaluation), and stages it with the pivot and the heavy atoms it
+    // rotates in the pair-force tile, idle by now; the torques about the axes are then summed four at a time. Bound by
+    // VALU issue where waves are many and by the serial chain where they are few: every lane forming every
+    // axis, and a wave sum and two lane selects per torsion, took 46 instructions per torsion, this 21:
+    // 1,048,576 evaluations of 40 atoms and 8 torsions 4.13 -> 3.83 ms, 256 plain ligands 582 -> 566 ms.
     const float4* lx4 = reinterpret_cast<const float4*>(s_lds + C.lx());
-    const int nt = C.ntors(), lt = C.lt();
-#pragma unroll 1
-    for (int t = 0; t < nt; t++) {
-        const TorsEnt te = tors_ent_at<APL>(lt, t);
-        const float4 xt = lx4[te.to], xf = lx4[te.from];
-        float ux = xt.x - xf.x, uy = xt.y - xf.y, uz = xt.z - xf.z;
-        const float inv = frsq(sq_dist(ux, uy, uz));
-        ux *= inv; uy *= inv; uz *= inv;
-        float st = 0.0f;
+    const int nt = C.ntors(), lt = C.lt(), lf = C.lx() + 4 * TW * APL;
+    constexpr int RE = (6 + 2 * APL + 3) & ~3, CAP = 3 * TW * APL / RE;
+    static_assert(CAP % 4 == 0, "whole groups of four torsions");
+    unsigned long long hv[APL];
 #pragma unroll
-        for (int k = 0; k < APL; k++) {
-            if (((tors_mask_at<APL>(lt, t, k) >> ln) & 1ull) && heavy(C, k)) {
-                const float lx = P.x[k] - xt.x, ly = P.y[k] - xt.y, lz = P.z[k] - xt.z;
-                const float cx = msub2(ly, fz[k], lz, fy[k]), cy = msub2(lz, fx[k], lx, fz[k]),
-                            cz = msub2(lx, fy[k], ly, fx[k]);
-                st += madd3(cx, ux, cy, uy, cz, uz);
+    for (int k = 0; k < APL; k++) hv[k] = tballot<TW>(heavy(C, k));
+#pragma unroll 1
+    for (int t0 = 0; t0 < nt; t0 += CAP) {
+        const int t1 = nt < t0 + CAP ? nt : t0 + CAP;
+        wave_lds_fence();
+        if (ln >= t0 && ln < t1) {
+            const TorsEnt te = tors_ent_at<APL>(lt, ln);
+            const float4 xt = lx4[te.to], xf = lx4[te.from];
+            float ux = xt.x - xf.x, uy = xt.y - xf.y, uz = xt.z - xf.z;
+            const float inv = frsq(sq_dist(ux, uy, uz));
+            ux *= inv; uy *= inv; uz *= inv;
+            float* r = s_lds + lf + (ln - t0) * RE;
+            *reinterpret_cast<float4*>(r) = make_float4(ux, uy, uz, xt.x);
+            r[4] = xt.y;
+            r[5] = xt.z;
+#pragma unroll
+            for (int k = 0; k < APL; k++) {
+                const unsigned long long m = tors_mask_at<APL>(lt, ln, k) & hv[k];
+                r[6 + 2 * k] = __uint_as_float(uint32_t(m));
+                r[7 + 2 * k] = __uint_as_float(uint32_t(m >> 32));
             }
         }
-        v = tsum<TW>(st);
-        gout = ln == 6 + t ? v : gout;
+        wave_lds_fence();
+        // this lane's part of the torque about the axis of record i; past the last torsion whatever the tile
+        // holds, which ends up on lanes past the gradient
+        const auto torque = [&](int i) {
+            const float* r = s_lds + lf + i * RE;
+            const float4 u = *reinterpret_cast<const float4*>(r), w = *reinterpret_cast<const float4*>(r + 4);
+            float st = 0.0f;
+#pragma unroll
+            for (int k = 0; k < APL; k++) {
+                const uint32_t lo = __builtin_amdgcn_readfirstlane(__float_as_uint(k == 0 ? w.z : r[6 + 2 * k]));
+                const uint32_t hi = __builtin_amdgcn_readfirstlane(__float_as_uint(k == 0 ? w.w : r[7 + 2 * k]));
+                const float lx = P.x[k] - u.w, ly = P.y[k] - w.x, lz = P.z[k] - w.y;
+                const float cx = msub2(ly, fz[k], lz, fy[k]), cy = msub2(lz, fx[k], lx, fz[k]),
+                            cz = msub2(lx, fy[k], ly, fx[k]);
+                const float q = madd3(cx, u.x, cy, u.y, cz, u.z);
+                const bool in = __builtin_amdgcn_inverse_ballot_w64(tmask<TW>((unsigned long long)lo | ((unsigned long long)hi << 32)));
+                st = in ? st + q : st;
+            }
+            return st;
+        };
+#pragma unroll 1
+        for (int t = t0; t < t1; t += 4) {
+            // torsion t + i belongs on lane 6 + t + i, which takes value (i + 2) mod 4 of a sum of four
+            const float s0 = torque(t - t0), s1 = torque(t - t0 + 1);
+            float s2 = 0.0f, s3 = 0.0f;
+            if (t + 2 < t1) {
+                s2 = torque(t - t0 + 2);
+                s3 = torque(t - t0 + 3);
+            }
+            const float v = tsum4<TW>(ln, s2, s3, s0, s1);
+            gout = ln >= 6 + t ? v : gout;
+        }
+        wave_lds_fence();
     }
+    gout = ln < 6 + nt ? gout : 0.0f;
     // constraint docking (bfgs.cuh:176): the rigid components are never written and
     // keep the zeros the reference's gradient buffers start with
     if (C.L().constraint && ln < 6) gout = 0.0f;
