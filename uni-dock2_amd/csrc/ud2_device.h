@@ -1264,7 +1264,66 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW, LAZY>& C, cons
     // gradient on itself; the partner's share is staged in the pair-force tile (one plain write per
     // atom slot, every slot written on every diagonal) and atom c reads it back from the slot of atom
     // (c - d) mod natom, so no LDS atomics are needed
-    {
+    if constexpr (APL == 2) {
+        // two slots: the second holds the atoms from 64 on, often few. It is scored for 4 (2) diagonals at once where
+        // they fit 16 (32) lanes each, group g of the wave those of the g-th, from the coordinate tile; the
+        // gradients reach the pair-force tile when their diagonal's turn comes, and their energies the
+        // atoms' own lanes, so that every sum is formed in the order of the diagonals, with the bits of one slot
+        // after the other. A slot of its own for each diagonal left 48-63 of 64 lanes idle in half the work of a
+        // ligand of 65-80 atoms: 256 plain ligands of 10-80 atoms (58 of them past 64) 566 -> 511 ms.
+        const int extra = n - kWave, gs = extra <= 16 ? 4 : extra <= 32 ? 5 : 6, per = kWave >> gs;
+        const int la = ln & ((1 << gs) - 1), g = ln >> gs, a1 = kWave + la;
+        const float4 x1 = lx4[a1];
+        const uint32_t lut1 = uint32_t(__shfl(int(C.lut[1]), la));
+        float ax0 = 0.0f, ay0 = 0.0f, az0 = 0.0f, ax1 = 0.0f, ay1 = 0.0f, az1 = 0.0f;
+#pragma unroll 1
+        for (int d0 = 1; d0 <= nfold; d0 += per) {
+            const int cnt = nfold - d0 + 1 < per ? nfold - d0 + 1 : per;
+            unsigned long long m1 = uload(fm + (d0 - 1) * 2 + 1);
+            for (int i = 1; i < cnt; i++) m1 |= uload(fm + (d0 + i - 1) * 2 + 1) << (i << gs);
+            float bx = 0.0f, by = 0.0f, bz = 0.0f, e1 = 0.0f;
+            if (__builtin_amdgcn_inverse_ballot_w64(m1)) {
+                const uint32_t q = uint32_t(a1 + d0 + g);
+                const int j = int(min(q, q - uint32_t(n)));  // mod n
+                e1 = pair_grad(x1.x, x1.y, x1.z, x1.w, lut1, lx4[j], lfl[j], v_cap, bx, by, bz);
+            }
+#pragma unroll 1
+            for (int i = 0; i < cnt; i++) {
+                const int dg = d0 + i;
+                const unsigned long long m0 = uload(fm + (dg - 1) * 2);
+                float px = 0.0f, py = 0.0f, pz = 0.0f;
+                if (__builtin_amdgcn_inverse_ballot_w64(m0)) {
+                    const uint32_t q = uint32_t(ln + dg);
+                    const int j = int(min(q, q - uint32_t(n)));
+                    e += pair_grad(P.x[0], P.y[0], P.z[0], C.rad[0], C.lut[0], lx4[j], lfl[j], v_cap, px, py, pz);
+                }
+                s_lds[lf + ln] = px;
+                s_lds[lf + n3 + ln] = py;
+                s_lds[lf + 2 * n3 + ln] = pz;
+                if (g == i) {
+                    s_lds[lf + a1] = bx;
+                    s_lds[lf + n3 + a1] = by;
+                    s_lds[lf + 2 * n3 + a1] = bz;
+                }
+                const float es = bperm(lane_addr(la + (i << gs)), e1);
+                e += g == 0 ? es : 0.0f;
+                wave_lds_fence();
+                // lanes past the last atom read slots that mean nothing and collect what is never read
+                const uint32_t c = uint32_t(ln - dg);
+                const int src = int(min(c, c + uint32_t(n)));
+                const float* f = s_lds + lf;
+                ax0 = (ax0 + px) - f[src];
+                ay0 = (ay0 + py) - f[n3 + src];
+                az0 = (az0 + pz) - f[2 * n3 + src];
+                ax1 = (ax1 + f[kWave + ln]) - f[kWave + ln - dg];
+                ay1 = (ay1 + f[n3 + kWave + ln]) - f[n3 + kWave + ln - dg];
+                az1 = (az1 + f[2 * n3 + kWave + ln]) - f[2 * n3 + kWave + ln - dg];
+                wave_lds_fence();
+            }
+        }
+        fx[0] += ax0; fy[0] += ay0; fz[0] += az0;
+        fx[1] += ax1; fy[1] += ay1; fz[1] += az1;
+    } else {
         float ax[APL], ay[APL], az[APL];
 #pragma unroll
         for (int k = 0; k < APL; k++) ax[k] = ay[k] = az[k] = 0.0f;
