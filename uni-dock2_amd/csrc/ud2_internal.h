@@ -143,12 +143,13 @@ struct McArgs {
     unsigned long long* stats;  // optional: evals, gather bytes, pair evals, chains
 };
 
+constexpr int kOptFew = 64;  // selections up to this long travel with the kernel's arguments
 struct OptArgs {
     LigSetDev L;
     SceneDev S;
     PoseBufs P;
-    const int32_t* sel;  // selected poses: lig * nchain + chain
-    const int32_t* pos;  // output slot of each selected pose (null: its index in sel)
+    const int32_t* sel;  // selected poses: lig * nchain + chain (null: they are in few)
+    const int32_t* pos;  // output slot of each selected pose
     int32_t n_sel;
     int32_t mode;
     int32_t max_steps;
@@ -160,6 +161,7 @@ struct OptArgs {
     const float* dir;   // [n_sel][64] update direction (pose-update hook)
     float alpha;
     int32_t op;     // 0 BFGS, 1 energy+gradient, 2 pose update, 3 line search from H = I, 4 reset
+    int32_t few[kOptFew], few_pos[kOptFew];  // a short selection and its output slots
 };
 
 struct PoseVecArgs {

@@ -122,11 +122,11 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void opt_kernel(OptArgs) {
     Karg<OptArgs>* const K = kernel_args<OptArgs>();
     Karg<OptArgs>& A = *K;
     const int w = threadIdx.x / kWave;
-    const int s = blockIdx.x * kWavesPerBlock + w;
+    const int s = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + w);
     if (s >= A.n_sel) return;
-    const int pid = A.sel[s];
+    const int pid = A.sel ? A.sel[s] : A.few[s];
     const int lig = pid / A.P.nchain, chain = pid % A.P.nchain;
-    const int o = A.pos ? A.pos[s] : s;
+    const int o = A.sel ? A.pos[s] : A.few_pos[s];
     Ctx<APL> C;
     load_ctx(C, (KHead*)K, lig, MODE, w * A.lds_floats_per_wave, A.hdim_ld);
     WPose<APL> P;
