@@ -455,8 +455,9 @@ int run_opt(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P, const
         ids[k] = h[s];
         ids[n_sel + k] = s;
     }
-    // Up to kOptFew poses go with the kernel's arguments: a handful of poses is evaluated in 10 us, and copying their ids
-    // to the GPU twice, with a wait before, took 31 us more (37 poses 60 -> 29 us a call). More are copied, both lists at once.
+    // Up to kOptFew poses go with the kernel's arguments: a handful of poses is evaluated in 10 us, and copying
+    // their ids to the GPU twice, with a wait before, took 31 us more (37 poses 60 -> 29 us a call; 64 ids and their
+    // places are 512 bytes of arguments). More are copied, both lists at once.
     const bool few = n_sel <= kOptFew;
     if (!few) {
         int rc = ensure_sel(const_cast<ud2_ligset*>(ls), 2 * int64_t(n_sel));
@@ -512,8 +513,8 @@ McArgs mc_args(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P, co
 }
 
 // Searches of up to this many chains per CU, over all their launches, run each chain on a team of four waves (see
-// Team in ud2_device.h): a team evaluates 1.7 times what one wave would, on a chip that is idle otherwise. Both sides, plain searches at 128 chains per ligand, ms with one wave per chain / with a team: grid 128 chains 9.2 /
-// 5.9, 1,024 11.3 / 7.1, 2,048 15.4 / 12.6, 3,072 17.9 / 14.4, 4,096 19.2 / 18.0, 6,144 18.6 / 23.8; direct 128
+// Team in ud2_device.h): a team evaluates 1.7 times what one wave would, on a chip that is idle otherwise. Both
+// sides, plain searches at 128 chains per ligand, ms with one wave per chain / with a team: grid 128 chains 9.2 / 5.9, 1,024 11.3 / 7.1, 2,048 15.4 / 12.6, 3,072 17.9 / 14.4, 4,096 19.2 / 18.0, 6,144 18.6 / 23.8; direct 128
 // 10.8 / 8.9, 1,024 14.1 / 10.2, 1,536 18.4 / 13.1, 2,048 16.3 / 16.8, 3,072 24.4 / 25.3 (256 CUs).
 constexpr int kTeamMaxApl = 2, kTeamPerCuGrid = 12, kTeamPerCuDirect = 6;
 
@@ -1448,7 +1449,8 @@ int ud2_autotune(const ud2_scene* sc, const ud2_ligset* ls, const ud2_mc_params*
         // probe searches with the caller's parameters: each bucket's ligands, repeated until the launch
         // holds two rounds of the chip's resident whole-wave chains, searched with every variant (each
         // variant run once untimed first); a half-wave variant replaces whole waves only when it is at
-        // least 2% faster (in direct mode every variant runs whole waves). Repeated ligands write the same pose slots (the probe's poses are discarded).
+        // least 2% faster (in direct mode every variant runs whole waves). Repeated ligands write the same
+        // pose slots (the probe's poses are discarded).
         const DevLig& last = ls->h_ligs.back();
         const int64_t n_atoms = int64_t(last.atom_off) + last.natom, n_tors = int64_t(last.tors_off) + last.ntors;
         float *x = nullptr, *c = nullptr, *rv = nullptr, *dh = nullptr, *e = nullptr;
