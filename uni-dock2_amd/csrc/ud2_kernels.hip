@@ -345,9 +345,12 @@ __device__ __forceinline__ uint32_t rmsd_below(const float* xo, const float* con
 // block splits into more groups (up to 8, 32 candidates a round). The RMSDs are a serial sum per pair,
 // so what bounds the kernel is the latency of those sums and how many run at once. One pose at a time
 // against the leaders so far (a thread per leader, three barriers a pose) took 4,410 us for 64 ligands
-// of 512 poses; this takes 290 us. Blocks of 512 threads took 315 us.
+// of 512 poses; this takes 290 us. Blocks of 512 threads took 315 us. With up to 64 poses the block
+// (a power of two, blockDim.x) is what the first round can use, a wave for every four poses: 4,096 ligands of
+// 1 / 8 / 32 poses take 20 / 73 / 228 us, in blocks of 1,024 threads 326 / 373 / 520 us (one pose at a time 19 / 170 / 940).
 constexpr int kClusterThreads = 1024;
 __global__ __launch_bounds__(kClusterThreads) void cluster_kernel(ClusterArgs A) {
+    const int nt = blockDim.x;
     const int lig = blockIdx.x;
     if (lig >= A.n_lig) return;
     const int E = A.nchain, tid = threadIdx.x, ln = lane();
@@ -359,11 +362,11 @@ __global__ __launch_bounds__(kClusterThreads) void cluster_kernel(ClusterArgs A)
     uint16_t* list = order + E;                                     // [E] remaining ranks, compacted
     const DevLig d = A.L.ligs[lig];
     const float* e = A.e + (size_t)lig * E;
-    for (int i = tid; i < E; i += kClusterThreads) {
+    for (int i = tid; i < E; i += nt) {
         const float ei = e[i];
         es[i] = ei != ei ? INFINITY : ei;
     }
-    for (int w = tid; w < n_words; w += kClusterThreads) {
+    for (int w = tid; w < n_words; w += nt) {
         const int m = E - w * kWave;
         left[w] = m >= kWave ? ~0ull : (1ull << m) - 1ull;
     }
@@ -376,7 +379,7 @@ __global__ __launch_bounds__(kClusterThreads) void cluster_kernel(ClusterArgs A)
         n += __popcll(heavy[k]);
     }
     __syncthreads();
-    for (int i = tid; i < E; i += kClusterThreads) {
+    for (int i = tid; i < E; i += nt) {
         const float ei = es[i];
         int rank = 0;
         for (int j = 0; j < E; j++) {
@@ -398,7 +401,7 @@ __global__ __launch_bounds__(kClusterThreads) void cluster_kernel(ClusterArgs A)
         int total = 0;
         for (int w = 0; w < n_words; w++) total += __popcll(left[w]);
         if (total == 0) break;
-        for (int r = tid; r < E; r += kClusterThreads) {
+        for (int r = tid; r < E; r += nt) {
             const unsigned long long m = left[r / kWave];
             if ((m >> (r % kWave)) & 1ull) {
                 int at = __popcll(m & ((1ull << (r % kWave)) - 1ull));
@@ -409,10 +412,10 @@ __global__ __launch_bounds__(kClusterThreads) void cluster_kernel(ClusterArgs A)
         }
         __syncthreads();
         int groups = 1;
-        while (groups < 8 && (2 * groups) * ((total + kWave - 1) / kWave) * kWave <= kClusterThreads) groups *= 2;
-        const int per = kClusterThreads / groups, g = __builtin_amdgcn_readfirstlane(tid / per);
+        while (groups < 8 && (2 * groups) * ((total + kWave - 1) / kWave) * kWave <= nt) groups *= 2;
+        const int per = nt / groups, g = __builtin_amdgcn_readfirstlane(tid / per);
         const int n_cand = min(kClusterCand * groups, total);
-        if (kClusterCand * g < n_cand) {
+        if (total > 1 && kClusterCand * g < n_cand) {  // the last pose left leads, whatever it is near
             const float* xc[kClusterCand];
 #pragma unroll
             for (int k = 0; k < kClusterCand; k++) {
@@ -437,7 +440,7 @@ __global__ __launch_bounds__(kClusterThreads) void cluster_kernel(ClusterArgs A)
         if (tid < n_cand && ((lead >> tid) & 1u))
             A.leaders[(size_t)lig * E + n_lead + __popc(lead & ((1u << tid) - 1u))] = order[list[tid]];
         n_lead += __popc(lead);
-        for (int q = tid; q < total; q += kClusterThreads)
+        for (int q = tid; q < total; q += nt)
             if (q < n_cand || (near[q] & lead)) {
                 const int r = list[q];
                 atomicAnd(&left[r / kWave], ~(1ull << (r % kWave)));
@@ -797,7 +800,13 @@ hipError_t launch_cluster(const ClusterArgs& a, hipStream_t s) {
     if (a.n_lig <= 0) return hipSuccess;
     const size_t lds = cluster_near_words(a.nchain) * sizeof(float) + (a.nchain + kWave - 1) / kWave * sizeof(uint64_t) +
                        2 * a.nchain * sizeof(uint16_t);
-    hipLaunchKernelGGL(cluster_kernel, dim3(a.n_lig), dim3(kClusterThreads), lds, s, a);
+    // up to 64 poses: a wave for every four of them
+    int threads = kClusterThreads;
+    if (a.nchain <= kWave) {
+        threads = kWave;
+        while (threads < 8 * kWave && threads / kWave * kClusterCand < a.nchain) threads *= 2;
+    }
+    hipLaunchKernelGGL(cluster_kernel, dim3(a.n_lig), dim3(threads), lds, s, a);
     return hipGetLastError();
 }
 
