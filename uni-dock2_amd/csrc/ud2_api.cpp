@@ -1546,7 +1546,7 @@ int ud2_cluster(const ud2_ligset* ls, const ud2_poses* P, float rmsd_limit, int3
     int rc = check_poses(ls, P);
     if (rc) return rc;
     if (!leaders_d || !nleaders_d) return fail(UD2_ERR_ARG, "null output");
-    if (size_t(2) * P->nchain * sizeof(int) > 64 * 1024) return fail(UD2_ERR_LIMIT, "nchain too large for clustering");
+    if (P->nchain > kClusterMaxPoses) return fail(UD2_ERR_LIMIT, "nchain too large for clustering");
     ClusterArgs A;
     A.L = ls->view();
     A.x = P->x_d;

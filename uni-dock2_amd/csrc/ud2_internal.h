@@ -189,8 +189,16 @@ struct ClusterArgs {
     int32_t* nleaders;  // [n_lig]
 };
 
-// 32-bit words of the clustering kernel's first LDS array (one per pose, an even number of them).
+// 32-bit words of the clustering kernel's first LDS array (one per pose, an even number of them), and the bytes of all:
+// that, a bit per rank, and two 16-bit indices per pose.
 __host__ __device__ constexpr size_t cluster_near_words(int nchain) { return size_t(nchain + 1) & ~size_t(1); }
+__host__ __device__ constexpr size_t cluster_lds_bytes(int nchain) {
+    return cluster_near_words(nchain) * sizeof(uint32_t) + size_t((nchain + kWave - 1) / kWave) * sizeof(uint64_t) +
+           2 * size_t(nchain) * sizeof(uint16_t);
+}
+constexpr int kClusterMaxPoses = 8192;
+static_assert(kClusterMaxPoses <= 65536 && cluster_lds_bytes(kClusterMaxPoses) <= 160 * 1024,
+              "a ligand's poses are ranked in 16 bits, in the LDS of one block");
 
 struct ScoreArgs {
     LigSetDev L;

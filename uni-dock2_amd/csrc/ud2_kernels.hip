@@ -798,15 +798,13 @@ hipError_t launch_posevec(PoseVecArgs a, int apl, int n_blocks, hipStream_t s) {
 
 hipError_t launch_cluster(const ClusterArgs& a, hipStream_t s) {
     if (a.n_lig <= 0) return hipSuccess;
-    const size_t lds = cluster_near_words(a.nchain) * sizeof(float) + (a.nchain + kWave - 1) / kWave * sizeof(uint64_t) +
-                       2 * a.nchain * sizeof(uint16_t);
     // up to 64 poses: a wave for every four of them
     int threads = kClusterThreads;
     if (a.nchain <= kWave) {
         threads = kWave;
         while (threads < 8 * kWave && threads / kWave * kClusterCand < a.nchain) threads *= 2;
     }
-    hipLaunchKernelGGL(cluster_kernel, dim3(a.n_lig), dim3(threads), lds, s, a);
+    hipLaunchKernelGGL(cluster_kernel, dim3(a.n_lig), dim3(threads), cluster_lds_bytes(a.nchain), s, a);
     return hipGetLastError();
 }
 
