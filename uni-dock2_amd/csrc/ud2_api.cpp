@@ -230,7 +230,7 @@ int set_error(int code, const std::string& msg) { return fail(code, msg); }
 
 struct ud2_scene {
     int device = 0;
-    float4* d_rec = nullptr;
+    float4* d_rec = nullptr;  // [nrec + 1]
     int32_t nrec = 0;
     float box_lo[3], box_hi[3];
     float* d_maps = nullptr;     // [types][nz][ny][nx]
@@ -243,7 +243,7 @@ struct ud2_scene {
     int32_t* d_slot = nullptr;
     // reach lists of the direct sum (SceneDev::reach)
     float4* d_reach = nullptr;
-    int32_t* d_reach_off = nullptr;
+    int2* d_reach_off = nullptr;
     int32_t rn[3] = {0, 0, 0};
     float rorigin[3] = {0, 0, 0}, redge = 1.0f;
     float rec_lo[3], rec_hi[3];
@@ -704,7 +704,9 @@ namespace {
 // within 8 A at all; coarser where that makes more than kReachCells cells or kReachEntries entries. A
 // finer cell lists fewer atoms out of the cutoff (2 A: 1.65 listed per atom in reach, 3 A: 2.06) and
 // the lists then take more memory (a 30 A box: 15,625 cells, 15 MB). The margin holds the atoms of most poses
-// that the penalty is about to push back into the box.
+// that the penalty is about to push back into the box. They are built with the scene, for every scene: 0.12 ms, a
+// quarter of it waiting for their size. (Built at the first direct sum, a captured or allocation-free search could not
+// have them.) With a copy of every cell's count to the host and its sum back, 0.24 ms.
 constexpr double kReachEdge = 2.0, kReachMargin = 10.0, kReachDist = 8.02;
 constexpr int64_t kReachCells = 1 << 14, kReachEntries = 1 << 23;
 
@@ -731,8 +733,9 @@ int build_reach(ud2_scene* sc, const std::vector<float4>& rec) {
         any = any && hi[d] > lo[d];
     }
     if (!any) return UD2_OK;
-    double edge = kReachEdge;
-    for (;; edge *= 1.25) {
+    ReachArgs A{};
+    unsigned long long total = 0;
+    for (double edge = kReachEdge;; edge *= 1.25) {
         int64_t cells = 1;
         for (int d = 0; d < 3; d++) {
             const double n = std::ceil((hi[d] - lo[d]) / edge);
@@ -744,39 +747,35 @@ int build_reach(ud2_scene* sc, const std::vector<float4>& rec) {
         }
         if (cells > kReachCells) continue;
         sc->redge = float(edge);
-        ReachArgs A{};
         A.rec = sc->d_rec;
         A.nrec = sc->nrec;
+        A.total = reinterpret_cast<unsigned long long*>(sc->d_rec + sc->nrec);
         for (int d = 0; d < 3; d++) {
             A.rn[d] = sc->rn[d];
             A.rorigin[d] = sc->rorigin[d] = float(lo[d]);
         }
         A.edge = sc->redge;
-        std::vector<int32_t> off(cells + 1, 0);
-        if (sc->d_reach_off) UD2_HIP(hipFree(sc->d_reach_off));
-        sc->d_reach_off = nullptr;
-        UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_reach_off), off.size() * sizeof(int32_t)));
-        A.count = sc->d_reach_off;
+        if (!sc->d_reach_off)  // fewer cells in every further round
+            UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_reach_off), size_t(cells) * sizeof(int2)));
         A.off = sc->d_reach_off;
+        if (total) UD2_HIP(launch_fill_i32(reinterpret_cast<int32_t*>(A.total), 0, 2, nullptr));
         UD2_HIP(launch_reach(A, false, nullptr));
-        UD2_HIP(hipMemcpy(off.data() + 1, sc->d_reach_off, cells * sizeof(int32_t), hipMemcpyDeviceToHost));
-        int64_t total = 0;
-        for (int64_t c = 1; c <= cells; c++) {
-            total += (off[c] + kReachPad - 1) / kReachPad * kReachPad;
-            off[c] = int32_t(std::min(total, kReachEntries + kReachPad));
-        }
-        if (total > kReachEntries && cells > 1) continue;
-        if (total > kReachEntries) {  // one cell and still too many: the whole receptor, by scalar loads
-            for (int d = 0; d < 3; d++) sc->rn[d] = 0;
-            return UD2_OK;
-        }
-        UD2_HIP(hipMemcpy(sc->d_reach_off, off.data(), off.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-        UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_reach), std::max<size_t>(total, 1) * sizeof(float4)));
-        A.reach = sc->d_reach;
-        UD2_HIP(launch_reach(A, true, nullptr));
-        UD2_HIP(hipStreamSynchronize(nullptr));
+        UD2_HIP(hipMemcpy(&total, A.total, sizeof(total), hipMemcpyDeviceToHost));
+        if (total <= (unsigned long long)kReachEntries || cells == 1) break;
+    }
+    hipError_t e = hipErrorOutOfMemory;
+    if (total <= (unsigned long long)kReachEntries)
+        e = hipMalloc(reinterpret_cast<void**>(&sc->d_reach), std::max<size_t>(total, 1) * sizeof(float4));
+    if (e == hipErrorOutOfMemory) {  // one cell and still too many, or no memory: the whole receptor, by scalar loads
+        (void)hipGetLastError();
+        for (int d = 0; d < 3; d++) sc->rn[d] = 0;
         return UD2_OK;
     }
+    UD2_HIP(e);
+    A.reach = sc->d_reach;
+    UD2_HIP(launch_reach(A, true, nullptr));
+    UD2_HIP(hipStreamSynchronize(nullptr));
+    return UD2_OK;
 }
 
 }  // namespace
@@ -810,7 +809,9 @@ int ud2_scene_create(const float* rec_xyz_h, const int32_t* rec_types_h, int32_t
     }
     for (int t = 0; t < kNumTypes; t++) sc->slot_of_type[t] = -1;
     sc->nrec = int32_t(rec.size());
+    rec.push_back(make_float4(0.0f, 0.0f, 0.0f, 0.0f));  // where the entries of the reach lists are counted
     int rc = upload(&sc->d_rec, rec);
+    rec.pop_back();
     if (!rc) rc = build_reach(sc, rec);
     if (rc) {
         ud2_scene_destroy(sc);

@@ -347,8 +347,9 @@ __device__ __forceinline__ Reach reach_of(SceneArg& S, float px, float py, float
     Reach r{0, 0, false};
     if (gx >= 0.0f && gx < float(S.rn[0]) && gy >= 0.0f && gy < float(S.rn[1]) && gz >= 0.0f && gz < float(S.rn[2])) {
         const int c = (int(gz) * S.rn[1] + int(gy)) * S.rn[0] + int(gx);
-        r.begin = S.reach_off[c];
-        r.end = S.reach_off[c + 1];
+        const int2 at = S.reach_off[c];
+        r.begin = at.x;
+        r.end = at.y;
     } else {
         r.whole = px >= S.rec_lo[0] && px <= S.rec_hi[0] && py >= S.rec_lo[1] && py <= S.rec_hi[1] &&
                   pz >= S.rec_lo[2] && pz <= S.rec_hi[2];

@@ -97,10 +97,10 @@ struct SceneDev {
     const int32_t* slot_tab;  // [kNumTypes] map of each XS type (-1 = none), device memory
     // Reach lists of the direct sum: the space around the box in cells of edge 1 / rinv from rorigin, and per
     // cell the receptor atoms that a point in it can have within the cutoff, in receptor order: entries
-    // reach_off[cell] .. reach_off[cell + 1] of reach (x, y, z, atom_word), their number padded to a
+    // reach_off[cell].x .. reach_off[cell].y of reach (x, y, z, atom_word), their number padded to a
     // multiple of 4 with atoms out of any reach. Beyond rec_lo .. rec_hi no receptor atom is in reach.
     const float4* reach;
-    const int32_t* reach_off;
+    const int2* reach_off;
     int32_t rn[3];
     float rorigin[3], rinv;
     float rec_lo[3], rec_hi[3];
@@ -212,14 +212,14 @@ struct ScoreArgs {
     int32_t decomp_stride;
 };
 
-// Reach lists (SceneDev::reach): counts of every cell's list (fill false), or the lists.
+// Reach lists (SceneDev::reach): every cell's place among the entries (fill false), or the entries.
 struct ReachArgs {
     const float4* rec;
     int32_t nrec;
     int32_t rn[3];
     float rorigin[3], edge;
-    int32_t* count;      // [cells]
-    const int32_t* off;  // [cells + 1]
+    int2* off;                  // [cells]
+    unsigned long long* total;  // entries of all lists, zero at first
     float4* reach;
 };
 constexpr int kReachPad = 4;  // a list's length is a multiple of this

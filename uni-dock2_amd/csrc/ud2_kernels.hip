@@ -199,20 +199,58 @@ __global__ __launch_bounds__(kWave* kWavesPerBlock) void posevec_kernel(PoseVecA
     }
 }
 
+// Whether a receptor atom can be within the cutoff of a point of the box lo .. hi.
+__device__ __forceinline__ bool in_reach(const float4& r, const float lo[3], const float hi[3]) {
+    const float ex = fmaxf(fmaxf(lo[0] - r.x, r.x - hi[0]), 0.0f);
+    const float ey = fmaxf(fmaxf(lo[1] - r.y, r.y - hi[1]), 0.0f);
+    const float ez = fmaxf(fmaxf(lo[2] - r.z, r.z - hi[2]), 0.0f);
+    return sq_dist(ex, ey, ez) < kR2Reach;
+}
+
+// The atoms rec[c0 .. c0 + kNearChunk) in reach of the box lo .. hi, compacted in receptor order into near (x, y, z,
+// atom_word) by a block of 256 threads; returns their number. wave_n: the counts of 64 atoms each.
+constexpr int kNearChunk = 1024;
+__device__ __forceinline__ int near_atoms(const float4* rec, int nrec, int c0, const float lo[3], const float hi[3],
+                                          float4* near, int* wave_n) {
+    const int tid = threadIdx.x, ln = lane(), w = tid / kWave;
+    // atom c0 + 256 i + tid on thread tid
+    float4 r[kNearChunk / 256];
+    unsigned long long keep[kNearChunk / 256];
+#pragma unroll
+    for (int i = 0; i < kNearChunk / 256; i++) {
+        const int j = c0 + 256 * i + tid;
+        r[i] = rec[j < nrec ? j : nrec - 1];
+        keep[i] = __ballot(j < nrec && in_reach(r[i], lo, hi));
+        if (ln == 0) wave_n[4 * i + w] = __popcll(keep[i]);
+    }
+    __syncthreads();
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < kNearChunk / 256; i++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            if (v == w && ((keep[i] >> ln) & 1ull))
+                near[n + __popcll(keep[i] & ((1ull << ln) - 1ull))] =
+                    make_float4(r[i].x, r[i].y, r[i].z, __uint_as_float(atom_word(__float_as_int(r[i].w))));
+            n += wave_n[4 * i + v];
+        }
+    __syncthreads();
+    return n;
+}
+
 // Grid maps: one thread per grid point, all probe types at once, a block of 8 x 8 x 4 points (a wave 8 x 4
 // x 2, so that its lanes mostly agree on which receptor atoms are in reach). The block first compacts, in
 // receptor order, the atoms within the cutoff of its bounding box into LDS (about 190 of 2,000 at
-// 0.021 atoms / A^3), kGridChunk receptor atoms at a time; each point then sums those in the cutoff in
+// 0.021 atoms / A^3), kNearChunk receptor atoms at a time; each point then sums those in the cutoff in
 // the receptor's order, which gives the bits of the sum over the whole receptor. The slots come
 // sorted by probe radius: the terms that depend on the distance alone are formed once per radius (4 for the 8
 // default types), and the flag terms per slot from scalar registers. Bound by VALU issue and the two
 // exponentials per radius. The loop over the whole receptor for every point, with every term per type,
 // took 785 us for 81^3 points, 8 types and 2,000 atoms.
-constexpr int kGridChunk = 1024;
 __global__ __launch_bounds__(256) void grid_kernel(GridArgs A) {
     const SceneDev& S = A.S;
-    __shared__ float4 near[kGridChunk];  // x, y, z, atom_word
-    __shared__ int wave_n[kGridChunk / 64];
+    __shared__ float4 near[kNearChunk];  // x, y, z, atom_word
+    __shared__ int wave_n[kNearChunk / kWave];
     const int tid = threadIdx.x, ln = lane(), w = tid / kWave;
     const int nb[2] = {(S.gn[0] + 7) / 8, (S.gn[1] + 7) / 8};
     const int b0[3] = {int(blockIdx.x % nb[0]) * 8, int((blockIdx.x / nb[0]) % nb[1]) * 8,
@@ -232,32 +270,8 @@ __global__ __launch_bounds__(256) void grid_kernel(GridArgs A) {
     float acc[kMaxSlots];
 #pragma unroll
     for (int k = 0; k < kMaxSlots; k++) acc[k] = 0.0f;
-    for (int c0 = 0; c0 < S.nrec; c0 += kGridChunk) {
-        // which of the chunk's atoms are in reach; atom c0 + 256 i + tid on thread tid
-        float4 r[kGridChunk / 256];
-        unsigned long long keep[kGridChunk / 256];
-#pragma unroll
-        for (int i = 0; i < kGridChunk / 256; i++) {
-            const int j = c0 + 256 * i + tid;
-            r[i] = S.rec[j < S.nrec ? j : S.nrec - 1];
-            const float ex = fmaxf(fmaxf(lo[0] - r[i].x, r[i].x - hi[0]), 0.0f);
-            const float ey = fmaxf(fmaxf(lo[1] - r[i].y, r[i].y - hi[1]), 0.0f);
-            const float ez = fmaxf(fmaxf(lo[2] - r[i].z, r[i].z - hi[2]), 0.0f);
-            keep[i] = __ballot(j < S.nrec && sq_dist(ex, ey, ez) < kR2Reach);
-            if (ln == 0) wave_n[4 * i + w] = __popcll(keep[i]);
-        }
-        __syncthreads();
-        int n = 0;
-#pragma unroll
-        for (int i = 0; i < kGridChunk / 256; i++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                if (v == w && ((keep[i] >> ln) & 1ull))
-                    near[n + __popcll(keep[i] & ((1ull << ln) - 1ull))] =
-                        make_float4(r[i].x, r[i].y, r[i].z, __uint_as_float(atom_word(__float_as_int(r[i].w))));
-                n += wave_n[4 * i + v];
-            }
-        __syncthreads();
+    for (int c0 = 0; c0 < S.nrec; c0 += kNearChunk) {
+        const int n = near_atoms(S.rec, S.nrec, c0, lo, hi, near, wave_n);
         for (int j = 0; j < n; j++) {
             const float4 q = near[j];
             const float dx = q.x - px, dy = q.y - py, dz = q.z - pz;
@@ -565,45 +579,103 @@ hipError_t launch_fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Reach lists: one wave per cell takes the receptor in chunks of 64 atoms and keeps, in receptor order, those
-// within reach of the cell's cube (widened a little for points that round into it).
+// Reach lists. A block takes a brick of 4 x 4 x 2 cells, eight per wave: it compacts the receptor atoms in reach of the
+// brick into LDS, kNearChunk receptor atoms at a time, and every wave keeps, in receptor order, those
+// within reach of each of its cells' cubes (widened a little for points that round into them). The first launch
+// counts and gives every wave's lists their place, the second writes them. Bound by latency, at few waves: 2,000 atoms and
+// 15,625 cells take 18 + 16 us. A wave per cell over the whole receptor took 27 + 46 us.
+constexpr int kReachBrick[3] = {4, 4, 2}, kReachPerWave = 4 * 4 * 2 / kWavesPerBlock;
 template <bool FILL>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) void reach_kernel(ReachArgs A) {
-    const int cell = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave, ln = lane();
-    if (cell >= A.rn[0] * A.rn[1] * A.rn[2]) return;
-    const int c[3] = {cell % A.rn[0], (cell / A.rn[0]) % A.rn[1], cell / (A.rn[0] * A.rn[1])};
+    __shared__ float4 near[kNearChunk];
+    __shared__ int wave_n[kNearChunk / kWave];
+    const int ln = lane(), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int nb[2] = {(A.rn[0] + kReachBrick[0] - 1) / kReachBrick[0], (A.rn[1] + kReachBrick[1] - 1) / kReachBrick[1]};
+    const int b0[3] = {int(blockIdx.x % nb[0]) * kReachBrick[0], int((blockIdx.x / nb[0]) % nb[1]) * kReachBrick[1],
+                       int(blockIdx.x / (nb[0] * nb[1])) * kReachBrick[2]};
+    const auto low = [&](int d, int c) { return A.rorigin[d] + A.edge * float(c) - 1e-3f; };
+    const auto high = [&](int d, int c) { return A.rorigin[d] + A.edge * float(c + 1) + 1e-3f; };
     float lo[3], hi[3];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        lo[d] = A.rorigin[d] + A.edge * float(c[d]) - 1e-3f;
-        hi[d] = A.rorigin[d] + A.edge * float(c[d] + 1) + 1e-3f;
+        lo[d] = low(d, b0[d]);
+        hi[d] = high(d, b0[d] + kReachBrick[d] - 1);
     }
-    int n = 0;
-    float4* out = FILL ? A.reach + A.off[cell] : nullptr;
-    for (int j0 = 0; j0 < A.nrec; j0 += kWave) {
-        const int j = j0 + ln;
-        const float4 r = A.rec[j < A.nrec ? j : A.nrec - 1];
-        const float ex = fmaxf(fmaxf(lo[0] - r.x, r.x - hi[0]), 0.0f);
-        const float ey = fmaxf(fmaxf(lo[1] - r.y, r.y - hi[1]), 0.0f);
-        const float ez = fmaxf(fmaxf(lo[2] - r.z, r.z - hi[2]), 0.0f);
-        const unsigned long long m = __ballot(j < A.nrec && sq_dist(ex, ey, ez) < kR2Reach);
-        if (FILL && ((m >> ln) & 1ull))
-            out[n + __popcll(m & ((1ull << ln) - 1ull))] =
-                make_float4(r.x, r.y, r.z, __uint_as_float(atom_word(__float_as_int(r.w))));
-        n += __popcll(m);
+    int cell[kReachPerWave], n[kReachPerWave], at[kReachPerWave];  // cell -1: none
+    const auto place = [&](int k, int c[3]) {
+        const int i = kReachPerWave * w + k;
+        c[0] = b0[0] + i % kReachBrick[0];
+        c[1] = b0[1] + i / kReachBrick[0] % kReachBrick[1];
+        c[2] = b0[2] + i / (kReachBrick[0] * kReachBrick[1]);
+    };
+#pragma unroll
+    for (int k = 0; k < kReachPerWave; k++) {
+        int c[3];
+        place(k, c);
+        cell[k] = c[0] < A.rn[0] && c[1] < A.rn[1] && c[2] < A.rn[2] ? (c[2] * A.rn[1] + c[1]) * A.rn[0] + c[0] : -1;
+        n[k] = 0;
+        at[k] = FILL && cell[k] >= 0 ? A.off[cell[k]].x : 0;
     }
-    if (!FILL) {
-        if (ln == 0) A.count[cell] = n;
+    for (int c0 = 0; c0 < A.nrec; c0 += kNearChunk) {
+        const int m = near_atoms(A.rec, A.nrec, c0, lo, hi, near, wave_n);
+#pragma unroll
+        for (int k = 0; k < kReachPerWave; k++) {
+            if (cell[k] < 0) continue;
+            int c[3];
+            place(k, c);
+            float clo[3], chi[3];
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                clo[d] = low(d, c[d]);
+                chi[d] = high(d, c[d]);
+            }
+            for (int j0 = 0; j0 < m; j0 += kWave) {
+                const int j = j0 + ln;
+                const float4 r = near[j < m ? j : m - 1];
+                const unsigned long long keep = __ballot(j < m && in_reach(r, clo, chi));
+                if (FILL && ((keep >> ln) & 1ull)) A.reach[at[k] + n[k] + __popcll(keep & ((1ull << ln) - 1ull))] = r;
+                n[k] += __popcll(keep);
+            }
+        }
+        __syncthreads();  // before the next chunk overwrites near
+    }
+    if (FILL) {
+#pragma unroll
+        for (int k = 0; k < kReachPerWave; k++)
+            if (cell[k] >= 0 && ln < (kReachPad - n[k] % kReachPad) % kReachPad)
+                A.reach[at[k] + n[k] + ln] = make_float4(1e18f, 1e18f, 1e18f, 0.0f);
         return;
     }
-    const int pad = (kReachPad - n % kReachPad) % kReachPad;
-    if (ln < pad) out[n + ln] = make_float4(1e18f, 1e18f, 1e18f, 0.0f);
+    // one atomic per block: a thousand on one word take 15 us
+    __shared__ unsigned long long base[kWavesPerBlock + 1];
+    unsigned long long sum = 0;
+#pragma unroll
+    for (int k = 0; k < kReachPerWave; k++) sum += (n[k] + kReachPad - 1) / kReachPad * kReachPad;
+    if (ln == 0) base[w] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        sum = 0;
+        for (int v = 0; v < kWavesPerBlock; v++) sum += base[v];
+        base[kWavesPerBlock] = atomicAdd(A.total, sum);
+    }
+    __syncthreads();
+    if (ln != 0) return;
+    unsigned long long next = base[kWavesPerBlock];
+    for (int v = 0; v < w; v++) next += base[v];
+#pragma unroll
+    for (int k = 0; k < kReachPerWave; k++) {
+        if (cell[k] < 0) continue;
+        const int len = (n[k] + kReachPad - 1) / kReachPad * kReachPad;
+        A.off[cell[k]] = make_int2(int(next), int(next) + len);  // lists of more than kReachEntries are not used
+        next += len;
+    }
 }
 
 hipError_t launch_reach(const ReachArgs& a, bool fill, hipStream_t s) {
-    const int64_t n = (int64_t)a.rn[0] * a.rn[1] * a.rn[2];
+    int64_t n = 1;
+    for (int d = 0; d < 3; d++) n *= (a.rn[d] + kReachBrick[d] - 1) / kReachBrick[d];
     if (n <= 0) return hipSuccess;
-    const dim3 grid((unsigned)((n + kWavesPerBlock - 1) / kWavesPerBlock)), block(kWave * kWavesPerBlock);
+    const dim3 grid((unsigned)n), block(kWave * kWavesPerBlock);
     if (fill) hipLaunchKernelGGL(reach_kernel<true>, grid, block, 0, s, a);
     else hipLaunchKernelGGL(reach_kernel<false>, grid, block, 0, s, a);
     return hipGetLastError();
