@@ -798,7 +798,8 @@ int ud2_scene_create(const float* rec_xyz_h, const int32_t* rec_types_h, int32_t
         v.x = rec_xyz_h[3 * i];
         v.y = rec_xyz_h[3 * i + 1];
         v.z = rec_xyz_h[3 * i + 2];
-        std::memcpy(&v.w, &t, sizeof(int));
+        const uint32_t word = atom_word(float_bits(kVdwHost[t]), uint32_t(kFlagsHost[t]));
+        std::memcpy(&v.w, &word, sizeof(word));
         rec.push_back(v);
     }
     ud2_scene* sc = new ud2_scene();

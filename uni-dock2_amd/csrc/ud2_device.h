@@ -327,11 +327,7 @@ __device__ __forceinline__ float add_flag_terms(float e0, float h, float b, int 
     return fmaf_((flags & 2) ? -0.587439f : 0.0f, b, e);
 }
 
-// A receptor atom's vdW radius and type flags in one word: the radius is in [1, 4), so its bits less
-// those of 1.0 take 24 bits; the doubled flags (as pair_lut takes them) take the bits above.
-__device__ __forceinline__ uint32_t atom_word(int type) {
-    return (__float_as_uint(c_vdw[type]) - 0x3F800000u) | (uint32_t(2 * c_tflags[type]) << 24);
-}
+// A receptor atom's vdW radius and type flags in one word (ud2_internal.h, atom_word).
 __device__ __forceinline__ float word_radius(uint32_t w) { return __uint_as_float((w & 0xFFFFFFu) + 0x3F800000u); }
 __device__ __forceinline__ uint32_t word_flags2(uint32_t w) { return w >> 24; }
 
@@ -357,27 +353,41 @@ __device__ __forceinline__ Reach reach_of(SceneArg& S, float px, float py, float
     return r;
 }
 
+// A load of read-only data at an address every lane agrees on, through the constant address space:
+// a scalar load into SGPRs (the data is written before the kernel starts and never during it).
+template <class T>
+__device__ __forceinline__ T uload(const T* p) {
+    return *(const __attribute__((address_space(4))) T*)(p);
+}
+
 // f(x, y, z, atom_word) for each of them, in receptor order. A list is read four entries ahead of their use
 // (each lane its own list, so a load touches a line per lane, which bounds it together with the pair terms'
-// VALU work); the whole receptor by scalar loads. The atoms out of reach added nothing to the sum, so it
-// has the same bits. Against the loop over 2,000 atoms for every ligand atom: 20,011 direct evaluations of a
-// 57-atom ligand 1,266 -> 238 us, the re-score and decomposition of 10,210 poses 982 -> 152 us, a
-// direct-mode search of 8 ligands 745 -> 43 ms.
+// VALU work); the whole receptor by scalar loads one entry ahead, by all lanes once one of them needs it: its loop costs the wave the same
+// for one lane as for 64. The atoms out of reach added nothing to the sum, so it has the same bits. Against the loop over
+// 2,000 atoms for every ligand atom: 20,011 direct evaluations of a 57-atom ligand 1,266 -> 238 us, the re-score and
+// decomposition of 10,210 poses 982 -> 152 us, a direct-mode search of 8 ligands 745 -> 43 ms; those evaluations 30 A
+// off the box, over the whole receptor, 843 us.
 template <class F>
 __device__ __forceinline__ void for_reach(SceneArg& S, const Reach& r, F f) {
+    if (__ballot(r.whole) != 0ull) {
+        typedef float f32x4_t __attribute__((ext_vector_type(4)));
+        const f32x4_t* rec = reinterpret_cast<const f32x4_t*>(S.rec);
+        const int nrec = S.nrec;
+        f32x4_t q = uload(rec);  // there is an entry past the last
+#pragma unroll 1
+        for (int j = 0; j < nrec; j++) {
+            const f32x4_t next = uload(rec + j + 1);
+            f(q.x, q.y, q.z, __float_as_uint(q.w));
+            q = next;
+        }
+        return;
+    }
     for (int j = r.begin; j < r.end; j += kReachPad) {
         float4 q[kReachPad];
 #pragma unroll
         for (int i = 0; i < kReachPad; i++) q[i] = S.reach[j + i];
 #pragma unroll
         for (int i = 0; i < kReachPad; i++) f(q[i].x, q[i].y, q[i].z, __float_as_uint(q[i].w));
-    }
-    if (r.whole) {
-#pragma unroll 1
-        for (int j = 0; j < S.nrec; j++) {
-            const float4 q = S.rec[j];
-            f(q.x, q.y, q.z, atom_word(__float_as_int(q.w)));
-        }
     }
 }
 
@@ -1025,13 +1035,6 @@ __device__ __forceinline__ float bias_forces(const Ctx<APL, TW, LAZY>& C, const 
         }
     }
     return e;
-}
-
-// A load of read-only data at an address every lane agrees on, through the constant address space:
-// a scalar load into SGPRs (the data is written before the kernel starts and never during it).
-template <class T>
-__device__ __forceinline__ T uload(const T* p) {
-    return *(const __attribute__((address_space(4))) T*)(p);
 }
 
 // Byte address of lane l for ds_bpermute.

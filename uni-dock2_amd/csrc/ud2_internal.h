@@ -35,6 +35,12 @@ constexpr float kRampNoPair = 4.0f;  // kh of a lane that scores no pair (packed
 __host__ __device__ constexpr float ramp_hyd(int flags) { return (flags & 1) ? kRampHyd : kRampNone; }
 __host__ __device__ constexpr float ramp_hb(int flags) { return (flags & 2) ? kRampHb : 0.0f; }
 
+// A receptor atom's vdW radius and type flags in one word: the radius is in [1, 4), so its bits less
+// those of 1.0 take 24 bits; the doubled flags (as pair_lut takes them) take the bits above.
+constexpr uint32_t atom_word(uint32_t radius_bits, uint32_t flags) {
+    return (radius_bits - 0x3F800000u) | (2 * flags) << 24;
+}
+
 // One ligand of a ligand set on the device.
 struct DevLig {
     int32_t natom, ntors, npair, nheavy;
@@ -87,7 +93,7 @@ struct LigSetDev {
 
 // Device view of a scene: receptor, box and (optional) grid maps.
 struct SceneDev {
-    const float4* rec;  // heavy receptor atoms: x, y, z, type (int bits)
+    const float4* rec;  // [nrec + 1] heavy receptor atoms: x, y, z, atom_word; the last one means nothing
     int32_t nrec;
     float box_lo[3], box_hi[3];
     const float4* cells;  // maps cell-major: [slot][cz][cy][cx] x {c000 c100 c010 c110}, {c001 c101 c011 c111}
@@ -97,7 +103,7 @@ struct SceneDev {
     const int32_t* slot_tab;  // [kNumTypes] map of each XS type (-1 = none), device memory
     // Reach lists of the direct sum: the space around the box in cells of edge 1 / rinv from rorigin, and per
     // cell the receptor atoms that a point in it can have within the cutoff, in receptor order: entries
-    // reach_off[cell].x .. reach_off[cell].y of reach (x, y, z, atom_word), their number padded to a
+    // reach_off[cell].x .. reach_off[cell].y of reach (as rec), their number padded to a
     // multiple of 4 with atoms out of any reach. Beyond rec_lo .. rec_hi no receptor atom is in reach.
     const float4* reach;
     const int2* reach_off;

@@ -230,8 +230,7 @@ __device__ __forceinline__ int near_atoms(const float4* rec, int nrec, int c0, c
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             if (v == w && ((keep[i] >> ln) & 1ull))
-                near[n + __popcll(keep[i] & ((1ull << ln) - 1ull))] =
-                    make_float4(r[i].x, r[i].y, r[i].z, __uint_as_float(atom_word(__float_as_int(r[i].w))));
+                near[n + __popcll(keep[i] & ((1ull << ln) - 1ull))] = r[i];
             n += wave_n[4 * i + v];
         }
     __syncthreads();
