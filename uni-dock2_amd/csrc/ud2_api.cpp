@@ -296,6 +296,7 @@ struct ud2_ligset {
     std::vector<int32_t> h_order;
     int32_t* d_order = nullptr;
     int32_t cls_pos[kMaxApl + 1] = {0}, cls_cnt[kMaxApl + 1] = {0}, cls_dmax[kMaxApl + 1] = {0};
+    double load = 0.0;  // work of the set's ligands in units of the costliest one's
     // The one-atom-per-lane class split for the MC search by kernel variant: part v (the ligands
     // that variant v runs, in the work order above) at split[part_pos[v] .. + part_cnt[v]), its
     // largest 6 + ntors part_dmax[v]. Rebuilt when the tile policy or table changes (split_version).
@@ -512,20 +513,33 @@ McArgs mc_args(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P, co
     return A;
 }
 
-// Searches of up to this many chains per CU, over all their launches, run each chain on a team of four waves (see
-// Team in ud2_device.h): a team evaluates 1.7 times what one wave would, on a chip that is idle otherwise. Both
-// sides, plain searches at 128 chains per ligand, ms with one wave per chain / with a team: grid 128 chains 9.2 / 5.9, 1,024 11.3 / 7.1, 2,048 15.4 / 12.6, 3,072 17.9 / 14.4, 4,096 19.2 / 18.0, 6,144 18.6 / 23.8; direct 128
-// 10.8 / 8.9, 1,024 14.1 / 10.2, 1,536 18.4 / 13.1, 2,048 16.3 / 16.8, 3,072 24.4 / 25.3 (256 CUs).
-constexpr int kTeamMaxApl = 2, kTeamPerCuGrid = 12, kTeamPerCuDirect = 6;
+// Searches of few chains run each chain on a team of four waves (see Team in ud2_device.h), which ends a chain in
+// about half the time and takes about twice one wave's time on the chip. A CU holds three to six teams, so what counts is
+// the work in units of the costliest chain: the chains where all ligands are of one size, fewer where the small
+// ones are done before the largest. Time of a plain grid search with teams over that with one wave per chain (256 CUs,
+// 128 chains per ligand, 6 and 10 steps of 28 iterations), by units per CU:
+//   ligands of one size, 9 to 120 atoms              4: 0.47-0.81   6: 0.64-0.97   7: 0.72-1.02   7.5: 0.76-1.02   8: 0.79-1.30   12: 1.10-1.58
+//   10-30, 10-60, 30-60, 45-60, 10-80, 50-80, 65-80  to 5: 0.36-0.75   5-7: 0.54-0.97   7-8: 0.65-0.90   8-9: 0.80-1.20   above: 0.89-1.22
+// In direct mode, ligands of one size: 2 chains per CU 0.48-0.71, 4: 0.47-0.94, 6: 0.54-0.92; sets of 10-60 atoms: 8: 1.03, 12: 1.04.
+constexpr int kTeamMaxApl = 2;
+constexpr double kTeamLoadPerCu = 8.0;                    // grid: fewer units of work than this,
+constexpr int kTeamPerCuGrid = 12, kTeamPerCuDirect = 6;  // and at most so many chains
+
+bool team_search(const ud2_ligset* ls, const McArgs& A, int nchain) {
+    if (A.mc_steps <= 0 || A.opt_steps <= 0) return false;
+    const int64_t chains = int64_t(ls->n_lig) * nchain, cus = n_cus();
+    if (A.mode == kDirect) return chains <= kTeamPerCuDirect * cus;
+    return chains <= kTeamPerCuGrid * cus && ls->load * nchain < kTeamLoadPerCu * double(cus);
+}
 
 // One persistent MC launch over n ligands of the work order at order (atoms-per-lane class apl, kernel
 // variant, largest 6 + ntors dmax), its queue head at counter.
-// chains: those of the whole search, with its other launches.
+// team: the search runs its chains on teams (where the class has a build for it).
 // shared: the launch runs beside the one-slot class of the same search. A wider class then takes one block
 // per CU less than it could alone, so one-slot waves fit beside it (three two-slot waves of 168 VGPRs fill
 // a SIMD's register file, and the one-slot launch would wait for the whole two-slot queue to drain).
 int launch_mc_part(McArgs A, int apl, int variant, const int32_t* order, int n, int32_t* counter, int dmax,
-                   int nchain, hipStream_t st, int64_t chains, bool shared = false) {
+                   int nchain, hipStream_t st, bool team, bool shared = false) {
     if (n <= 0) return UD2_OK;
     // in direct mode the sum over the receptor outweighs what two chains per wave share: whole waves only
     if (A.mode == kDirect) variant = kMcWhole;
@@ -539,9 +553,7 @@ int launch_mc_part(McArgs A, int apl, int variant, const int32_t* order, int n, 
     const int lds_bytes = A.lds_floats_per_wave * kWavesPerBlock * int(sizeof(float));
     if (lds_bytes > 160 * 1024) return fail(UD2_ERR_LIMIT, "per-block LDS exceeds 160 KB");
     const int64_t items = int64_t(n) * ((nchain + cpw - 1) / cpw);
-    const int team_per_cu = A.mode == kDirect ? kTeamPerCuDirect : kTeamPerCuGrid;
-    if (variant == kMcWhole && apl <= kTeamMaxApl && A.mc_steps > 0 && A.opt_steps > 0 &&
-        chains <= int64_t(team_per_cu) * n_cus() &&
+    if (team && variant == kMcWhole && apl <= kTeamMaxApl &&
         lds_bytes + team_floats(apl) * int(sizeof(float)) <= 160 * 1024) {
         UD2_HIP(launch_mc_team(A, apl, int(items), st));
         return UD2_OK;
@@ -613,6 +625,7 @@ int launch_mc_classes(const ud2_ligset* ls, const ud2_poses* P, McArgs A, int32_
     for (int v = 0; v < kMcVariants; v++)
         if (ls->part_cnt[v] > 0)
             parts.push_back({1, v, ls->part_cnt[v], ls->part_dmax[v], ls->d_split + ls->part_pos[v], heads + v});
+    const bool team = team_search(ls, A, P->nchain);
     UD2_HIP(launch_fill_i32(heads, 0, kMcHeads, st));
     std::lock_guard<std::mutex> lock(g_side_mu);
     SideStreams* S = parts.size() > 1 ? side_streams(may_create) : nullptr;
@@ -628,7 +641,7 @@ int launch_mc_classes(const ud2_ligset* ls, const ud2_poses* P, McArgs A, int32_
             used[k] = true;
         }
         rc = launch_mc_part(A, p.apl, p.variant, p.order, p.n, p.head, p.dmax, P->nchain, s,
-                            int64_t(ls->n_lig) * P->nchain, S != nullptr && ls->cls_cnt[1] > 0);
+                            team, S != nullptr && ls->cls_cnt[1] > 0);
         if (rc) return rc;
     }
     for (int k = 0; S && k < kMcSide; k++)
@@ -1162,6 +1175,12 @@ int ud2_ligset_create(const ud2_ligand_batch* b, ud2_ligset** out) {
             if (ligs[a].apl != ligs[c].apl) return ligs[a].apl > ligs[c].apl;
             return cost(a) > cost(c);
         });
+        double sum = 0.0, most = 0.0;
+        for (int k = 0; k < n; k++) {
+            sum += cost(k);
+            most = std::max(most, cost(k));
+        }
+        ls->load = sum / most;
         for (int k = 0; k < n; k++) {
             const DevLig& d = ligs[ls->h_order[k]];
             if (ls->cls_cnt[d.apl]++ == 0) ls->cls_pos[d.apl] = k;
@@ -1492,8 +1511,7 @@ int ud2_autotune(const ud2_scene* sc, const ud2_ligset* ls, const ud2_mc_params*
                     for (int v = 0; v < kMcVariants; v++) {
                         UD2_HIP(launch_fill_i32(head, 0, 1, st));
                         UD2_HIP(hipEventRecord(ev0, st));
-                        const int r = launch_mc_part(A, 1, v, ord, reps, head, dmax, nchain, st,
-                                                     int64_t(reps) * nchain);
+                        const int r = launch_mc_part(A, 1, v, ord, reps, head, dmax, nchain, st, false);
                         if (r) return r;
                         UD2_HIP(hipEventRecord(ev1, st));
                         UD2_HIP(hipEventSynchronize(ev1));
