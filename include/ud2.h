@@ -199,8 +199,9 @@ int ud2_mc_noalloc(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P
  * (UD2_MC_WHOLE), or two chains of the ligand per wave, one per 32-lane half, with the register
  * allocation held to 4, 3 or 2 waves per SIMD (UD2_MC_HALF4 / 3 / 2). The variant is chosen per
  * (natom, ntors) bucket: natom 1-8, 9-16, 17-24, 25-32 by ntors 0-3, 4-7, 8-11, 12-14
- * (bucket = natom index * 4 + ntors index). Larger ligands always run one chain per wave. The
- * choice is process-wide and applies to the searches launched after it is set; a ligand set's
+ * (bucket = natom index * 4 + ntors index). Larger ligands, and every ligand in direct mode, run one
+ * chain per wave whatever is chosen; a search of few chains runs each chain on four waves, unless
+ * UD2_TILE_ALWAYS asks for a half-wave variant. The choice is process-wide and applies to the searches launched after it is set; a ligand set's
  * first search after a change copies its new work split to the device and synchronises. */
 #define UD2_MC_WHOLE 0
 #define UD2_MC_HALF4 1
@@ -210,7 +211,7 @@ int ud2_mc_noalloc(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P
 #define UD2_TUNE_BUCKETS 16
 #define UD2_TILE_AUTO 0    /* per bucket, from the table (UD2_MC_WHOLE everywhere until tuned) */
 #define UD2_TILE_NEVER 1   /* UD2_MC_WHOLE for every ligand */
-#define UD2_TILE_ALWAYS 2  /* the half-wave variant `variant` (0: UD2_MC_HALF4) for every ligand that fits */
+#define UD2_TILE_ALWAYS 2  /* the half-wave variant `variant` (0: UD2_MC_HALF4) for every ligand that fits (grid mode) */
 int ud2_set_tile_policy(int32_t policy, int32_t variant);
 /* The policy, and per bucket the variant (variant_h), the probe times in ms per variant
  * (ms_h[b][v]; -1 unmeasured) and the bucket's ranges natom lo, hi, ntors lo, hi (range_h[b][4]);
@@ -220,7 +221,7 @@ int ud2_tune_info(int32_t* policy_h, int32_t* variant_h, float* ms_h, int32_t* r
  * ligands with each variant (params' mode, mc_steps and opt_steps, nchain chains each (0: 8), the
  * ligands repeated to fill the GPU twice over) and keeps a half-wave variant in the table only
  * where it is at least 2% faster than whole waves. With cache_path, buckets found in that file for
- * this GPU model, CU count and mode are taken from it instead, and the file is rewritten with
+ * this GPU model, CU count, mode and version of the search kernels are taken from it instead, and the file is rewritten with
  * every bucket known. Allocates its probe buffers; synchronises the stream. */
 int ud2_autotune(const ud2_scene* sc, const ud2_ligset* ls, const ud2_mc_params* params, int32_t nchain,
                  const char* cache_path, void* stream);

@@ -304,6 +304,7 @@ struct ud2_ligset {
     int32_t* d_split = nullptr;
     mutable int32_t part_pos[kMcVariants] = {0}, part_cnt[kMcVariants] = {0}, part_dmax[kMcVariants] = {0};
     mutable int64_t split_version = 0;
+    mutable bool split_forced = false;  // by UD2_TILE_ALWAYS
     int32_t* d_sel_all = nullptr; // scratch for all-pose selections
     int64_t sel_all_cap = 0;
     int32_t* d_bias_start = nullptr;  // [atoms + 1], null without sites
@@ -384,6 +385,7 @@ int refresh_split(const ud2_ligset* ls, hipStream_t st) {
         UD2_HIP(hipStreamSynchronize(st));
     }
     ls->split_version = version;
+    ls->split_forced = policy == UD2_TILE_ALWAYS;
     return UD2_OK;
 }
 
@@ -622,10 +624,13 @@ int launch_mc_classes(const ud2_ligset* ls, const ud2_poses* P, McArgs A, int32_
         if (ls->cls_cnt[apl] > 0)
             parts.push_back({apl, kMcWhole, ls->cls_cnt[apl], ls->cls_dmax[apl], ls->d_order + ls->cls_pos[apl],
                              heads + kMcVariants + apl - 2});
+    // the tuned table comes from launches that fill the chip, where a team has no place: a search of few chains keeps its
+    // teams (2 ligands of 20 atoms at 128 chains, 6 steps: 2.1 ms, two chains per wave 7.1)
+    const bool team = team_search(ls, A, P->nchain);
     for (int v = 0; v < kMcVariants; v++)
         if (ls->part_cnt[v] > 0)
-            parts.push_back({1, v, ls->part_cnt[v], ls->part_dmax[v], ls->d_split + ls->part_pos[v], heads + v});
-    const bool team = team_search(ls, A, P->nchain);
+            parts.push_back({1, team && !ls->split_forced ? int(kMcWhole) : v, ls->part_cnt[v], ls->part_dmax[v],
+                             ls->d_split + ls->part_pos[v], heads + v});
     UD2_HIP(launch_fill_i32(heads, 0, kMcHeads, st));
     std::lock_guard<std::mutex> lock(g_side_mu);
     SideStreams* S = parts.size() > 1 ? side_streams(may_create) : nullptr;
@@ -1433,7 +1438,7 @@ int ud2_autotune(const ud2_scene* sc, const ud2_ligset* ls, const ud2_mc_params*
     UD2_HIP(hipGetDevice(&dev));
     hipDeviceProp_t prop;
     UD2_HIP(hipGetDeviceProperties(&prop, dev));
-    const std::string key = std::string("ud2-mc-tune 2 ") + prop.gcnArchName + " cus " + std::to_string(n_cus()) +
+    const std::string key = std::string("ud2-mc-tune 3 ") + prop.gcnArchName + " cus " + std::to_string(n_cus()) +
                             " mode " + std::to_string(prm->mode);
     bool have[kTuneBuckets] = {};
     int8_t choice[kTuneBuckets] = {};
