@@ -121,6 +121,12 @@ int ud2_scene_gather_probe(const ud2_scene* sc, int64_t n_gathers, int64_t span_
  * FP32 FMA chains of iters steps (8 * iters unpacked v_fma_f32 per thread) and write their sum to
  * out_d[thread]. Its instruction rate is the ceiling for the search kernels' plain FP32 VALU work. */
 int ud2_valu_probe(int64_t n_threads, int32_t iters, float* out_d, void* stream);
+/* Device memory of the scene's reach lists (no reference counterpart): per cell of the space around the
+ * box the receptor atoms that a point in it can have within the cutoff, built with the scene. The
+ * direct sums (direct mode, final score, decomposition) read them, and without them go over the whole
+ * receptor, with the same results. *bytes_h (optional) = their bytes, 0 without; keep 0 frees them (no
+ * call on the scene may run meanwhile). */
+int ud2_scene_reach(ud2_scene* sc, int32_t keep, int64_t* bytes_h);
 int ud2_scene_destroy(ud2_scene* sc);
 
 /* ------------------------------------------------------------- ligands

@@ -244,6 +244,7 @@ struct ud2_scene {
     // reach lists of the direct sum (SceneDev::reach)
     float4* d_reach = nullptr;
     int2* d_reach_off = nullptr;
+    int64_t reach_bytes = 0;
     int32_t rn[3] = {0, 0, 0};
     float rorigin[3] = {0, 0, 0}, redge = 1.0f;
     float rec_lo[3], rec_hi[3];
@@ -728,6 +729,15 @@ namespace {
 constexpr double kReachEdge = 2.0, kReachMargin = 10.0, kReachDist = 8.02;
 constexpr int64_t kReachCells = 1 << 14, kReachEntries = 1 << 23;
 
+void drop_reach(ud2_scene* sc) {
+    for (int d = 0; d < 3; d++) sc->rn[d] = 0;
+    if (sc->d_reach) (void)hipFree(sc->d_reach);
+    if (sc->d_reach_off) (void)hipFree(sc->d_reach_off);
+    sc->d_reach = nullptr;
+    sc->d_reach_off = nullptr;
+    sc->reach_bytes = 0;
+}
+
 int build_reach(ud2_scene* sc, const std::vector<float4>& rec) {
     double lo[3], hi[3];
     for (int d = 0; d < 3; d++) {
@@ -786,11 +796,12 @@ int build_reach(ud2_scene* sc, const std::vector<float4>& rec) {
         e = hipMalloc(reinterpret_cast<void**>(&sc->d_reach), std::max<size_t>(total, 1) * sizeof(float4));
     if (e == hipErrorOutOfMemory) {  // one cell and still too many, or no memory: the whole receptor, by scalar loads
         (void)hipGetLastError();
-        for (int d = 0; d < 3; d++) sc->rn[d] = 0;
+        drop_reach(sc);
         return UD2_OK;
     }
     UD2_HIP(e);
     A.reach = sc->d_reach;
+    sc->reach_bytes = int64_t(total * sizeof(float4)) + int64_t(sc->rn[0]) * sc->rn[1] * sc->rn[2] * int64_t(sizeof(int2));
     UD2_HIP(launch_reach(A, true, nullptr));
     UD2_HIP(hipStreamSynchronize(nullptr));
     return UD2_OK;
@@ -976,14 +987,20 @@ int ud2_valu_probe(int64_t n_threads, int32_t iters, float* out_d, void* stream)
     return UD2_OK;
 }
 
+int ud2_scene_reach(ud2_scene* sc, int32_t keep, int64_t* bytes_h) {
+    if (!sc) return fail(UD2_ERR_ARG, "null scene");
+    if (!keep) drop_reach(sc);
+    if (bytes_h) *bytes_h = sc->reach_bytes;
+    return UD2_OK;
+}
+
 int ud2_scene_destroy(ud2_scene* sc) {
     if (!sc) return UD2_OK;
     if (sc->d_rec) hipFree(sc->d_rec);
     if (sc->d_maps) hipFree(sc->d_maps);
     if (sc->d_cells) (void)hipFree(sc->d_cells);
     if (sc->d_slot) (void)hipFree(sc->d_slot);
-    if (sc->d_reach) (void)hipFree(sc->d_reach);
-    if (sc->d_reach_off) (void)hipFree(sc->d_reach_off);
+    drop_reach(sc);
     delete sc;
     return UD2_OK;
 }

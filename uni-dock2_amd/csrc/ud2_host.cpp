@@ -962,17 +962,28 @@ constexpr int64_t kMiB = 1048576;
 // Device memory of one batch in this library's layout (the counterpart of predict_gpu_flex,
 // screening.cpp:53-127): pose buffers, topology and the clustering / selection arrays.
 struct BatchSize {
-    int64_t n_lig = 0, natom = 0, ntors = 0, npair = 0, nbias = 0;
+    int64_t n_lig = 0, natom = 0, ntors = 0, npair = 0, nbias = 0, nstep = 0;
     void add(const Lig& L) {
         n_lig++;
         natom += L.natom;
         ntors += L.ntors;
         npair += int64_t(L.pairs.size() / 2);
         nbias += int64_t(L.bias.size() / 5);
+        nstep += pair_steps(L);
+    }
+    // Steps of the ligand's pair table, 1 KB each: two diagonals a step up to 32 atoms; up to 64 atoms about what the pairs
+    // and the busiest atom's pairs (four a step) need, which holds what the packing takes; none for larger ligands.
+    static int64_t pair_steps(const Lig& L) {
+        if (L.pairs.empty() || L.natom > 64) return 0;
+        if (L.natom <= 32) return (L.natom / 2 + 1) / 2;
+        std::vector<int> deg(L.natom, 0);
+        for (int32_t a : L.pairs)
+            if (a >= 0 && a < L.natom) deg[a]++;
+        return std::max<int64_t>(int64_t(L.pairs.size() / 2) / 50, (*std::max_element(deg.begin(), deg.end()) + 3) / 4) + 3;
     }
     int64_t bytes(int64_t nchain) const {
         const int64_t poses = nchain * (3 * natom + ntors) * 4 + n_lig * nchain * 7 * 4;
-        const int64_t topo = natom * 48 + ntors * 64 + npair * 8 + nbias * 32 + n_lig * 128;
+        const int64_t topo = natom * 48 + ntors * 64 + npair * 8 + nbias * 32 + n_lig * 128 + nstep * 1024;
         const int64_t cluster = n_lig * nchain * 4 * 3;
         return poses + topo + cluster;
     }
@@ -1027,15 +1038,25 @@ int run(const Params& p0, const char* json, size_t len, const std::string& out_d
         check(ud2_scene_build_grids(sc.h, kGridSpacing, pv.data(), int32_t(pv.size())), "ud2_scene_build_grids");
     }
     // device memory budget (decide_memory_limit_mb, core.cpp:32-63), less the scene's share
-    // (predict_gpu_fix, screening.cpp:44-51): receptor, maps and their cell-major copy
+    // (predict_gpu_fix, screening.cpp:44-51): receptor, maps and their cell-major copy, and the reach lists,
+    // which are given up where the batches would otherwise not hold every ligand
     int32_t gn[3] = {0, 0, 0}, n_types = 0;
     float origin[3], spacing = 0.0f;
     if (p.inter_mode == UD2_MODE_GRID) check(ud2_scene_grid_info(sc.h, gn, origin, &spacing, &n_types), "grid info");
     const int64_t fix_bytes = int64_t(R.types.size()) * 16 +
                               int64_t(n_types) * gn[0] * gn[1] * gn[2] * 4 +
                               (n_types ? int64_t(n_types) * (gn[0] - 1) * (gn[1] - 1) * (gn[2] - 1) * 32 : 0);
-    const int64_t fix_mb = fix_bytes / kMiB;
+    int64_t reach_bytes = 0, largest = 0;
+    check(ud2_scene_reach(sc.h, 1, &reach_bytes), "reach lists");
+    for (auto& L : ligs) {
+        BatchSize one;
+        one.add(L);
+        largest = std::max(largest, one.bytes(p.exhaustiveness));
+    }
     const int64_t limit_mb = memory_limit_mb(p.max_gpu_mem);
+    if (reach_bytes > 0 && largest / kMiB >= limit_mb - (fix_bytes + reach_bytes) / kMiB)
+        check(ud2_scene_reach(sc.h, 0, &reach_bytes), "reach lists");
+    const int64_t fix_mb = (fix_bytes + reach_bytes) / kMiB;
     if (limit_mb < fix_mb)
         raise("GPU memory (" + std::to_string(limit_mb) + " MB) is not enough for the receptor (" +
                   std::to_string(fix_mb) + " MB)",

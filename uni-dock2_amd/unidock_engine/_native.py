@@ -121,6 +121,7 @@ def lib():
         "ud2_scene_grid_info": (C.c_int, [vp, vp, vp, vp, vp]),
         "ud2_scene_download_maps": (C.c_int, [vp, vp]),
         "ud2_scene_gather_probe": (C.c_int, [vp, i64, i64, C.c_uint32, vp, vp]),
+        "ud2_scene_reach": (C.c_int, [vp, C.c_int32, vp]),
         "ud2_scene_destroy": (C.c_int, [vp]),
         "ud2_valu_probe": (C.c_int, [i64, i32, vp, vp]),
         "ud2_ligset_create": (C.c_int, [vp, vp]),
@@ -169,7 +170,7 @@ EXPORTED = (
     "ud2_version", "ud2_last_error", "ud2_device_count", "ud2_set_device", "ud2_synchronize", "ud2_device_memory",
     "ud2_scene_create",
     "ud2_scene_build_grids", "ud2_scene_set_grids", "ud2_scene_grid_info", "ud2_scene_download_maps",
-    "ud2_scene_gather_probe", "ud2_valu_probe", "ud2_scene_destroy", "ud2_ligset_create", "ud2_ligset_destroy", "ud2_ligset_set_bias",
+    "ud2_scene_gather_probe", "ud2_valu_probe", "ud2_scene_reach", "ud2_scene_destroy", "ud2_ligset_create", "ud2_ligset_destroy", "ud2_ligset_set_bias",
     "ud2_ligset_set_constraint", "ud2_ligset_pose_layout", "ud2_ligset_sizes", "ud2_dock", "ud2_init_poses",
     "ud2_score_posevecs", "ud2_energy_grad", "ud2_pose_update", "ud2_line_search", "ud2_optimize", "ud2_mc", "ud2_mc_noalloc",
     "ud2_set_tile_policy", "ud2_tune_info", "ud2_autotune",
@@ -227,6 +228,12 @@ class Scene:
         out = np.zeros((nt, n[2], n[1], n[0]), dtype=np.float32)
         check(lib().ud2_scene_download_maps(self.h, _ptr(out)), "ud2_scene_download_maps")
         return out
+
+    def reach_bytes(self, keep: bool = True) -> int:
+        """Device memory of the reach lists; keep=False frees them (the same results without them)."""
+        n = C.c_int64()
+        check(lib().ud2_scene_reach(self.h, int(keep), C.byref(n)), "ud2_scene_reach")
+        return n.value
 
     def close(self):
         if self.h:

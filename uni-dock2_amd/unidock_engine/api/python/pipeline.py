@@ -94,18 +94,30 @@ class BatchSize:
     src/screening/screening.cpp:53-127): pose buffers, topology, clustering / selection arrays."""
 
     def __init__(self):
-        self.n_lig = self.natom = self.ntors = self.npair = self.nbias = 0
+        self.n_lig = self.natom = self.ntors = self.npair = self.nbias = self.nstep = 0
 
     def add(self, lig) -> "BatchSize":
         b = BatchSize()
         b.n_lig, b.natom, b.ntors = self.n_lig + 1, self.natom + lig.natom, self.ntors + lig.ntors
         b.npair = self.npair + lig.npair
         b.nbias = self.nbias + (0 if lig.bias is None else len(lig.bias))
+        b.nstep = self.nstep + self.pair_steps(lig)
         return b
+
+    @staticmethod
+    def pair_steps(lig) -> int:
+        """Steps of the ligand's pair table, 1 KB each: two diagonals a step up to 32 atoms; up to 64 atoms
+        about what the pairs and the busiest atom's pairs (four a step) need, which holds what the
+        packing takes; none for larger ligands."""
+        if lig.npair == 0 or lig.natom > 64:
+            return 0
+        if lig.natom <= 32:
+            return (lig.natom // 2 + 1) // 2
+        return max(lig.npair // 50, (int(np.bincount(np.asarray(lig.pairs).reshape(-1)).max()) + 3) // 4) + 3
 
     def bytes(self, nchain: int) -> int:
         poses = nchain * (3 * self.natom + self.ntors) * 4 + self.n_lig * nchain * 7 * 4
-        topo = self.natom * 48 + self.ntors * 64 + self.npair * 8 + self.nbias * 32 + self.n_lig * 128
+        topo = self.natom * 48 + self.ntors * 64 + self.npair * 8 + self.nbias * 32 + self.n_lig * 128 + self.nstep * 1024
         return poses + topo + self.n_lig * nchain * 4 * 3
 
 
@@ -123,11 +135,11 @@ def memory_limit_mb(user_mb: int) -> int:
 
 def scene_bytes(receptor, scene) -> int:
     """The scene's device memory (predict_gpu_fix, screening.cpp:44-51): receptor atoms, grid maps
-    and their cell-major copy."""
+    and their cell-major copy, reach lists."""
     n, _, _, nt = scene.grid_info()
     n0, n1, n2 = (int(v) for v in n)
     maps = nt * n0 * n1 * n2 * 4 + (nt * (n0 - 1) * (n1 - 1) * (n2 - 1) * 32 if nt else 0)
-    return receptor.natom * 16 + maps
+    return receptor.natom * 16 + maps + scene.reach_bytes()
 
 
 def memory_batches(ligands, group, nchain: int, limit_mb: int):
@@ -324,8 +336,12 @@ def core_pipeline(p: dict, box: Box, doc: dict, inter_mode: int = N.MODE_GRID) -
         return []
     eng = DockEngine(receptor, box, mode=inter_mode)
     eng.ensure_types(ligands)
-    fix_mb = (scene_bytes(receptor, eng.scene) if inter_mode == N.MODE_GRID else receptor.natom * 16) // MIB
     limit_mb = memory_limit_mb(p["max_gpu_mem"])
+    # the reach lists are given up where the batches would otherwise not hold every ligand
+    largest = max(BatchSize().add(lig).bytes(p["exhaustiveness"]) for lig in ligands)
+    if largest // MIB >= limit_mb - scene_bytes(receptor, eng.scene) // MIB:
+        eng.scene.reach_bytes(keep=False)
+    fix_mb = scene_bytes(receptor, eng.scene) // MIB
     if limit_mb < fix_mb:
         raise RuntimeError(f"GPU memory ({limit_mb} MB) is not enough for the receptor ({fix_mb} MB)")
     files = []
