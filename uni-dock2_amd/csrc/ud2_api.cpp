@@ -75,25 +75,6 @@ void set_pair(uint4& t, int i, int j, const int32_t* types) {
     t.w = float_bits(ramp_hb(fl));
 }
 
-// Pair steps of a ligand of at most 32 atoms (LigSetDev::pack), from its folded diagonals (mask bit l of diagonal
-// d: the pair {l, (l + d) mod na} is scored). Appends the steps' entries and returns their number.
-int pack_diagonals(int na, const unsigned long long* fold, int nfold, const int32_t* types, std::vector<uint4>& pack) {
-    for (int d = 1; d <= nfold; d += 2) {
-        const size_t base = pack.size();
-        pack.resize(base + kWave, kNoPair);
-        for (int l = 0; l < kWave; l++) {
-            const int a = l & 31, dl = d + (l >> 5);
-            uint4& t = pack[base + l];
-            if (a >= na) continue;
-            const int j = (a + dl) % na;
-            if (dl <= nfold && ((fold[dl - 1] >> a) & 1ull)) set_pair(t, a, j, types);
-            t.x = uint32_t(16 * j);
-            t.y = uint32_t(4 * ((a + na - d % na) % na)) | (uint32_t(4 * (32 + (a + na - (d + 1) % na) % na)) << 8);
-        }
-    }
-    return (nfold + 1) / 2;
-}
-
 // Packed pair steps of a ligand of 33-64 atoms (LigSetDev::pack). Each step holds at most 63 pairs,
 // one per lane, with every atom i (gradient +p) of at most two of them and j (-p) of at most two, so
 // an atom collects its shares with four lane reads. Greedy first fit, the pairs of the busiest atoms
@@ -1169,10 +1150,18 @@ int ud2_ligset_create(const ud2_ligand_batch* b, ud2_ligset** out) {
             if (n_steps < 0) return fail(UD2_ERR_STATE, tag + "packed pair steps do not cover the pairs");
             d.npack = n_steps;
         }
-        if (na <= kWave / 2 && !pl.empty())
-            d.npack = pack_diagonals(na, fold.data() + d.fold_off, d.nfold, b->types_h + a0, pack);
+        if (na <= kWave / 2 && !pl.empty()) d.npack = (d.nfold + 1) / 2;
     }
-    pack.resize(pack.size() + kWave, kNoPair);  // the kernels load one step ahead
+    // the tables of the ligands of up to 32 atoms follow, written on the GPU from their diagonals, and one step more: the
+    // kernels load one step ahead
+    int64_t steps = int64_t(pack.size() / kWave);
+    bool diagonals = false;
+    for (DevLig& d : ligs)
+        if (d.natom <= kWave / 2 && d.npack > 0) {
+            d.pack_off = int32_t(steps);
+            steps += d.npack;
+            diagonals = true;
+        }
     ud2_ligset* ls = new ud2_ligset();
     hipGetDevice(&ls->device);
     ls->n_lig = n;
@@ -1219,7 +1208,14 @@ int ud2_ligset_create(const ud2_ligand_batch* b, ud2_ligset** out) {
     if (!rc) rc = upload(&ls->d_mask, mask);
     if (!rc) rc = upload(&ls->d_pairs, pairs);
     if (!rc) rc = upload(&ls->d_fold, fold);
-    if (!rc) rc = upload(&ls->d_pack, pack);
+    const auto tables = [&]() {
+        UD2_HIP(hipMalloc(reinterpret_cast<void**>(&ls->d_pack), size_t(steps + 1) * kWave * sizeof(uint4)));
+        if (!pack.empty())
+            UD2_HIP(hipMemcpy(ls->d_pack, pack.data(), pack.size() * sizeof(uint4), hipMemcpyHostToDevice));
+        if (diagonals) UD2_HIP(launch_pack_diagonals(ls->view(), n, ls->d_pack, nullptr));
+        return int(UD2_OK);
+    };
+    if (!rc) rc = tables();
     if (!rc) rc = upload(&ls->d_counter, std::vector<int32_t>(std::max(kMcHeads, kMaxApl + 1), 0));
     if (!rc) rc = upload(&ls->d_order, ls->h_order);
     if (!rc) rc = upload(&ls->d_split, std::vector<int32_t>(std::max(ls->cls_cnt[1], 1), 0));

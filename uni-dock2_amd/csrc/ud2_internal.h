@@ -52,7 +52,7 @@ struct DevLig {
     int32_t fold_off;   // into fold_mask
     int32_t nfold;      // natom / 2 folded pair diagonals, apl mask words each
     int32_t pack_off;   // into pack (steps of 64 lanes)
-    int32_t npack;      // packed pair steps (ligands of 33-64 atoms; 0 otherwise)
+    int32_t npack;      // pair steps of its table (LigSetDev::pack; ligands of at most 64 atoms)
 };
 
 // Device view of a ligand set.
@@ -383,6 +383,7 @@ hipError_t launch_opt(OptArgs a, int apl, hipStream_t s);
 hipError_t launch_posevec(PoseVecArgs a, int apl, int n_blocks, hipStream_t s);
 hipError_t launch_cluster(const ClusterArgs& a, hipStream_t s);
 hipError_t launch_final_score(const ScoreArgs& a, int apl, bool decomp, hipStream_t s);
+hipError_t launch_pack_diagonals(const LigSetDev& L, int n_lig, uint4* pack, hipStream_t s);
 hipError_t launch_fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s);
 int mc_blocks_per_cu(int apl, int variant, int mode, int lds_bytes_per_block);
 // LDS floats of a wave slice before its torsion table: coordinates + pair forces (7 * 64 * apl) and two

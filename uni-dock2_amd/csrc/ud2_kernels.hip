@@ -572,6 +572,37 @@ __global__ void fill_i32_kernel(int32_t* p, int32_t v, int64_t n) {
 }
 
 // ------------------------------------------------------------- launchers
+// Pair steps of the ligands of at most 32 atoms (LigSetDev::pack) from their folded diagonals (mask bit l of diagonal
+// d: the pair {l, (l + d) mod natom} is scored), a ligand per block, a lane per entry. On the GPU, where a table is
+// written in its 64 lanes' order; formed on the host and copied, they made a set of 1,000 ligands of 12-31 atoms
+// take 5.4 ms instead of 3.7.
+__global__ __launch_bounds__(kWave) void pack_diagonals_kernel(LigSetDev L, uint4* __restrict__ pack) {
+    const DevLig d = L.ligs[blockIdx.x];
+    if (d.natom > kWave / 2) return;
+    const int ln = lane(), a = ln & 31, na = d.natom;
+    const auto type = [&](int i) { return __float_as_int(L.atom_x0[d.atom_off + i].w); };
+    for (int s = 0; s < d.npack; s++) {
+        const int dg = 2 * s + 1, dl = dg + (ln >> 5);
+        uint4 t = make_uint4(0u, 0u, __float_as_uint(kRampNoPair), 0u);
+        if (a < na) {
+            const int j = (a + dl) % na;
+            if (dl <= d.nfold && ((L.fold_mask[d.fold_off + dl - 1] >> a) & 1ull)) {
+                const int fl = pair_flags(type(a), type(j));
+                t.z = __float_as_uint(ramp_hyd(fl));
+                t.w = __float_as_uint(ramp_hb(fl));
+            }
+            t.x = uint32_t(16 * j);
+            t.y = uint32_t(4 * ((a + na - dg % na) % na)) | (uint32_t(4 * (32 + (a + na - (dg + 1) % na) % na)) << 8);
+        }
+        pack[(size_t)(d.pack_off + s) * kWave + ln] = t;
+    }
+}
+
+hipError_t launch_pack_diagonals(const LigSetDev& L, int n_lig, uint4* pack, hipStream_t s) {
+    hipLaunchKernelGGL(pack_diagonals_kernel, dim3(n_lig), dim3(kWave), 0, s, L, pack);
+    return hipGetLastError();
+}
+
 hipError_t launch_fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(fill_i32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, v, n);
