@@ -1074,14 +1074,25 @@ __device__ __forceinline__ float pair_core(float rx, float ry, float rz, float r
 }
 
 // The pair of an atom at (xi, yi, zi) (radius ri, pair-flag table lut) with the LDS slot (x, y, z, radius) xj of
-// doubled type flags fj2; zero beyond the 8 A cutoff.
+// doubled type flags fj2; zero beyond the 8 A cutoff. SKIP: by a branch, which pays where a wave's pairs are often all
+// beyond it; three and four slots per lane are computed side by side without (8 ligands of 200 atoms searched 53.6 -> 46.7 ms,
+// 100,000 evaluations of one 8.17 -> 7.59).
+template <bool SKIP = true>
 __device__ __forceinline__ float pair_grad(float xi, float yi, float zi, float ri, uint32_t lut, float4 xj, int fj2,
                                            float v_cap, float& px, float& py, float& pz) {
     const float rx = xi - xj.x, ry = yi - xj.y, rz = zi - xj.z;
     const float rr = sq_dist(rx, ry, rz);
-    if (!(rr < kR2Cut)) return 0.0f;
+    const bool in = rr < kR2Cut;
+    if (SKIP && !in) return 0.0f;
     const int fl = int(lut >> fj2) & 3;
-    return pair_core(rx, ry, rz, rr, ri + xj.w, ramp_hyd(fl), ramp_hb(fl), v_cap, px, py, pz);
+    const float e = pair_core(rx, ry, rz, rr, ri + xj.w, ramp_hyd(fl), ramp_hb(fl), v_cap, px, py, pz);
+    if constexpr (!SKIP) {
+        px = in ? px : 0.0f;
+        py = in ? py : 0.0f;
+        pz = in ? pz : 0.0f;
+        return in ? e : 0.0f;
+    }
+    return e;
 }
 
 // cal_e_f_tile (bfgs.cuh:221-394): energy under the curl cap v_cap and the
@@ -1340,7 +1351,7 @@ __device__ __forceinline__ float energy_forces(const Ctx<APL, TW, LAZY>& C, cons
                 float px = 0.0f, py = 0.0f, pz = 0.0f;
                 if (__builtin_amdgcn_inverse_ballot_w64(m)) {
                     const int q = a + dg < n ? a + dg : a + dg - n;
-                    e += pair_grad(P.x[k], P.y[k], P.z[k], C.rad[k], C.lut[k], lx4[q], lfl[q], v_cap, px, py, pz);
+                    e += pair_grad<false>(P.x[k], P.y[k], P.z[k], C.rad[k], C.lut[k], lx4[q], lfl[q], v_cap, px, py, pz);
                 }
                 ax[k] += px; ay[k] += py; az[k] += pz;
                 s_lds[lf + a] = px;
