@@ -1170,11 +1170,11 @@ int ud2_ligset_create(const ud2_ligand_batch* b, ud2_ligset** out) {
     ls->h_order.resize(n);
     std::iota(ls->h_order.begin(), ls->h_order.end(), 0);
     {
-        // Estimated time of one chain: energy evaluations per chain (measured to grow by about 36
-        // per atom from about 2,800) times the VALU instructions of one evaluation (about 1,500
-        // fixed; the pair loop: per atom 23.5 on the two-diagonal path of ligands of at most 32
-        // atoms, about 95 per packed step for 33-64 atoms, per atom 41.5 per slot on the diagonal
-        // paths of wider ligands; 64 per torsion for its update and gradient).
+        // Weight of one chain, in units that mean nothing by themselves (only ratios are used): energy evaluations, growing
+        // with the atoms, times a fixed part, the pair loop (per atom up to 32 atoms, per packed step up to 64,
+        // per atom and slot beyond) and the torsions. Against the time of a chain on a full GPU (12-200 atoms, 0-20 torsions,
+        // 28 iterations a step) the weights of flexible ligands of up to 64 atoms agree within 15 %, and those of
+        // 65-200 atoms among themselves within 30 %, a quarter low beside the smaller ones; rigid ligands take half of theirs.
         auto cost = [&](int l) {
             const DevLig& d = ligs[l];
             const double pairs = d.natom <= kWave / 2 ? 23.5 * d.natom

@@ -17,18 +17,17 @@ namespace ud2 {
 // chain and stores nothing. The best pose goes to the pose buffers whenever it improves (the
 // reference copies it to out_pose at the same points, mc.cu:389-392).
 // OCC is the occupancy hint (waves per SIMD the register allocation must allow). One-atom-per-lane
-// ligands fit six waves per SIMD in LDS; the whole-wave kernel runs at six (80 VGPRs, 31 spilled): five
+// ligands fit six waves per SIMD in LDS; the whole-wave kernel runs at six (80 VGPRs, 39 spilled): five
 // waves with 96 VGPRs and none spilled measure the same on 256 ligands, and the learned kernel 3 % slower.
-// The search is bound by VALU issue, the LDS pipe and latency together. The half-wave kernel needs about 180 VGPRs without spills, so it comes at 4
-// (spilling), 3 and 2 waves. The two-slot kernel runs at three waves per SIMD (168 VGPRs, a few spilled;
-// its LDS allows three blocks per CU), the three- and four-slot kernels at two: on ligands of 65-80
-// atoms three waves measured 25 % faster than the two that an unconstrained allocation (239 VGPRs)
-// allowed.
+// The search is bound by VALU issue, the LDS pipe and latency together. The half-wave kernel (128-137 VGPRs, none
+// spilled) comes at 4, 3 and 2 waves. The two-slot kernel runs at three waves per SIMD (127 VGPRs; its LDS
+// allows three blocks per CU), the three- and four-slot kernels at two (145 and 171): on ligands of 65-80
+// atoms three waves measured 25 % faster than two.
 // MODE is the inter term: the grid builds hold nothing of the direct sum and the other way round.
 // TEAM: the four waves of a block run one chain (see Team). A search of few chains leaves most of the chip's 1,024
 // SIMDs idle and lasts as long as one chain's serial work, 2.4 energies per line search; a team's rounds of four
-// trials make that 1.2, with two barriers each: one ligand of 24 atoms at 128 chains 22.8 -> 14.0 ms, 8 ligands in
-// direct mode 41.6 -> 23.6 ms, a three-stage pipeline of 16 ligands 61.9 -> 47.0 ms.
+// trials make that 1.2, with two barriers each: on one GPU, one ligand of 24 atoms at 128 chains and 10 steps 10.1 -> 5.2 ms,
+// in direct mode (5 steps) 13.0 -> 6.7 ms, one of 80 atoms 41.3 -> 21.7 and 47.5 -> 21.8 ms.
 template <int APL, int TW, int OCC, int MODE, bool TEAM = false>
 __global__ __launch_bounds__(kWave* kWavesPerBlock) __attribute__((amdgpu_waves_per_eu(OCC)))
 void mc_kernel(McArgs) {
@@ -822,7 +821,8 @@ hipError_t launch_mc_team(McArgs a, int apl, int n_blocks, hipStream_t s) {
 // waves: the most waves per SIMD the launch can keep resident (2, 4 or more). The one-slot whole-wave
 // search runs the build held to that many: with few other waves to hide its latency behind, a chain is
 // faster with fewer spills (128 chains, one wave each: 32.4 ligands/s on the six-wave build, 33.9 on the
-// four-wave one). Grid searches that fill only two waves per SIMD go to teams.
+// four-wave one). On maps the four-wave build serves two waves per SIMD too (it spills nothing); most such searches
+// run on teams.
 hipError_t launch_mc(McArgs a, int apl, int variant, int n_blocks, int waves, hipStream_t s) {
     if (variant != kMcWhole && apl != 1) return hipErrorInvalidValue;
     if (a.mode == kDirect) {  // whole waves at two or four waves per SIMD (one slot), as below otherwise

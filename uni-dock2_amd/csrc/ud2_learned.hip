@@ -111,8 +111,8 @@ __device__ __forceinline__ MlpDev network(Karg<MlpDev>& w) {
 // 16 rows of ligands with 15 torsions need 832 B per block more than a quarter
 // of the CU's 160 KB, and run three waves per SIMD); the occupancy hint holds
 // the register allocation to the 80 VGPRs that six waves allow, which measured
-// 6 % faster than four waves at 128 VGPRs despite the spills (the search is
-// latency bound), and four waves faster than three. POL >= 0 compiles one
+// 6 % faster than four waves at 128 VGPRs despite the spills, and four waves faster
+// than three; at six it is bound by VALU issue (1.04 of the FMA probe's rate). POL >= 0 compiles one
 // policy only, on grid maps (the learned search); POL = -1 takes policy and inter term from the arguments. Wider ligands run at
 // three waves per SIMD (two slots) or two (three and four), as the MC kernel does.
 template <int APL, int POL>
