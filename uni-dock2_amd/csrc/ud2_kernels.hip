@@ -425,7 +425,7 @@ __global__ __launch_bounds__(kClusterThreads) void cluster_kernel(ClusterArgs A)
         __syncthreads();
         int groups = 1;
         while (groups < 8 && (2 * groups) * ((total + kWave - 1) / kWave) * kWave <= nt) groups *= 2;
-        const int per = nt / groups, g = __builtin_amdgcn_readfirstlane(tid / per);
+        const int per = nt / groups, g = __builtin_amdgcn_readfirstlane(tid >> (31 - __clz(per)));
         const int n_cand = min(kClusterCand * groups, total);
         if (total > 1 && kClusterCand * g < n_cand) {  // the last pose left leads, whatever it is near
             const float* xc[kClusterCand];
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(kClusterThreads) void cluster_kernel(ClusterArgs A)
                 xc[k] = xb + stride * (size_t)__builtin_amdgcn_readfirstlane(int(order[list[i]]));
             }
             const uint32_t real = (1u << min(kClusterCand, n_cand - kClusterCand * g)) - 1u;
-            for (int q0 = (tid % per) & ~(kWave - 1); q0 < total; q0 += per) {
+            for (int q0 = tid & (per - 1) & ~(kWave - 1); q0 < total; q0 += per) {
                 const int q = q0 + ln;
                 const bool live = q < total;
                 const float* xo = xb + stride * (size_t)order[list[live ? q : 0]];
