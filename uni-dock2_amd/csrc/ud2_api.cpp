@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstring>
 #include <fstream>
+#include <functional>
 #include <mutex>
 #include <numeric>
 #include <sstream>
@@ -832,36 +833,72 @@ int ud2_scene_create(const float* rec_xyz_h, const int32_t* rec_types_h, int32_t
     return UD2_OK;
 }
 
-static int set_probe_types(ud2_scene* sc, const int32_t* probe_types_h, int32_t n_types) {
+namespace {
+
+// A scene's maps: what is checked of a request for them before anything of the scene changes.
+struct GridPlan {
+    int32_t gn[3];
+    float origin[3], spacing;
+    std::vector<int32_t> probe_types;
+    int32_t slot_of_type[kNumTypes];
+    int64_t points = 1;
+};
+
+int plan_probes(GridPlan& g, const int32_t* probe_types_h, int32_t n_types) {
     if (n_types <= 0 || n_types > kNumTypes || !probe_types_h) return fail(UD2_ERR_ARG, "bad probe type list");
-    for (int t = 0; t < kNumTypes; t++) sc->slot_of_type[t] = -1;
-    sc->probe_types.assign(probe_types_h, probe_types_h + n_types);
+    for (int t = 0; t < kNumTypes; t++) g.slot_of_type[t] = -1;
+    g.probe_types.assign(probe_types_h, probe_types_h + n_types);
     for (int k = 0; k < n_types; k++) {
         int t = probe_types_h[k];
         if (t <= 0 || t >= kNumTypes) return fail(UD2_ERR_ARG, "probe type out of range (hydrogen has no map)");
-        if (sc->slot_of_type[t] >= 0) return fail(UD2_ERR_ARG, "duplicate probe type");
-        sc->slot_of_type[t] = k;
+        if (g.slot_of_type[t] >= 0) return fail(UD2_ERR_ARG, "duplicate probe type");
+        g.slot_of_type[t] = k;
     }
-    if (sc->d_slot) (void)hipFree(sc->d_slot);
-    sc->d_slot = nullptr;
-    return upload(&sc->d_slot, std::vector<int32_t>(sc->slot_of_type, sc->slot_of_type + kNumTypes));
+    return UD2_OK;
 }
 
-namespace {
-
-// (Re)builds the cell-major copy of the scene's maps.
-int make_cells(ud2_scene* sc) {
-    if (sc->d_cells) UD2_HIP(hipFree(sc->d_cells));
+void drop_grids(ud2_scene* sc) {
+    for (void* p : {(void*)sc->d_maps, (void*)sc->d_cells, (void*)sc->d_slot})
+        if (p) (void)hipFree(p);
+    sc->d_maps = nullptr;
     sc->d_cells = nullptr;
-    const size_t ncell = size_t(sc->gn[0] - 1) * (sc->gn[1] - 1) * (sc->gn[2] - 1) * sc->probe_types.size();
-    UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_cells), std::max<size_t>(ncell, 1) * 2 * sizeof(float4)));
-    BrickArgs B;
-    B.maps = sc->d_maps;
-    B.cells = sc->d_cells;
-    for (int d = 0; d < 3; d++) B.gn[d] = sc->gn[d];
-    B.nslot = int32_t(sc->probe_types.size());
-    UD2_HIP(launch_brick(B, nullptr));
-    return UD2_OK;
+    sc->d_slot = nullptr;
+    sc->probe_types.clear();
+    for (int t = 0; t < kNumTypes; t++) sc->slot_of_type[t] = -1;
+    for (int d = 0; d < 3; d++) sc->gn[d] = 0;
+    sc->gspacing = 0.0f;
+}
+
+// The plan's maps in place of the scene's: filled by `fill`, then copied cell-major. Without maps where a step fails.
+int make_grids(ud2_scene* sc, const GridPlan& g, const std::function<int()>& fill) {
+    drop_grids(sc);
+    for (int d = 0; d < 3; d++) {
+        sc->gn[d] = g.gn[d];
+        sc->gorigin[d] = g.origin[d];
+    }
+    sc->gspacing = g.spacing;
+    sc->probe_types = g.probe_types;
+    std::copy(g.slot_of_type, g.slot_of_type + kNumTypes, sc->slot_of_type);
+    const auto make = [&]() -> int {
+        int rc = upload(&sc->d_slot, std::vector<int32_t>(g.slot_of_type, g.slot_of_type + kNumTypes));
+        if (rc) return rc;
+        UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_maps), size_t(g.points) * g.probe_types.size() * sizeof(float)));
+        rc = fill();
+        if (rc) return rc;
+        const size_t ncell = size_t(g.gn[0] - 1) * (g.gn[1] - 1) * (g.gn[2] - 1) * g.probe_types.size();
+        UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_cells), ncell * 2 * sizeof(float4)));
+        BrickArgs B;
+        B.maps = sc->d_maps;
+        B.cells = sc->d_cells;
+        for (int d = 0; d < 3; d++) B.gn[d] = g.gn[d];
+        B.nslot = int32_t(g.probe_types.size());
+        UD2_HIP(launch_brick(B, nullptr));
+        UD2_HIP(hipDeviceSynchronize());
+        return UD2_OK;
+    };
+    const int rc = make();
+    if (rc) drop_grids(sc);
+    return rc;
 }
 
 }  // namespace
@@ -869,64 +906,56 @@ int make_cells(ud2_scene* sc) {
 int ud2_scene_build_grids(ud2_scene* sc, float spacing, const int32_t* probe_types_h, int32_t n_types) {
     if (!sc) return fail(UD2_ERR_ARG, "null scene");
     if (!(spacing > 0.0f)) return fail(UD2_ERR_ARG, "spacing must be positive");
-    int rc = set_probe_types(sc, probe_types_h, n_types);
+    GridPlan g;
+    int rc = plan_probes(g, probe_types_h, n_types);
     if (rc) return rc;
-    int64_t npt = 1;
     for (int d = 0; d < 3; d++) {
         float size = sc->box_hi[d] - sc->box_lo[d];
-        sc->gn[d] = int32_t(std::lround(double(size) / double(spacing))) + 1;
-        if (sc->gn[d] < 2) return fail(UD2_ERR_ARG, "box smaller than two grid points");
-        sc->gorigin[d] = sc->box_lo[d];
-        npt *= sc->gn[d];
+        g.gn[d] = int32_t(std::lround(double(size) / double(spacing))) + 1;
+        if (g.gn[d] < 2) return fail(UD2_ERR_ARG, "box smaller than two grid points");
+        g.origin[d] = sc->box_lo[d];
+        g.points *= g.gn[d];
     }
-    sc->gspacing = spacing;
-    if (sc->d_maps) UD2_HIP(hipFree(sc->d_maps));
-    sc->d_maps = nullptr;
-    UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_maps), size_t(npt) * n_types * sizeof(float)));
-    GridArgs A{};
-    A.S = sc->view();
-    std::vector<int32_t> by_radius(n_types);
-    std::iota(by_radius.begin(), by_radius.end(), 0);
-    std::stable_sort(by_radius.begin(), by_radius.end(),
-                     [&](int a, int b) { return kVdwHost[probe_types_h[a]] < kVdwHost[probe_types_h[b]]; });
-    for (int k = 0; k < n_types; k++) {
-        const int t = probe_types_h[by_radius[k]];
-        A.radius[k] = kVdwHost[t];
-        A.lut[k] = pair_lut_host(t);
-        A.slot[k] = by_radius[k];
-    }
-    A.nslot = n_types;
-    A.maps = sc->d_maps;
-    UD2_HIP(launch_grid_build(A, nullptr));
-    rc = make_cells(sc);
-    if (rc) return rc;
-    UD2_HIP(hipDeviceSynchronize());
-    return UD2_OK;
+    g.spacing = spacing;
+    return make_grids(sc, g, [&]() -> int {
+        GridArgs A{};
+        A.S = sc->view();
+        std::vector<int32_t> by_radius(n_types);
+        std::iota(by_radius.begin(), by_radius.end(), 0);
+        std::stable_sort(by_radius.begin(), by_radius.end(), [&](int a, int b) {
+            return kVdwHost[g.probe_types[a]] < kVdwHost[g.probe_types[b]];
+        });
+        for (int k = 0; k < n_types; k++) {
+            const int t = g.probe_types[by_radius[k]];
+            A.radius[k] = kVdwHost[t];
+            A.lut[k] = pair_lut_host(t);
+            A.slot[k] = by_radius[k];
+        }
+        A.nslot = n_types;
+        A.maps = sc->d_maps;
+        UD2_HIP(launch_grid_build(A, nullptr));
+        return UD2_OK;
+    });
 }
 
 int ud2_scene_set_grids(ud2_scene* sc, const int32_t n_h[3], const float origin_h[3], float spacing,
                         const int32_t* probe_types_h, int32_t n_types, const float* maps_h) {
     if (!sc || !n_h || !origin_h || !maps_h) return fail(UD2_ERR_ARG, "null argument");
     if (!(spacing > 0.0f)) return fail(UD2_ERR_ARG, "spacing must be positive");
-    int rc = set_probe_types(sc, probe_types_h, n_types);
+    GridPlan g;
+    int rc = plan_probes(g, probe_types_h, n_types);
     if (rc) return rc;
-    int64_t npt = 1;
     for (int d = 0; d < 3; d++) {
         if (n_h[d] < 2) return fail(UD2_ERR_ARG, "grid needs at least two points per axis");
-        sc->gn[d] = n_h[d];
-        sc->gorigin[d] = origin_h[d];
-        npt *= n_h[d];
+        g.gn[d] = n_h[d];
+        g.origin[d] = origin_h[d];
+        g.points *= n_h[d];
     }
-    sc->gspacing = spacing;
-    if (sc->d_maps) UD2_HIP(hipFree(sc->d_maps));
-    sc->d_maps = nullptr;
-    size_t bytes = size_t(npt) * n_types * sizeof(float);
-    UD2_HIP(hipMalloc(reinterpret_cast<void**>(&sc->d_maps), bytes));
-    UD2_HIP(hipMemcpy(sc->d_maps, maps_h, bytes, hipMemcpyHostToDevice));
-    rc = make_cells(sc);
-    if (rc) return rc;
-    UD2_HIP(hipDeviceSynchronize());
-    return UD2_OK;
+    g.spacing = spacing;
+    return make_grids(sc, g, [&]() -> int {
+        UD2_HIP(hipMemcpy(sc->d_maps, maps_h, size_t(g.points) * n_types * sizeof(float), hipMemcpyHostToDevice));
+        return UD2_OK;
+    });
 }
 
 int ud2_scene_grid_info(const ud2_scene* sc, int32_t n_h[3], float origin_h[3], float* spacing_h,
@@ -978,9 +1007,7 @@ int ud2_scene_reach(ud2_scene* sc, int32_t keep, int64_t* bytes_h) {
 int ud2_scene_destroy(ud2_scene* sc) {
     if (!sc) return UD2_OK;
     if (sc->d_rec) hipFree(sc->d_rec);
-    if (sc->d_maps) hipFree(sc->d_maps);
-    if (sc->d_cells) (void)hipFree(sc->d_cells);
-    if (sc->d_slot) (void)hipFree(sc->d_slot);
+    drop_grids(sc);
     drop_reach(sc);
     delete sc;
     return UD2_OK;
