@@ -404,6 +404,7 @@ int check_mode(const ud2_scene* sc, const ud2_ligset* ls, int32_t mode) {
 
 int ensure_sel(ud2_ligset* ls, int64_t n) {
     if (n <= ls->sel_all_cap) return UD2_OK;
+    ls->sel_all_cap = 0;
     if (ls->d_sel_all) UD2_HIP(hipFree(ls->d_sel_all));
     ls->d_sel_all = nullptr;
     UD2_HIP(hipMalloc(reinterpret_cast<void**>(&ls->d_sel_all), size_t(n) * sizeof(int32_t)));
