@@ -207,8 +207,9 @@ int ud2_mc_noalloc(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P
  * (natom, ntors) bucket: natom 1-8, 9-16, 17-24, 25-32 by ntors 0-3, 4-7, 8-11, 12-14
  * (bucket = natom index * 4 + ntors index). Larger ligands, and every ligand in direct mode, run one
  * chain per wave whatever is chosen; a search of few chains runs each chain on four waves, unless
- * UD2_TILE_ALWAYS asks for a half-wave variant. The choice is process-wide and applies to the searches launched after it is set; a ligand set's
- * first search after a change copies its new work split to the device and synchronises. */
+ * UD2_TILE_ALWAYS asks for a half-wave variant. The choice is process-wide and applies to the
+ * searches launched after it is set; a ligand set's first search after a change copies its new work
+ * split to the device and synchronises. */
 #define UD2_MC_WHOLE 0
 #define UD2_MC_HALF4 1
 #define UD2_MC_HALF3 2
@@ -227,8 +228,8 @@ int ud2_tune_info(int32_t* policy_h, int32_t* variant_h, float* ms_h, int32_t* r
  * ligands with each variant (params' mode, mc_steps and opt_steps, nchain chains each (0: 8), the
  * ligands repeated to fill the GPU twice over) and keeps a half-wave variant in the table only
  * where it is at least 2% faster than whole waves. With cache_path, buckets found in that file for
- * this GPU model, CU count, mode and version of the search kernels are taken from it instead, and the file is rewritten with
- * every bucket known. Allocates its probe buffers; synchronises the stream. */
+ * this GPU model, CU count, mode and version of the search kernels are taken from it instead, and
+ * the file is rewritten with every bucket known. Allocates its probe buffers; synchronises the stream. */
 int ud2_autotune(const ud2_scene* sc, const ud2_ligset* ls, const ud2_mc_params* params, int32_t nchain,
                  const char* cache_path, void* stream);
 /* Greedy leader clustering per ligand by heavy-atom RMSD (cluster_cu,

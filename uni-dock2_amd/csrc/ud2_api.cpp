@@ -504,9 +504,9 @@ McArgs mc_args(const ud2_scene* sc, const ud2_ligset* ls, const ud2_poses* P, co
 // the work in units of the costliest chain: the chains where all ligands are of one size, fewer where the small
 // ones are done before the largest. Time of a plain grid search with teams over that with one wave per chain (256 CUs,
 // 128 chains per ligand, 6 and 10 steps of 28 iterations), by units per CU:
-//   ligands of one size, 9 to 120 atoms              4: 0.47-0.81   6: 0.64-0.97   7: 0.72-1.02   7.5: 0.76-1.02   8: 0.79-1.30   12: 1.10-1.58
-//   10-30, 10-60, 30-60, 45-60, 10-80, 50-80, 65-80  to 5: 0.36-0.75   5-7: 0.54-0.97   7-8: 0.65-0.90   8-9: 0.80-1.20   above: 0.89-1.22
-// In direct mode, ligands of one size: 2 chains per CU 0.48-0.71, 4: 0.47-0.94, 6: 0.54-0.92; sets of 10-60 atoms: 8: 1.03, 12: 1.04.
+//   ligands of one size, 9 to 120 atoms: 4 0.47-0.81, 6 0.64-0.97, 7 0.72-1.02, 7.5 0.76-1.02, 8 0.79-1.30, 12 1.10-1.58;
+//   seven ranges of sizes in 10-80 atoms: up to 5 0.36-0.75, 5-7 0.54-0.97, 7-8 0.65-0.90, 8-9 0.80-1.20, above 0.89-1.22.
+// In direct mode, by chains per CU: ligands of one size 2 0.48-0.71, 4 0.47-0.94, 6 0.54-0.92; 10-60 atoms 8 1.03, 12 1.04.
 constexpr int kTeamMaxApl = 2;
 constexpr double kTeamLoadPerCu = 8.0;                    // grid: fewer units of work than this,
 constexpr int kTeamPerCuGrid = 12, kTeamPerCuDirect = 6;  // and at most so many chains
